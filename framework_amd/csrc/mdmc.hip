@@ -199,7 +199,7 @@ int plan_tiling(const uint32_t dims[3], Plan *p, const int *opt) {
   // prefix is the grand total)
   p->ntiles = (uint32_t)(p->nsegs / kScanTile + 1);
   p->classify_blocks = (uint64_t)p->XT * p->NRB * p->NKC;
-  p->vec4 = (p->X % 4 == 0) && env_int("MDMC_VEC4", 1) != 0;
+  p->vec4 = p->X >= 4 && env_int("MDMC_VEC4", 1) != 0;
   p->ptR = pt_rows(W / 4);
   p->ptKP = pt_planes(W / 4);
   // context options (0: default): cell rows and planes per tile, columns per group
@@ -479,7 +479,7 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
     ProfScope ps(ctx, 0, st);
     if (!p.zmarch) {
       PtArgs pa{ca, p.band, p.NKBp, p.NRBp};
-      const bool vec = p.vec4 && ((uintptr_t)d_field % 16 == 0);
+      const bool vec = p.vec4 && ((uintptr_t)d_field % sizeof(float) == 0);
       rc = launch_classify_pt(p.W, p.ptR, p.ptKP, vec, pa, (uint32_t)p.pt_blocks, st);
     } else {
       rc = launch_classify(p.W, p.R, ca, (uint32_t)p.classify_blocks, st);
@@ -732,7 +732,7 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     b.tile_off = (uint32_t)tile_off;
     b.NRB = NRB;
     b.NKP = NKP;
-    b.vec = (X % 4 == 0 && (reinterpret_cast<uintptr_t>(mv.field) & 15u) == 0) ? 1u : 0u;
+    b.vec = (X >= 4 && (reinterpret_cast<uintptr_t>(mv.field) & 3u) == 0) ? 1u : 0u;
     b.seg_off = (uint32_t)seg_off;
     b.nsegs = (uint32_t)nsegs;
     b.mnx = mv.xyz_min[0];

@@ -18,7 +18,7 @@ struct Plan {
   uint64_t nsegs, nslots, max_chunks, classify_blocks;
   uint64_t ncoord;  // point coordinates kept for the emit: X + Y + Z (summed over a batch)
   int empty;
-  int vec4;    // rows are a multiple of 4 points
+  int vec4;    // rows hold at least 4 points: 16-byte row loads
   int zmarch;  // use the z-marching classify kernel
   uint32_t ptR, ptKP;        // plane tiles: cell rows, cell planes
   uint32_t band, NKBp, NRBp; // plane tiles: columns per group, plane blocks, row blocks

@@ -445,9 +445,13 @@ __device__ __forceinline__ void zero_scan_state(const ClassifyArgs &a, uint32_t 
   zero_tickets(a.scan_ticket, tid);
 }
 
+// 4 consecutive points of a row (16 bytes at the alignment of a float).
+typedef float Float4Row __attribute__((ext_vector_type(4), aligned(4)));
+
 // One plane tile (x-tile xt, row block rb, plane block kb) of the volume `a`.
-// VEC: rows start on 16-byte boundaries and hold a multiple of 4 points, so a
-// lane's 4 points are one 16-byte load; otherwise 4 separate loads.
+// VEC: rows hold at least 4 points, so a lane's 4 points are one 16-byte load
+// (the rows may start anywhere: the load needs the alignment of a float only);
+// otherwise 4 separate loads.
 template <int W4, int R, int KP, bool VEC>
 __device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t xt, uint32_t rb,
                                                  uint32_t kb, uint32_t *s_w, uint32_t *s_tab,
@@ -477,11 +481,17 @@ __device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t
     float4 v[kRowsPerWave][KP + 1][W4];
     float ve[kRowsPerWave][KP + 1];
     uint32_t xob[W4][VEC ? 1 : 4];  // byte offsets of the lane's points in a row
+    uint32_t xsh[W4];               // points its load starts before its first point
 #pragma unroll
     for (int c = 0; c < W4; ++c) {
       if constexpr (VEC) {
-        xob[c][0] = min(x0 + 256u * c + 4u * lane, g.X - 4u) * 4u;
+        // the lane that holds the row's end loads the row's last 4 points and
+        // shifts its sign bits (lanes past the end hold bits no cell uses)
+        const uint32_t xs = x0 + 256u * c + 4u * lane, xl = min(xs, g.X - 4u);
+        xob[c][0] = xl * 4u;
+        xsh[c] = min(xs - xl, 4u);
       } else {
+        xsh[c] = 0u;
 #pragma unroll
         for (int e = 0; e < 4; ++e) xob[c][e] = min(x0 + 256u * c + 4u * lane + (uint32_t)e, g.X - 1u) * 4u;
       }
@@ -497,7 +507,8 @@ __device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t
 #pragma unroll
         for (int c = 0; c < W4; ++c) {
           if constexpr (VEC) {
-            v[i][p][c] = *reinterpret_cast<const float4 *>(rowb + xob[c][0]);
+            const Float4Row w = *reinterpret_cast<const Float4Row *>(rowb + xob[c][0]);
+            v[i][p][c] = make_float4(w.x, w.y, w.z, w.w);
           } else {
             v[i][p][c].x = *reinterpret_cast<const float *>(rowb + xob[c][0]);
             v[i][p][c].y = *reinterpret_cast<const float *>(rowb + xob[c][1]);
@@ -517,9 +528,11 @@ __device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t
       for (int p = 0; p <= KP; ++p) {
         uint32_t nib[W4];
 #pragma unroll
-        for (int c = 0; c < W4; ++c)
+        for (int c = 0; c < W4; ++c) {
           nib[c] = (uint32_t)(v[i][p][c].x < iso) | ((uint32_t)(v[i][p][c].y < iso) << 1) |
                    ((uint32_t)(v[i][p][c].z < iso) << 2) | ((uint32_t)(v[i][p][c].w < iso) << 3);
+          if constexpr (VEC) nib[c] >>= xsh[c];
+        }
         const uint32_t ext = (uint32_t)(ve[i][p] < iso);
 #pragma unroll
         for (int c = 0; c < W4; ++c) {
@@ -740,7 +753,7 @@ struct BatchVol {
   ClassifyArgs c;         // per-volume field and tiling; record pointers start at seg_off
   uint32_t tile_off;      // first flattened classify tile
   uint32_t NRB, NKP;      // row blocks and plane blocks of the volume
-  uint32_t vec;           // rows are 16-byte aligned multiples of 4 points
+  uint32_t vec;           // rows hold at least 4 points (16-byte row loads)
   uint32_t seg_off, nsegs;
   float mnx, mny, mnz, rgx, rgy, rgz;
   float *verts;
