@@ -199,7 +199,6 @@ int plan_tiling(const uint32_t dims[3], Plan *p, const int *opt) {
   // prefix is the grand total)
   p->ntiles = (uint32_t)(p->nsegs / kScanTile + 1);
   p->classify_blocks = (uint64_t)p->XT * p->NRB * p->NKC;
-  p->vec4 = p->X >= 4 && env_int("MDMC_VEC4", 1) != 0;
   p->ptR = pt_rows(W / 4);
   p->ptKP = pt_planes(W / 4);
   // context options (0: default): cell rows and planes per tile, columns per group
@@ -479,8 +478,7 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
     ProfScope ps(ctx, 0, st);
     if (!p.zmarch) {
       PtArgs pa{ca, p.band, p.NKBp, p.NRBp};
-      const bool vec = p.vec4 && ((uintptr_t)d_field % sizeof(float) == 0);
-      rc = launch_classify_pt(p.W, p.ptR, p.ptKP, vec, pa, (uint32_t)p.pt_blocks, st);
+      rc = launch_classify_pt(p.W, p.ptR, p.ptKP, pt_tail(p.X, p.XT, p.cap), pa, (uint32_t)p.pt_blocks, st);
     } else {
       rc = launch_classify(p.W, p.R, ca, (uint32_t)p.classify_blocks, st);
     }
@@ -634,10 +632,20 @@ uint64_t batch_key_of(const mdmc_volume *vols, uint32_t n) {
   return h;
 }
 
-// Device table (n BatchVol), bases (n uint2), batch counts (4 words); two
-// pinned staging tables of n entries.
+// Bytes of a batch's uploaded tables: n BatchVol, then the volumes' first
+// tiles and the tile total (n + 1 words), then their first segments (n words).
+constexpr size_t batch_table_bytes(uint32_t n) {
+  return n * sizeof(BatchVol) + (2 * (size_t)n + 1) * sizeof(uint32_t);
+}
+uint32_t *batch_tile_off(void *tables, uint32_t n) {
+  return reinterpret_cast<uint32_t *>(static_cast<char *>(tables) + n * sizeof(BatchVol));
+}
+uint32_t *batch_seg_off(void *tables, uint32_t n) { return batch_tile_off(tables, n) + n + 1; }
+
+// Device tables, bases (n uint2), batch counts (4 words); two pinned staging
+// copies of the tables.
 int ensure_batch_buffers(mdmc_ctx *ctx, uint32_t n) {
-  const size_t o_base = align256(n * sizeof(BatchVol));
+  const size_t o_base = align256(batch_table_bytes(n));
   const size_t o_cnt = o_base + align256(n * sizeof(uint2));
   const size_t need = o_cnt + 256;
   if ((need > ctx->bdev_bytes || n > ctx->bhost_cap) && ctx->capturing_now)
@@ -660,7 +668,7 @@ int ensure_batch_buffers(mdmc_ctx *ctx, uint32_t n) {
     }
     ctx->bhost_cap = 0;
     for (int i = 0; i < 2; ++i) {
-      if (hipHostMalloc(reinterpret_cast<void **>(&ctx->bhost[i]), kMaxBatch * sizeof(BatchVol)) != hipSuccess) {
+      if (hipHostMalloc(reinterpret_cast<void **>(&ctx->bhost[i]), batch_table_bytes(kMaxBatch)) != hipSuccess) {
         (void)hipGetLastError();
         return fail(MDMC_ERR_NOMEM, "pinned staging allocation failed");
       }
@@ -674,10 +682,10 @@ int ensure_batch_buffers(mdmc_ctx *ctx, uint32_t n) {
 
 BatchVol *batch_table_dev(mdmc_ctx *ctx) { return static_cast<BatchVol *>(ctx->bdev); }
 uint2 *batch_base_dev(mdmc_ctx *ctx, uint32_t n) {
-  return reinterpret_cast<uint2 *>(static_cast<char *>(ctx->bdev) + align256(n * sizeof(BatchVol)));
+  return reinterpret_cast<uint2 *>(static_cast<char *>(ctx->bdev) + align256(batch_table_bytes(n)));
 }
 uint32_t *batch_counts_dev(mdmc_ctx *ctx, uint32_t n) {
-  return reinterpret_cast<uint32_t *>(static_cast<char *>(ctx->bdev) + align256(n * sizeof(BatchVol)) +
+  return reinterpret_cast<uint32_t *>(static_cast<char *>(ctx->bdev) + align256(batch_table_bytes(n)) +
                                       align256(n * sizeof(uint2)));
 }
 
@@ -692,7 +700,7 @@ int staging_acquire(mdmc_ctx *ctx, int slot, hipStream_t st) {
 }
 
 int staging_upload(mdmc_ctx *ctx, int slot, uint32_t n, hipStream_t st) {
-  HIP_TRY(hipMemcpyAsync(ctx->bdev, ctx->bhost[slot], n * sizeof(BatchVol), hipMemcpyHostToDevice, st));
+  HIP_TRY(hipMemcpyAsync(ctx->bdev, ctx->bhost[slot], batch_table_bytes(n), hipMemcpyHostToDevice, st));
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cs));
   if (cs == hipStreamCaptureStatusNone) {
@@ -712,6 +720,7 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
                      uint32_t W4, uint32_t KP, const Scratch &S, uint64_t *nsegs_total, uint64_t *cells_total,
                      uint32_t *tiles_total) {
   const uint32_t cap = 256u * W4;
+  uint32_t *const tiles0 = batch_tile_off(ctx->bhost[slot], n), *const segs0 = batch_seg_off(ctx->bhost[slot], n);
   uint64_t seg_off = 0, tile_off = 0, cells = 0, coord_off = 0;
   for (uint32_t v = 0; v < n; ++v) {
     const mdmc_volume &mv = vols[v];
@@ -729,11 +738,11 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     b.c.seg_counts = S.seg_counts + seg_off;
     b.c.slots = S.slots + seg_off * cap;
     b.c.gmap = S.gmap + seg_off * (cap / 64);
-    b.tile_off = (uint32_t)tile_off;
+    b.tile_off = tiles0[v] = (uint32_t)tile_off;
     b.NRB = NRB;
     b.NKP = NKP;
-    b.vec = (X >= 4 && (reinterpret_cast<uintptr_t>(mv.field) & 3u) == 0) ? 1u : 0u;
-    b.seg_off = (uint32_t)seg_off;
+    b.tail = empty ? kPtTailFull : pt_tail(X, XT, cap);
+    b.seg_off = segs0[v] = (uint32_t)seg_off;
     b.nsegs = (uint32_t)nsegs;
     b.mnx = mv.xyz_min[0];
     b.mny = mv.xyz_min[1];
@@ -753,6 +762,7 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     tile_off += (uint64_t)XT * NRB * NKP;
     cells += (uint64_t)cx * cy * cz;
   }
+  tiles0[n] = (uint32_t)tile_off;
   *nsegs_total = seg_off;
   *cells_total = cells;
   *tiles_total = (uint32_t)tile_off;
@@ -852,6 +862,7 @@ int batch_count(mdmc_ctx *ctx, const mdmc_volume *vols, uint32_t n, mdmc_counts 
   uint32_t *bcounts = batch_counts_dev(ctx, n);
   BatchArgs ba{};
   ba.vols = batch_table_dev(ctx);
+  ba.tile_off = batch_tile_off(ctx->bdev, n);
   ba.nvol = n;
   ba.total_tiles = tiles;
   ba.zero.scan_state = S.scan_state;
@@ -943,6 +954,7 @@ int batch_emit(mdmc_ctx *ctx, const mdmc_volume *vols, uint32_t n, mdmc_counts *
   be.a.totals = S.totals;
   be.a.v.status = batch_counts_dev(ctx, n) + 3;
   be.vols = batch_table_dev(ctx);
+  be.seg_off = batch_seg_off(ctx->bdev, n);
   be.base = batch_base_dev(ctx, n);
   be.nvol = n;
   {

@@ -18,7 +18,6 @@ struct Plan {
   uint64_t nsegs, nslots, max_chunks, classify_blocks;
   uint64_t ncoord;  // point coordinates kept for the emit: X + Y + Z (summed over a batch)
   int empty;
-  int vec4;    // rows hold at least 4 points: 16-byte row loads
   int zmarch;  // use the z-marching classify kernel
   uint32_t ptR, ptKP;        // plane tiles: cell rows, cell planes
   uint32_t band, NKBp, NRBp; // plane tiles: columns per group, plane blocks, row blocks
@@ -67,12 +66,25 @@ inline int launch_classify_w(uint32_t R, const ClassifyArgs &a, uint32_t blocks,
   }
 }
 
-template <int W4, int R, int KP>
-inline void launch_classify_pt_t(bool vec, const PtArgs &a, uint32_t blocks, hipStream_t st) {
-  if (vec)
-    hipLaunchKernelGGL((k_classify_pt<W4, R, KP, true>), dim3(blocks), dim3(kPtThreads), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_classify_pt<W4, R, KP, false>), dim3(blocks), dim3(kPtThreads), 0, st, a);
+template <int W4, int R, int KP, uint32_t TAIL>
+inline void launch_classify_pt_k(const PtArgs &a, uint32_t blocks, hipStream_t st) {
+  hipLaunchKernelGGL((k_classify_pt<W4, R, KP, TAIL>), dim3(blocks), dim3(kPtThreads), 0, st, a);
+}
+
+// TAILS: the shape has kernels for narrow last x-tiles (the default shapes).
+template <int W4, int R, int KP, bool TAILS = false>
+inline void launch_classify_pt_t(uint32_t tail, const PtArgs &a, uint32_t blocks, hipStream_t st) {
+  if (tail == kPtTailTiny) return launch_classify_pt_k<W4, R, KP, kPtTailTiny>(a, blocks, st);
+  if constexpr (TAILS) {
+    if (tail == kPtTail16) return launch_classify_pt_k<W4, R, KP, kPtTail16>(a, blocks, st);
+    if (tail == kPtTail32) return launch_classify_pt_k<W4, R, KP, kPtTail32>(a, blocks, st);
+    if constexpr (W4 == 2) {
+      if (tail == kPtTail64) return launch_classify_pt_k<W4, R, KP, kPtTail64>(a, blocks, st);
+      if (tail == kPtTail256_16) return launch_classify_pt_k<W4, R, KP, kPtTail256_16>(a, blocks, st);
+      if (tail == kPtTail256_32) return launch_classify_pt_k<W4, R, KP, kPtTail256_32>(a, blocks, st);
+    }
+  }
+  launch_classify_pt_k<W4, R, KP, kPtTailFull>(a, blocks, st);
 }
 
 // Compiled plane-tile shapes besides the defaults (pt_rows, pt_planes).
@@ -84,21 +96,21 @@ inline bool pt_shape_supported(uint32_t W4, int R, int KP) {
 // cell planes of the 15-row shapes by default
 inline uint32_t pt_planes15(uint32_t W4) { return W4 == 1 ? 2u : 1u; }
 
-// Plane-tile kernel (W = 4, 8 or 16); vec: 16-byte row loads.
-inline int launch_classify_pt(uint32_t W, uint32_t R, uint32_t KP, bool vec, const PtArgs &a,
+// Plane-tile kernel (W = 4, 8 or 16); tail: parts of the last x-tile (pt_tail).
+inline int launch_classify_pt(uint32_t W, uint32_t R, uint32_t KP, uint32_t tail, const PtArgs &a,
                               uint32_t blocks, hipStream_t st) {
   switch (W) {
     case 4:
-      if (R == 7 && KP == 4) { launch_classify_pt_t<1, 7, 4>(vec, a, blocks, st); return 0; }
-      if (R == 15 && KP == 2) { launch_classify_pt_t<1, 15, 2>(vec, a, blocks, st); return 0; }
+      if (R == 7 && KP == 4) { launch_classify_pt_t<1, 7, 4, true>(tail, a, blocks, st); return 0; }
+      if (R == 15 && KP == 2) { launch_classify_pt_t<1, 15, 2>(tail, a, blocks, st); return 0; }
       return -1;
     case 8:
-      if (R == 7 && KP == 2) { launch_classify_pt_t<2, 7, 2>(vec, a, blocks, st); return 0; }
-      if (R == 7 && KP == 3) { launch_classify_pt_t<2, 7, 3>(vec, a, blocks, st); return 0; }
-      if (R == 15 && KP == 1) { launch_classify_pt_t<2, 15, 1>(vec, a, blocks, st); return 0; }
-      if (R == 15 && KP == 2) { launch_classify_pt_t<2, 15, 2>(vec, a, blocks, st); return 0; }
+      if (R == 7 && KP == 2) { launch_classify_pt_t<2, 7, 2, true>(tail, a, blocks, st); return 0; }
+      if (R == 7 && KP == 3) { launch_classify_pt_t<2, 7, 3>(tail, a, blocks, st); return 0; }
+      if (R == 15 && KP == 1) { launch_classify_pt_t<2, 15, 1>(tail, a, blocks, st); return 0; }
+      if (R == 15 && KP == 2) { launch_classify_pt_t<2, 15, 2>(tail, a, blocks, st); return 0; }
       return -1;
-    case 16: launch_classify_pt_t<4, (int)pt_rows(4), (int)pt_planes(4)>(vec, a, blocks, st); return 0;
+    case 16: launch_classify_pt_t<4, (int)pt_rows(4), (int)pt_planes(4)>(tail, a, blocks, st); return 0;
     default: return -1;
   }
 }

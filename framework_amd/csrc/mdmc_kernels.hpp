@@ -128,6 +128,17 @@ __device__ __forceinline__ uint32_t wave_incl_scan_dpp(uint32_t x) {
   return x;
 }
 
+// The same over each 16 or 32 lanes.
+template <int LW>
+__device__ __forceinline__ uint32_t row_incl_scan_dpp(uint32_t x) {
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowShr + 1, 0xF, 0xF, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowShr + 2, 0xF, 0xF, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowShr + 4, 0xF, 0xF, true);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowShr + 8, 0xF, 0xF, true);
+  if constexpr (LW >= 32) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowBcast15, 0xA, 0xF, false);
+  return x;
+}
+
 __device__ __forceinline__ uint32_t mbcnt64(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -400,6 +411,22 @@ struct PtArgs {
 constexpr uint32_t pt_rows(uint32_t) { return 7u; }
 constexpr uint32_t pt_planes(uint32_t W4) { return W4 >= 4 ? 1u : (W4 == 2 ? 2u : 4u); }
 
+// Parts of a row's last x-tile, by its points (see PtWide): full chunks << 8 |
+// lanes of the narrow part.  kPtTailFull: the x-tile's full mapping (also
+// where the narrow part's 32-bit lane offsets do not reach).  kPtTailTiny:
+// rows of less than 4 points, which a 16-byte load would leave.
+constexpr uint32_t kPtTailFull = 0u, kPtTailTiny = 1u, kPtTail16 = 16u, kPtTail32 = 32u, kPtTail64 = 64u,
+                   kPtTail256_16 = 256u + 16u, kPtTail256_32 = 256u + 32u;
+__host__ __device__ constexpr uint32_t pt_tail(uint32_t X, uint32_t XT, uint32_t cap) {
+  const uint32_t np = X - (XT - 1u) * cap;  // points of the last x-tile
+  if (X < 4u) return kPtTailTiny;
+  if (X > (1u << 24) || cap > 512u) return kPtTailFull;
+  if (np <= 64u) return kPtTail16;
+  if (np <= 128u) return kPtTail32;
+  if (cap == 256u) return kPtTailFull;
+  return np <= 256u ? kPtTail64 : np <= 320u ? kPtTail256_16 : np <= 384u ? kPtTail256_32 : kPtTailFull;
+}
+
 template <int W4, int R, int KP>
 struct PtShape {
   static_assert(W4 >= 1 && W4 <= 4, "x-tile is at most 1024 cells");
@@ -448,98 +475,243 @@ __device__ __forceinline__ void zero_scan_state(const ClassifyArgs &a, uint32_t 
 // 4 consecutive points of a row (16 bytes at the alignment of a float).
 typedef float Float4Row __attribute__((ext_vector_type(4), aligned(4)));
 
-// One plane tile (x-tile xt, row block rb, plane block kb) of the volume `a`.
-// VEC: rows hold at least 4 points, so a lane's 4 points are one 16-byte load
-// (the rows may start anywhere: the load needs the alignment of a float only);
-// otherwise 4 separate loads.
-template <int W4, int R, int KP, bool VEC>
-__device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t xt, uint32_t rb,
-                                                 uint32_t kb, uint32_t *s_w, uint32_t *s_tab,
-                                                 uint32_t tab_entry = 0u, bool store_tab = false) {
-  using S = PtShape<W4, R, KP>;
-  static_assert(KP * R <= kPtRowsMax, "row counts are staged in kPtRowsMax LDS entries");
-  uint2 *s_cnt = reinterpret_cast<uint2 *>(s_tab + 512);
-  constexpr int kRowsPerWave = (R + 1) / 4;
-  constexpr uint32_t CAP = 256u * W4;
-  constexpr uint32_t kRowWords = S::kRowWords;
-  constexpr uint32_t kPlaneWords = S::kPlaneWords;
-  const uint32_t lane = lane_id(), wave = wave_id();
-  const FieldDesc g = a.g;
-  const float iso = g.iso;
-  const uint32_t k = kb * KP;  // first cell plane of the tile
-  const uint32_t j0 = rb * R;
-  const bool tile_ok = (k < g.cz) && (j0 < g.cy);  // padding tiles do nothing
-  const uint32_t x0 = xt * CAP;
-  const size_t plane = (size_t)g.X * g.Y;
-  const bool has_extra = x0 + CAP < g.X;
+// Bit q: cell xb + q lies in the grid.
+__device__ __forceinline__ uint32_t cells_in_grid(uint32_t xb, uint32_t cx) {
+  return xb >= cx ? 0u : (cx - xb >= 4u ? 0xFu : (1u << (cx - xb)) - 1u);
+}
 
-  // ---- phase 1.  All loads are issued first, from in-bounds addresses:
-  // rows and planes past the grid are clamped to its last row / plane and
-  // lanes past the row end to its last 4 points; the cells that would use
-  // such values lie outside the grid and are never classified.
-  if (tile_ok) {
-    float4 v[kRowsPerWave][KP + 1][W4];
-    float ve[kRowsPerWave][KP + 1];
-    uint32_t xob[W4][VEC ? 1 : 4];  // byte offsets of the lane's points in a row
-    uint32_t xsh[W4];               // points its load starts before its first point
+// One 256-point chunk of a wave: a lane's 4 cells (corner bits w, LDS word
+// widx, lane l of the row's kRowWords) of cell row r, plane cp of the tile.
+struct PtChunk {
+  uint32_t widx, l, xb, x0, xvalid;  // xb: x of the first cell; xvalid: bit q, cell xb + q is in the grid
+  uint32_t y, z, r, cp, seg, grp;    // grp: the 64-cell group of the x-tile
+  uint32_t cnt_a, cnt_v, cnt_q;  // counts of the row before this chunk
+  bool yin, zin, interior;       // interior: every cell and its owned edges' rings lie in the grid
+};
+
+// Writes the chunk's records and group maps; returns the lane's inclusive
+// scan of the counts (active | vertices << 9 | quads << 20) over the LW lanes
+// that hold one row (64 or more: the wave), 0 when nothing is active.
+template <int LW, uint32_t CAP, uint32_t kRowWords, uint32_t kPlaneWords, int R, int KP>
+__device__ __forceinline__ uint32_t classify_chunk(const ClassifyArgs &a, const PtChunk &ch, uint32_t w,
+                                                   const uint32_t *s_w, const uint32_t *s_tab) {
+  const FieldDesc &g = a.g;
+  const uint32_t lane = lane_id();
+  const uint32_t widx = ch.widx, xb = ch.xb, x0 = ch.x0, y = ch.y, z = ch.z, r = ch.r, cp = ch.cp;
+  const bool yin = ch.yin, zin = ch.zin;
+  // all 20 corner bits equal -> none of the lane's 4 cells is active
+  if (__ballot(w != 0u && w != 0x1F1F1F1Fu) == 0ull) return 0u;
+  // per cell: key, and active (bit 0 of the second table entry)
+  uint32_t keys = 0, lact = 0;
 #pragma unroll
-    for (int c = 0; c < W4; ++c) {
-      if constexpr (VEC) {
-        // the lane that holds the row's end loads the row's last 4 points and
-        // shifts its sign bits (lanes past the end hold bits no cell uses)
-        const uint32_t xs = x0 + 256u * c + 4u * lane, xl = min(xs, g.X - 4u);
-        xob[c][0] = xl * 4u;
-        xsh[c] = min(xs - xl, 4u);
-      } else {
-        xsh[c] = 0u;
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t tq = (w >> q) & 0x03030303u;
+    const uint32_t key = ((tq * 0x41041u) >> 18) & 0xFFu;
+    keys |= key << (8 * q);
+    lact |= (s_tab[256u + key] & 1u) << q;
+  }
+  lact &= ch.xvalid;
+  if (__ballot(lact != 0u) == 0ull) return 0u;
+  // first table entry of each active cell (0 for inactive cells, so they
+  // count nothing)
+  uint32_t e4[4];
+  uint32_t amb = 0;  // bit q: cell q is a 2B/3B configuration
 #pragma unroll
-        for (int e = 0; e < 4; ++e) xob[c][e] = min(x0 + 256u * c + 4u * lane + (uint32_t)e, g.X - 1u) * 4u;
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t ent = s_tab[(keys >> (8 * q)) & 0xFFu];
+    e4[q] = ((lact >> q) & 1u) ? ent : 0u;
+    amb |= ((e4[q] >> 11) & 1u) << q;
+  }
+  const bool any_amb = __ballot(amb != 0u) != 0ull;
+  // 2B/3B cells (rare): the variant depends on the neighbour across the
+  // listed face.  Inside the tile the neighbour's corner bits are in LDS
+  // (the word one cell or lane over, or of the next row or plane); only a
+  // neighbour outside the tile is read from the field.
+  uint32_t l2m = 0;
+  if (any_amb) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (!((amb >> q) & 1u)) continue;
+      const uint32_t face = (e4[q] >> 12) & 7u;
+      int nx = (int)(xb + q), ny = (int)y, nz = (int)z;
+      bool in_tile;
+      uint32_t nidx = widx, nq = (uint32_t)q;
+      switch (face) {
+        case 0:
+          nx += 1;
+          in_tile = q < 3 || ch.l + 1u < kRowWords;
+          nidx = widx + (q == 3 ? 1u : 0u);
+          nq = (uint32_t)(q + 1) & 3u;
+          break;
+        case 1:
+          nx -= 1;
+          in_tile = q > 0 || ch.l > 0u;
+          nidx = widx - (q == 0 ? 1u : 0u);
+          nq = (uint32_t)(q + 3) & 3u;
+          break;
+        case 2: ny += 1; in_tile = r + 1u < (uint32_t)R; nidx = widx + kRowWords; break;
+        case 3: ny -= 1; in_tile = r > 0u; nidx = widx - kRowWords; break;
+        case 4: nz += 1; in_tile = cp + 1u < (uint32_t)KP; nidx = widx + kPlaneWords; break;
+        default: nz -= 1; in_tile = cp > 0u; nidx = widx - kPlaneWords; break;
       }
+      if (nx < 0 || ny < 0 || nz < 0 || nx >= (int)g.cx || ny >= (int)g.cy || nz >= (int)g.cz) continue;
+      uint32_t ent;
+      if (in_tile) {
+        const uint32_t tq = (s_w[nidx] >> nq) & 0x03030303u;
+        ent = s_tab[((tq * 0x41041u) >> 18) & 0xFFu];
+      } else {
+        ent = c_cfg_count[cell_cfg_global(g, (uint32_t)nx, (uint32_t)ny, (uint32_t)nz)];
+      }
+      l2m |= ((ent >> 11) & 1u) << q;
     }
-    const uint32_t xe = has_extra ? x0 + CAP : 0u;
+  }
+  // per cell: variant, vertex count, quad count; per-cell byte: nv (3
+  // bits) | nq (2 bits) << 3 | variant << 5
+  uint32_t pk = 0, info4 = 0, cfgs = 0;
+  if (ch.interior && !any_amb) {
+    // interior chunk (every cell and its owned edges' rings in the grid)
+    // without 2B/3B cells: the second table has it all
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t e2 = s_tab[256u + ((keys >> (8 * q)) & 0xFFu)];
+      cfgs |= (e4[q] >> 16) << (8 * q);
+      pk += e2 & 0x00FFFFFFu;
+      info4 |= (e2 >> 24) << (8 * q);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t e = e4[q] & 0xFFFFu, l2 = (l2m >> q) & 1u;
+      cfgs |= (e4[q] >> 16) << (8 * q);
+      const uint32_t nv = (e >> (4 * l2)) & 0xFu;
+      const bool xin = xb + q + 1 < g.cx;
+      const uint32_t qmask = (uint32_t)(xin && yin) | ((uint32_t)(xin && zin) << 1) |
+                             ((uint32_t)(yin && zin) << 2);
+      const uint32_t nq = (uint32_t)__popc((e >> 8) & 7u & qmask);
+      info4 |= (nv | (nq << 3) | (l2 << 5)) << (8 * q);
+      pk += ((lact >> q) & 1u) | (nv << 9) | (nq << 20);
+    }
+  }
+  const uint32_t incl = LW >= kWave ? wave_incl_scan_dpp(pk) : row_incl_scan_dpp<LW>(pk);
+  const uint32_t excl = incl - pk;
+  {
+    // Group map: the 16 lanes of a DPP row hold the 64 cells of one group
+    // (4 per lane); OR their nibbles into lane 15 of the row.
+    uint32_t mlo = (lane & 8u) ? 0u : lact << (4u * (lane & 7u));
+    uint32_t mhi = (lane & 8u) ? lact << (4u * (lane & 7u)) : 0u;
+    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 1, 0xF, 0xF, true);
+    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 1, 0xF, 0xF, true);
+    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 2, 0xF, 0xF, true);
+    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 2, 0xF, 0xF, true);
+    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 4, 0xF, 0xF, true);
+    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 4, 0xF, 0xF, true);
+    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 8, 0xF, 0xF, true);
+    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 8, 0xF, 0xF, true);
+    if ((lane & 15u) == 15u && (mlo | mhi) != 0u) {
+      const uint32_t first = ch.cnt_a + (incl & 0x1FFu) - (uint32_t)(__popc(mlo) + __popc(mhi));
+      a.gmap[(size_t)ch.seg * (CAP / 64u) + ch.grp] = make_uint4(mlo, mhi, first, 0u);
+    }
+  }
+  if (lact) {
+    uint32_t rank = ch.cnt_a + (excl & 0x1FFu);
+    uint32_t lvb = ch.cnt_v + ((excl >> 9) & 0x7FFu);
+    uint32_t lqb = ch.cnt_q + (excl >> 20);
+    uint64_t *dst = a.slots + (size_t)ch.seg * CAP;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (!((lact >> q) & 1u)) continue;
+      const uint32_t b = (info4 >> (8 * q)) & 0xFFu;
+      dst[rank] = make_record(xb + q - x0, (cfgs >> (8 * q)) & 0xFFu, b >> 5, lvb, lqb);
+      rank += 1;
+      lvb += b & 7u;
+      lqb += (b >> 3) & 3u;
+    }
+  }
+  return incl;
+}
+
+// The tile's row counts leave in one store (a store per row costs more).
+template <int R, int KP>
+__device__ __forceinline__ void store_row_counts(const ClassifyArgs &a, uint32_t xt, uint32_t j0, uint32_t k,
+                                                 const uint2 *s_cnt) {
+  __syncthreads();
+  if (threadIdx.x < (uint32_t)(KP * R)) {
+    const uint32_t m = threadIdx.x, cp = m / R, r = m - cp * R;
+    const uint32_t y = j0 + r, z = k + cp;
+    if (y < a.g.cy && z < a.g.cz) a.seg_counts[xt + a.XT * (y + a.g.cy * z)] = s_cnt[m];
+  }
+}
+
+// A tile's columns are C full chunks of 256 points (a lane holds 4 points of a
+// row, a wave takes one row at a time) and then, when LW is not 0, up to 4*LW
+// points of which a wave takes 64 / LW rows at a time, LW lanes each.  The
+// narrow part is for narrow grids and for the end of a row: there the full
+// mapping leaves most lanes past the row's end and costs as much.  x0 is the
+// part's first point.
+//
+// All loads of a part are issued first, from in-bounds addresses: rows and
+// planes past the grid are clamped to its last row / plane and lanes past the
+// row end to its last 4 points; the cells that would use such values lie
+// outside the grid and are never classified.
+template <int C, int R, int KP>
+struct PtWide {
+  static constexpr int kRowsPerWave = (R + 1) / 4;
+  static constexpr uint32_t kRowWords = C * kWave;
+  static constexpr uint32_t kPlaneWords = kRowWords * (R + 2);
+  Float4Row v[kRowsPerWave][KP + 1][C];
+  float ve[kRowsPerWave][KP + 1];
+  uint32_t xsh[C];  // points a lane's load starts before its first point
+
+  __device__ __forceinline__ void load(const FieldDesc &g, uint32_t x0, uint32_t k, uint32_t j0) {
+    const uint32_t lane = lane_id(), wave = wave_id();
+    const size_t plane = (size_t)g.X * g.Y;
+    // the lane that holds the row's end loads the row's last 4 points and
+    // shifts its sign bits (lanes past the end hold bits no cell uses)
+    uint32_t xob[C];  // byte offset of the lane's points in a row
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const uint32_t xs = x0 + 256u * c + 4u * lane, xl = min(xs, g.X - 4u);
+      xob[c] = xl * 4u;
+      xsh[c] = min(xs - xl, 4u);
+    }
+    const uint32_t xe = x0 + 256u * C < g.X ? x0 + 256u * C : 0u;
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) {
       const size_t yoff = (size_t)min(j0 + wave + 4u * i, g.Y - 1u) * g.X;
 #pragma unroll
       for (int p = 0; p <= KP; ++p) {
         const float *rowp = g.f + (size_t)min(k + p, g.Z - 1u) * plane + yoff;
-        const char *rowb = reinterpret_cast<const char *>(rowp);
 #pragma unroll
-        for (int c = 0; c < W4; ++c) {
-          if constexpr (VEC) {
-            const Float4Row w = *reinterpret_cast<const Float4Row *>(rowb + xob[c][0]);
-            v[i][p][c] = make_float4(w.x, w.y, w.z, w.w);
-          } else {
-            v[i][p][c].x = *reinterpret_cast<const float *>(rowb + xob[c][0]);
-            v[i][p][c].y = *reinterpret_cast<const float *>(rowb + xob[c][1]);
-            v[i][p][c].z = *reinterpret_cast<const float *>(rowb + xob[c][2]);
-            v[i][p][c].w = *reinterpret_cast<const float *>(rowb + xob[c][3]);
-          }
-        }
+        for (int c = 0; c < C; ++c)
+          v[i][p][c] = *reinterpret_cast<const Float4Row *>(reinterpret_cast<const char *>(rowp) + xob[c]);
         ve[i][p] = rowp[xe];
       }
     }
+  }
+
+  __device__ __forceinline__ void store(float iso, uint32_t *s_w) const {
+    const uint32_t lane = lane_id(), wave = wave_id();
     uint16_t *s_h = reinterpret_cast<uint16_t *>(s_w);
     const uint32_t base = wave * kRowWords + lane;
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) {
-      uint32_t v5[KP + 1][W4];
+      uint32_t v5[KP + 1][C];
 #pragma unroll
       for (int p = 0; p <= KP; ++p) {
-        uint32_t nib[W4];
+        uint32_t nib[C];
 #pragma unroll
-        for (int c = 0; c < W4; ++c) {
+        for (int c = 0; c < C; ++c) {
           nib[c] = (uint32_t)(v[i][p][c].x < iso) | ((uint32_t)(v[i][p][c].y < iso) << 1) |
                    ((uint32_t)(v[i][p][c].z < iso) << 2) | ((uint32_t)(v[i][p][c].w < iso) << 3);
-          if constexpr (VEC) nib[c] >>= xsh[c];
+          nib[c] >>= xsh[c];
         }
         const uint32_t ext = (uint32_t)(ve[i][p] < iso);
 #pragma unroll
-        for (int c = 0; c < W4; ++c) {
-          // first point of lane+1, or of the next chunk / next x-tile for lane 63
+        for (int c = 0; c < C; ++c) {
+          // first point of lane+1, or of the next chunk / the point past the part for lane 63
           uint32_t nb = lane_next(nib[c]);
           const uint32_t nxt =
-              (c + 1 < W4) ? (uint32_t)__builtin_amdgcn_readfirstlane(nib[(c + 1 < W4) ? c + 1 : c]) : ext;
+              (c + 1 < C) ? (uint32_t)__builtin_amdgcn_readfirstlane(nib[(c + 1 < C) ? c + 1 : c]) : ext;
           if (lane == kWave - 1) nb = nxt;
           v5[p][c] = nib[c] | ((nb & 1u) << 4);
         }
@@ -547,7 +719,7 @@ __device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t
 #pragma unroll
       for (int cp = 0; cp < KP; ++cp) {
 #pragma unroll
-        for (int c = 0; c < W4; ++c) {
+        for (int c = 0; c < C; ++c) {
           const uint16_t h = (uint16_t)(v5[cp][c] | (v5[cp + 1][c] << 8));
           // cell row r = wave + 4i sits at padded row r + 1; cell row r - 1 at r
           s_h[2u * (base + cp * kPlaneWords + (4u * i + 1u) * kRowWords + c * kWave)] = h;
@@ -556,179 +728,171 @@ __device__ __forceinline__ void classify_pt_tile(const ClassifyArgs &a, uint32_t
       }
     }
   }
+
+  // each wave classifies cell rows wave, wave+4, ... of the KP*R rows of the
+  // tile; the rows' counts go to s_cnt
+  template <uint32_t CAP>
+  __device__ static __forceinline__ void classify(const ClassifyArgs &a, uint32_t xt, uint32_t k, uint32_t j0,
+                                                  const uint32_t *s_w, const uint32_t *s_tab, uint2 *s_cnt) {
+    const FieldDesc &g = a.g;
+    const uint32_t lane = lane_id(), wave = wave_id();
+    const uint32_t x0 = xt * CAP;
+    uint32_t xvalid[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) xvalid[c] = cells_in_grid(x0 + 256u * c + 4u * lane, g.cx);
+    for (uint32_t m = wave; m < (uint32_t)(KP * R); m += kPtThreads / kWave) {
+      const uint32_t cp = m / R, r = m - cp * R;
+      const uint32_t y = j0 + r, z = k + cp;
+      if (y >= g.cy || z >= g.cz) continue;
+      const bool yin = y + 1 < g.cy, zin = z + 1 < g.cz;
+      uint32_t cnt_a = 0, cnt_v = 0, cnt_q = 0;
+      const uint32_t seg = xt + a.XT * (y + g.cy * z);
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const uint32_t widx = cp * kPlaneWords + (r + 1u) * kRowWords + c * kWave + lane;
+        const PtChunk ch{widx, lane + kWave * c, x0 + 256u * c + 4u * lane, x0, xvalid[c], y, z, r, cp, seg,
+                         4u * c + (lane >> 4), cnt_a, cnt_v, cnt_q, yin, zin,
+                         yin && zin && x0 + 256u * (c + 1u) < g.cx};
+        const uint32_t incl = classify_chunk<kWave, CAP, kRowWords, kPlaneWords, R, KP>(a, ch, s_w[widx], s_w, s_tab);
+        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        cnt_a += tot & 0x1FFu;
+        cnt_v += (tot >> 9) & 0x7FFu;
+        cnt_q += tot >> 20;
+      }
+      if (lane == 0) s_cnt[m] = make_uint2(cnt_a | (cnt_q << 16), cnt_v);
+    }
+  }
+};
+
+// TINY: rows of 2 or 3 points, read one point at a time.
+template <int LW, int R, int KP, bool TINY>
+struct PtNarrow {
+  static_assert(LW == 16 || LW == 32 || LW == 64, "whole DPP rows");
+  static constexpr int SR = kWave / LW;                // rows side by side in a wave
+  static constexpr int NS = (R + 1) / SR;              // sets of SR point rows in the tile
+  static constexpr int SPLIT = NS >= 4 ? 1 : 4 / NS;   // waves that share a row set, each with its cell planes
+  static constexpr int PP = (KP + SPLIT - 1) / SPLIT;  // cell planes of a wave
+  static constexpr int NI = NS >= 4 ? NS / 4 : 1;      // row sets of a wave
+  static constexpr uint32_t kPlaneWords = LW * (R + 2);
+  static_assert((R + 1) % SR == 0 && 4 % SPLIT == 0 && (NS % 4 == 0 || NS < 4), "row sets cover the point rows");
+  Float4Row v[NI][PP + 1];
+  uint32_t xsh;
+
+  __device__ static __forceinline__ uint32_t set0() { return wave_id() % (4u / SPLIT); }
+  __device__ static __forceinline__ uint32_t plane0() { return wave_id() / (4u / SPLIT) * PP; }
+
+  __device__ __forceinline__ void load(const FieldDesc &g, uint32_t x0, uint32_t k, uint32_t j0) {
+    const uint32_t lane = lane_id(), l = lane % LW, sub = lane / LW;
+    const size_t plane = (size_t)g.X * g.Y;
+    const uint32_t xs = x0 + 4u * l, xl = TINY ? 0u : min(xs, g.X - 4u);
+    xsh = TINY ? 0u : min(xs - xl, 4u);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t row = min(j0 + (set0() + 4u * i) * SR + sub, g.Y - 1u) - j0;
+      const uint32_t off = (row * g.X + xl) * 4u;
+#pragma unroll
+      for (int p = 0; p <= PP; ++p) {
+        const float *base = g.f + (size_t)min(k + plane0() + p, g.Z - 1u) * plane + (size_t)j0 * g.X;
+        if constexpr (TINY) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[i][p][e] = base[row * g.X + min((uint32_t)e, g.X - 1u)];
+        } else {
+          v[i][p] = *reinterpret_cast<const Float4Row *>(reinterpret_cast<const char *>(base) + off);
+        }
+      }
+    }
+  }
+
+  __device__ __forceinline__ void store(float iso, uint32_t *s_w) const {
+    const uint32_t lane = lane_id(), l = lane % LW, sub = lane / LW;
+    uint16_t *s_h = reinterpret_cast<uint16_t *>(s_w);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      uint32_t v5[PP + 1];
+#pragma unroll
+      for (int p = 0; p <= PP; ++p) {
+        const uint32_t nib = ((uint32_t)(v[i][p].x < iso) | ((uint32_t)(v[i][p].y < iso) << 1) |
+                              ((uint32_t)(v[i][p].z < iso) << 2) | ((uint32_t)(v[i][p].w < iso) << 3)) >> xsh;
+        v5[p] = nib | ((lane_next(nib) & 1u) << 4);  // (a row's last lane: a bit no cell uses)
+      }
+      const uint32_t r = (set0() + 4u * i) * SR + sub;  // cell row r sits at padded row r + 1, r - 1 at r
+#pragma unroll
+      for (int p = 0; p < PP; ++p) {
+        const uint32_t cp = plane0() + p;
+        if (cp >= (uint32_t)KP) continue;
+        const uint16_t h = (uint16_t)(v5[p] | (v5[p + 1] << 8));
+        s_h[2u * (cp * kPlaneWords + (r + 1u) * LW + l)] = h;
+        s_h[2u * (cp * kPlaneWords + r * LW + l) + 1u] = h;
+      }
+    }
+  }
+
+  // the part's columns start xoff points into the x-tile; with CARRY the rows'
+  // counts before it are in s_cnt
+  template <uint32_t CAP, bool CARRY>
+  __device__ static __forceinline__ void classify(const ClassifyArgs &a, uint32_t xt, uint32_t xoff, uint32_t k,
+                                                  uint32_t j0, const uint32_t *s_w, const uint32_t *s_tab,
+                                                  uint2 *s_cnt) {
+    const FieldDesc &g = a.g;
+    const uint32_t lane = lane_id(), wave = wave_id(), l = lane % LW, sub = lane / LW;
+    const uint32_t x0 = xt * CAP, xb = x0 + xoff + 4u * l, in_x = cells_in_grid(xb, g.cx);
+    for (uint32_t m0 = wave * SR; m0 < (uint32_t)(KP * R); m0 += 4u * SR) {
+      const uint32_t m = m0 + sub, cp = m / R, r = m - cp * R;
+      const uint32_t y = j0 + r, z = k + cp;
+      const bool row_ok = m < (uint32_t)(KP * R), ok = row_ok && y < g.cy && z < g.cz;
+      const uint32_t widx = ok ? cp * kPlaneWords + (r + 1u) * LW + l : 0u;
+      const uint2 before = CARRY && ok ? s_cnt[m] : make_uint2(0u, 0u);
+      const PtChunk ch{widx, l, xb, x0, ok ? in_x : 0u, y, z, r, cp, xt + a.XT * (y + g.cy * z),
+                       (xoff >> 6) + (l >> 4), before.x & 0xFFFFu, before.y, before.x >> 16,
+                       y + 1 < g.cy, z + 1 < g.cz, false};
+      const uint32_t incl =
+          classify_chunk<LW, CAP, (uint32_t)LW, kPlaneWords, R, KP>(a, ch, ok ? s_w[widx] : 0u, s_w, s_tab);
+      if (l == LW - 1 && row_ok)
+        s_cnt[m] = make_uint2(before.x + ((incl & 0x1FFu) | ((incl >> 20) << 16)), before.y + ((incl >> 9) & 0x7FFu));
+    }
+  }
+};
+
+// One plane tile with the parts TAIL names (pt_tail).
+template <uint32_t TAIL, uint32_t CAP, int R, int KP>
+__device__ __forceinline__ void classify_pt_parts(const ClassifyArgs &a, uint32_t xt, uint32_t k, uint32_t j0,
+                                                  uint32_t *s_w, uint32_t *s_tab, uint32_t tab_entry,
+                                                  bool store_tab) {
+  uint2 *s_cnt = reinterpret_cast<uint2 *>(s_tab + 512);
+  constexpr bool TINY = TAIL == kPtTailTiny;
+  constexpr int C = TAIL == kPtTailFull ? (int)(CAP / 256u) : TINY ? 0 : (int)(TAIL >> 8);
+  constexpr int LW = TAIL == kPtTailFull ? 0 : TINY ? 16 : (int)(TAIL & 0xFFu);
+  using W = PtWide<C ? C : 1, R, KP>;
+  using N = PtNarrow<LW ? LW : 16, R, KP, TINY>;
+  const bool tile_ok = (k < a.g.cz) && (j0 < a.g.cy);  // padding tiles do nothing
+  const uint32_t x0 = xt * CAP;
+  uint32_t *const s_n = s_w + (C ? KP * W::kPlaneWords : 0u);  // the narrow part's words
+  if (tile_ok) {
+    W w;
+    N n;
+    if constexpr (LW != 0) n.load(a.g, x0 + 256u * C, k, j0);
+    if constexpr (C != 0) w.load(a.g, x0, k, j0);
+    if constexpr (LW != 0) n.store(a.g.iso, s_n);
+    if constexpr (C != 0) w.store(a.g.iso, s_w);
+  }
   // the table entry was loaded before the field rows; storing it here keeps
   // its wait behind theirs
   if (store_tab) pt_store_tables(s_tab, tab_entry);
   __syncthreads();
   if (!tile_ok) return;  // uniform over the workgroup
-
-  // ---- phase 2: each wave classifies cell rows wave, wave+4, ... of the
-  // KP*R rows of the tile
-  uint32_t xvalid[W4];  // bit q: cell x0 + 256c + 4 lane + q lies in the grid
-#pragma unroll
-  for (int c = 0; c < W4; ++c) {
-    const uint32_t xb = x0 + 256u * c + 4u * lane;
-    xvalid[c] = xb >= g.cx ? 0u : (g.cx - xb >= 4u ? 0xFu : (1u << (g.cx - xb)) - 1u);
+  if constexpr (C != 0) W::template classify<CAP>(a, xt, k, j0, s_w, s_tab, s_cnt);
+  if constexpr (LW != 0) {
+    if constexpr (C != 0) __syncthreads();  // the full chunks' counts
+    N::template classify<CAP, C != 0>(a, xt, 256u * C, k, j0, s_n, s_tab, s_cnt);
   }
-  for (uint32_t m = wave; m < (uint32_t)(KP * R); m += kPtThreads / kWave) {
-    const uint32_t cp = m / R, r = m - cp * R;
-    const uint32_t y = j0 + r, z = k + cp;
-    if (y >= g.cy || z >= g.cz) continue;
-    const bool yin = y + 1 < g.cy, zin = z + 1 < g.cz;
-    uint32_t cnt_a = 0, cnt_v = 0, cnt_q = 0;
-    const uint32_t seg = xt + a.XT * (y + g.cy * z);
-#pragma unroll
-    for (int c = 0; c < W4; ++c) {
-      const uint32_t w = s_w[cp * kPlaneWords + (r + 1u) * kRowWords + c * kWave + lane];
-      // all 20 corner bits equal -> none of the lane's 4 cells is active
-      if (__ballot(w != 0u && w != 0x1F1F1F1Fu) == 0ull) continue;
-      const uint32_t xb = x0 + 256u * c + 4u * lane;
-      // per cell: key, and active (bit 0 of the second table entry)
-      uint32_t keys = 0, lact = 0;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t tq = (w >> q) & 0x03030303u;
-        const uint32_t key = ((tq * 0x41041u) >> 18) & 0xFFu;
-        keys |= key << (8 * q);
-        lact |= (s_tab[256u + key] & 1u) << q;
-      }
-      lact &= xvalid[c];
-      if (__ballot(lact != 0u) == 0ull) continue;
-      // first table entry of each active cell (0 for inactive cells, so they
-      // count nothing)
-      uint32_t e4[4];
-      uint32_t amb = 0;  // bit q: cell q is a 2B/3B configuration
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t ent = s_tab[(keys >> (8 * q)) & 0xFFu];
-        e4[q] = ((lact >> q) & 1u) ? ent : 0u;
-        amb |= ((e4[q] >> 11) & 1u) << q;
-      }
-      const bool any_amb = __ballot(amb != 0u) != 0ull;
-      // 2B/3B cells (rare): the variant depends on the neighbour across the
-      // listed face.  Inside the tile the neighbour's corner bits are in LDS
-      // (the word one cell or lane over, or of the next row or plane); only a
-      // neighbour outside the tile is read from the field.
-      uint32_t l2m = 0;
-      if (any_amb) {
-        const uint32_t widx = cp * kPlaneWords + (r + 1u) * kRowWords + c * kWave + lane;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          if (!((amb >> q) & 1u)) continue;
-          const uint32_t face = (e4[q] >> 12) & 7u;
-          int nx = (int)(xb + q), ny = (int)y, nz = (int)z;
-          bool in_tile;
-          uint32_t nidx = widx, nq = (uint32_t)q;
-          switch (face) {
-            case 0:
-              nx += 1;
-              in_tile = q < 3 || lane + kWave * c + 1u < kWave * W4;
-              nidx = widx + (q == 3 ? 1u : 0u);
-              nq = (uint32_t)(q + 1) & 3u;
-              break;
-            case 1:
-              nx -= 1;
-              in_tile = q > 0 || lane + kWave * c > 0u;
-              nidx = widx - (q == 0 ? 1u : 0u);
-              nq = (uint32_t)(q + 3) & 3u;
-              break;
-            case 2: ny += 1; in_tile = r + 1u < (uint32_t)R; nidx = widx + kRowWords; break;
-            case 3: ny -= 1; in_tile = r > 0u; nidx = widx - kRowWords; break;
-            case 4: nz += 1; in_tile = cp + 1u < (uint32_t)KP; nidx = widx + kPlaneWords; break;
-            default: nz -= 1; in_tile = cp > 0u; nidx = widx - kPlaneWords; break;
-          }
-          if (nx < 0 || ny < 0 || nz < 0 || nx >= (int)g.cx || ny >= (int)g.cy || nz >= (int)g.cz) continue;
-          uint32_t ent;
-          if (in_tile) {
-            const uint32_t tq = (s_w[nidx] >> nq) & 0x03030303u;
-            ent = s_tab[((tq * 0x41041u) >> 18) & 0xFFu];
-          } else {
-            ent = c_cfg_count[cell_cfg_global(g, (uint32_t)nx, (uint32_t)ny, (uint32_t)nz)];
-          }
-          l2m |= ((ent >> 11) & 1u) << q;
-        }
-      }
-      // per cell: variant, vertex count, quad count; per-cell byte: nv (3
-      // bits) | nq (2 bits) << 3 | variant << 5
-      uint32_t pk = 0, info4 = 0, cfgs = 0;
-      if (yin && zin && x0 + 256u * (c + 1u) < g.cx && !any_amb) {
-        // interior chunk (every cell and its owned edges' rings in the grid)
-        // without 2B/3B cells: the second table has it all
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t e2 = s_tab[256u + ((keys >> (8 * q)) & 0xFFu)];
-          cfgs |= (e4[q] >> 16) << (8 * q);
-          pk += e2 & 0x00FFFFFFu;
-          info4 |= (e2 >> 24) << (8 * q);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t e = e4[q] & 0xFFFFu, l2 = (l2m >> q) & 1u;
-          cfgs |= (e4[q] >> 16) << (8 * q);
-          const uint32_t nv = (e >> (4 * l2)) & 0xFu;
-          const bool xin = xb + q + 1 < g.cx;
-          const uint32_t qmask = (uint32_t)(xin && yin) | ((uint32_t)(xin && zin) << 1) |
-                                 ((uint32_t)(yin && zin) << 2);
-          const uint32_t nq = (uint32_t)__popc((e >> 8) & 7u & qmask);
-          info4 |= (nv | (nq << 3) | (l2 << 5)) << (8 * q);
-          pk += ((lact >> q) & 1u) | (nv << 9) | (nq << 20);
-        }
-      }
-      const uint32_t incl = wave_incl_scan_dpp(pk);
-      const uint32_t excl = incl - pk;
-      const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-      {
-        // Group map: the 16 lanes of a DPP row hold the 64 cells of one group
-        // (4 per lane); OR their nibbles into lane 15 of the row.
-        uint32_t mlo = (lane & 8u) ? 0u : lact << (4u * (lane & 7u));
-        uint32_t mhi = (lane & 8u) ? lact << (4u * (lane & 7u)) : 0u;
-        mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 1, 0xF, 0xF, true);
-        mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 1, 0xF, 0xF, true);
-        mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 2, 0xF, 0xF, true);
-        mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 2, 0xF, 0xF, true);
-        mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 4, 0xF, 0xF, true);
-        mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 4, 0xF, 0xF, true);
-        mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 8, 0xF, 0xF, true);
-        mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 8, 0xF, 0xF, true);
-        if ((lane & 15u) == 15u && (mlo | mhi) != 0u) {
-          const uint32_t first = cnt_a + (incl & 0x1FFu) - (uint32_t)(__popc(mlo) + __popc(mhi));
-          a.gmap[(size_t)seg * (CAP / 64u) + 4u * c + (lane >> 4)] = make_uint4(mlo, mhi, first, 0u);
-        }
-      }
-      if (lact) {
-        uint32_t rank = cnt_a + (excl & 0x1FFu);
-        uint32_t lvb = cnt_v + ((excl >> 9) & 0x7FFu);
-        uint32_t lqb = cnt_q + (excl >> 20);
-        uint64_t *dst = a.slots + (size_t)seg * CAP;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          if (!((lact >> q) & 1u)) continue;
-          const uint32_t b = (info4 >> (8 * q)) & 0xFFu;
-          dst[rank] = make_record(xb + q - x0, (cfgs >> (8 * q)) & 0xFFu, b >> 5, lvb, lqb);
-          rank += 1;
-          lvb += b & 7u;
-          lqb += (b >> 3) & 3u;
-        }
-      }
-      cnt_a += tot & 0x1FFu;
-      cnt_v += (tot >> 9) & 0x7FFu;
-      cnt_q += tot >> 20;
-    }
-    if (lane == 0) s_cnt[m] = make_uint2(cnt_a | (cnt_q << 16), cnt_v);
-  }
-  // the tile's row counts leave in one store (a store per row costs more)
-  __syncthreads();
-  if (threadIdx.x < (uint32_t)(KP * R)) {
-    const uint32_t m = threadIdx.x, cp = m / R, r = m - cp * R;
-    const uint32_t y = j0 + r, z = k + cp;
-    if (y < g.cy && z < g.cz) a.seg_counts[xt + a.XT * (y + g.cy * z)] = s_cnt[m];
-  }
+  store_row_counts<R, KP>(a, xt, j0, k, s_cnt);
 }
 
 // Single volume: block b -> tile through the XCD mapping (pt_tile_of).
-template <int W4, int R, int KP, bool VEC>
+// TAIL: the parts of the last x-tile.
+template <int W4, int R, int KP, uint32_t TAIL>
 __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >= 4 ? 4 : 8, W4 >= 4 ? 4 : 8))) void k_classify_pt(PtArgs pa) {
+  static_assert(KP * R <= kPtRowsMax, "row counts are staged in kPtRowsMax LDS entries");
   __shared__ uint32_t s_w[PtShape<W4, R, KP>::kLdsWords];
   __shared__ __align__(16) uint32_t s_tab[kPtTabWords];
   const ClassifyArgs &a = pa.c;
@@ -738,7 +902,11 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
     if (a.counts_out != nullptr && threadIdx.x < 4) a.counts_out[threadIdx.x] = 0u;
   }
   const PtTile t = pt_tile_of(blockIdx.x, a.XT, pa.NRB, pa.NKB, pa.B);
-  classify_pt_tile<W4, R, KP, VEC>(a, t.xt, t.rb, t.kb, s_w, s_tab, tab, true);
+  constexpr uint32_t CAP = 256u * W4;
+  if (TAIL != kPtTailFull && t.xt + 1u == a.XT)
+    classify_pt_parts<TAIL, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, s_tab, tab, true);
+  else if (TAIL != kPtTailTiny)
+    classify_pt_parts<kPtTailFull, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, s_tab, tab, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -751,9 +919,9 @@ constexpr uint32_t kMaxBatch = 1024;  // volumes per batch call
 
 struct BatchVol {
   ClassifyArgs c;         // per-volume field and tiling; record pointers start at seg_off
-  uint32_t tile_off;      // first flattened classify tile
   uint32_t NRB, NKP;      // row blocks and plane blocks of the volume
-  uint32_t vec;           // rows hold at least 4 points (16-byte row loads)
+  uint32_t tail;          // parts of the last x-tile (pt_tail)
+  uint32_t tile_off;      // first flattened classify tile
   uint32_t seg_off, nsegs;
   float mnx, mny, mnz, rgx, rgy, rgz;
   float *verts;
@@ -767,9 +935,24 @@ struct BatchVol {
 
 struct BatchArgs {
   BatchVol *vols;
+  const uint32_t *tile_off;  // first tile of each volume, then the total
   uint32_t nvol, total_tiles;
   ClassifyArgs zero;      // scan state of the batch (zeroed by block 0)
 };
+
+// Last volume v with off[v] <= t (off ascending, off[0] <= t; volumes without
+// tiles share an entry with the next).  The 64 lanes test every stride-th
+// entry, then the entries of the stride found: two loads and two ballots, no
+// table in LDS (a workgroup that first copied the offsets from the volume
+// descriptors touched a cache line per volume).
+__device__ __forceinline__ uint32_t volume_of(const uint32_t *off, uint32_t nvol, uint32_t t) {
+  static_assert(kMaxBatch <= kWave * kWave, "two rounds of 64");
+  const uint32_t lane = lane_id(), stride = (nvol + kWave - 1u) / kWave;
+  const uint32_t i = lane * stride;
+  const uint32_t m = (uint32_t)__popcll(__ballot(i < nvol && off[min(i, nvol - 1u)] <= t)) - 1u;
+  const uint32_t j = m * stride + lane;
+  return m * stride + (uint32_t)__popcll(__ballot(lane < stride && j < nvol && off[min(j, nvol - 1u)] <= t)) - 1u;
+}
 
 // Classify over the flattened tiles of all volumes (tiles of a volume in
 // memory order): with a grid of at least the tile count a workgroup per tile,
@@ -778,10 +961,7 @@ template <int W4, int R, int KP>
 __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 == 1 ? 8 : (W4 == 2 ? 6 : 4), W4 == 1 ? 8 : (W4 == 2 ? 6 : 4)))) void k_classify_batch(BatchArgs b) {
   __shared__ uint32_t s_w[PtShape<W4, R, KP>::kLdsWords];
   __shared__ __align__(16) uint32_t s_tab[kPtTabWords];
-  __shared__ uint32_t s_toff[kMaxBatch + 1];
   pt_init_table(s_tab);
-  for (uint32_t i = threadIdx.x; i <= b.nvol; i += kPtThreads)
-    s_toff[i] = i < b.nvol ? b.vols[i].tile_off : b.total_tiles;
   if (blockIdx.x == 0) {
     zero_scan_state(b.zero, threadIdx.x, kPtThreads);
     if (threadIdx.x < 4) b.zero.counts_out[threadIdx.x] = 0u;  // the batch's scan counts
@@ -798,22 +978,40 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 =
     t_step = (G >> 3) + (x < (G & 7u) ? 1u : 0u);
   }
   for (; t < t_end; t += t_step) {
-    // volume of tile t: the last v with tile_off[v] <= t
-    uint32_t lo = 0, hi = b.nvol;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (s_toff[mid] <= t) lo = mid; else hi = mid;
-    }
-    const uint32_t v = __builtin_amdgcn_readfirstlane(lo);
-    const BatchVol &bv = b.vols[v];
-    const ClassifyArgs &a = bv.c;
-    const uint32_t local = t - s_toff[v];
+    const uint32_t v = volume_of(b.tile_off, b.nvol, t);
+    // the volume's descriptor through the constant address space (nothing in
+    // this launch writes it), so that its fields are scalar loads and not
+    // vector registers
+    const __attribute__((address_space(4))) BatchVol *bv = (const __attribute__((address_space(4))) BatchVol *)b.vols + v;
+    ClassifyArgs a{};
+    a.g.f = bv->c.g.f;
+    a.g.X = bv->c.g.X;
+    a.g.Y = bv->c.g.Y;
+    a.g.Z = bv->c.g.Z;
+    a.g.cx = bv->c.g.cx;
+    a.g.cy = bv->c.g.cy;
+    a.g.cz = bv->c.g.cz;
+    a.g.iso = bv->c.g.iso;
+    a.XT = bv->c.XT;
+    a.seg_counts = bv->c.seg_counts;
+    a.slots = bv->c.slots;
+    a.gmap = bv->c.gmap;
+    const uint32_t nrb = bv->NRB;
+    const uint32_t local = t - bv->tile_off;
     const uint32_t xt = local % a.XT, u = local / a.XT;
     __syncthreads();  // the previous tile's LDS words are no longer read
-    if (bv.vec)
-      classify_pt_tile<W4, R, KP, true>(a, xt, u % bv.NRB, u / bv.NRB, s_w, s_tab);
+    const uint32_t k = u / nrb * KP, j0 = u % nrb * R, tail = xt + 1u == a.XT ? bv->tail : kPtTailFull;
+    constexpr uint32_t CAP = 256u * W4;
+    if (W4 <= 2 && tail == kPtTail16)
+      classify_pt_parts<kPtTail16, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+    else if (W4 <= 2 && tail == kPtTail32)
+      classify_pt_parts<kPtTail32, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+    else if (W4 == 2 && tail == kPtTail64)
+      classify_pt_parts<kPtTail64, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+    else if (tail == kPtTailTiny)
+      classify_pt_parts<kPtTailTiny, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
     else
-      classify_pt_tile<W4, R, KP, false>(a, xt, u % bv.NRB, u / bv.NRB, s_w, s_tab);
+      classify_pt_parts<kPtTailFull, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
   }
 }
 
@@ -1963,6 +2161,7 @@ __global__ __launch_bounds__(256) void k_coords_batch(const BatchVol *vols, uint
 struct BatchEmitArgs {
   EmitArgs a;  // arrays of the whole batch; a.v.status is the batch status word
   const BatchVol *vols;
+  const uint32_t *seg_off;  // first segment of each volume
   const uint2 *base;
   uint32_t nvol;
 };
@@ -1980,7 +2179,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
   const uint32_t num_chunks = (uint32_t)min((uint64_t)tot.num_chunks, a.max_chunks);
   if (!workgroup_has_chunks(num_chunks)) return;  // (uniform: before the barrier)
   for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = (&c_label[0][0])[i];
-  for (uint32_t i = threadIdx.x; i < b.nvol; i += kEmitThreads) s_soff[i] = b.vols[i].seg_off;
+  for (uint32_t i = threadIdx.x; i < b.nvol; i += kEmitThreads) s_soff[i] = b.seg_off[i];
   __syncthreads();
   const uint32_t lane = lane_id(), wave = wave_id();
   const uint32_t num_ne = min(tot.num_nonempty, a.nsegs);
