@@ -4,13 +4,13 @@
 //
 //   k_classify_pt  dense pass over the field in plane tiles (7 cell rows x
 //               one x-tile x 1-4 cell planes per 256-thread workgroup): point
-//               rows staged in LDS as sign bits, per-cell configuration keys
-//               by multiply-shift, uniform 256-cell chunks skipped with one
-//               ballot; active cells get their 2B/3B table variant, vertex and
-//               quad counts, a DPP-scan rank and a 64-bit record in their
-//               segment's slot range (segment = one cell row of one x-tile in
-//               one plane), plus a per-64-cell group map (active mask, first
-//               rank).  Workgroups map to tiles XCD by XCD (mdmc_tilemap.h).
+//               rows staged in LDS as sign bits, uniform 256-cell chunks
+//               skipped with one ballot, active cells found by bit operations
+//               and listed in LDS; listed cells get their 2B/3B table variant,
+//               vertex and quad counts, a DPP-scan rank and a 64-bit record in
+//               their segment's slot range (segment = one cell row of one
+//               x-tile in one plane), plus a per-64-cell group map (active
+//               mask, first rank).  Workgroups map to tiles XCD by XCD (mdmc_tilemap.h).
 //               k_classify is the z-marching form for any row length.
 //   k_scan      single-pass decoupled look-back scan (ticketed tiles) over the
 //               segment totals: vertex/quad bases per segment, the non-empty
@@ -386,10 +386,11 @@ __global__ __launch_bounds__(64) void k_classify(ClassifyArgs a) {
 // (the LDS has one padding row above and below, so every store is
 // unconditional and every address is the wave's base plus a constant).
 // Phase 2: each wave takes cell rows w, w+4, ...; one LDS read gives all 20
-// corner bits of the lane's 4 cells.  For cell q, t = (w >> q) & 0x03030303
-// holds the corner pairs (p0,p1), (p4,p5), (p3,p2), (p7,p6) in its bytes and
-// (t * 0x41041) >> 18 gathers them into an 8-bit key, which indexes a table of
-// configuration and counts.
+// corner bits of a lane's 4 cells.  The active ones go to a list, and the list
+// is classified a cell per lane (PtList): for a cell, t = (w >> q) &
+// 0x03030303 holds the corner pairs (p0,p1), (p4,p5), (p3,p2), (p7,p6) in its
+// bytes and (t * 0x41041) >> 18 gathers them into an 8-bit key, which indexes
+// a table of configuration and counts.
 constexpr int kPtThreads = 256;
 
 // key bits p0 p1 p4 p5 p3 p2 p7 p6 -> configuration bits p0..p7
@@ -437,32 +438,21 @@ struct PtShape {
   static constexpr uint32_t kLdsWords = KP * kPlaneWords;
 };
 
-// Two tables indexed by key, then the staging of a tile's row counts
-// (kPtRowsMax uint2):
-//   s_tab[key]        c_cfg_count of the key's configuration | cfg << 16
-//   s_tab[256 + key]  an interior cell's contribution, variant 0, all three
-//                     owned edges' rings in the grid: 1 | nv << 9 | nq << 20 (the
-//                     packed counts the wave scan adds up) | (nv | nq << 3) << 24
-//                     (its record byte); 0 for the inactive keys 0 and 255
-constexpr uint32_t kPtRowsMax = 64;
-constexpr uint32_t kPtTabWords = 512 + 2 * kPtRowsMax;
-// This thread's entry of the first table (a global load) ...
+// LDS of a tile besides its corner words.
+constexpr uint32_t kPtRowsMax = 64;    // cell rows of a tile
+constexpr uint32_t kPtListLen = 512;   // entries of a wave's list of active cells (a ring)
+struct PtShared {
+  uint32_t tab[256];                        // by key: c_cfg_count of its configuration | cfg << 16
+  uint2 cnt[kPtRowsMax];                    // row counts {active | quads << 16, vertices}
+  uint2 cnt2[kPtRowsMax];                   // the same of a second part
+  uint2 row[kPtRowsMax];                    // {segment, first list entry | y + 1, z + 1 in the grid << 16, 17}
+  uint16_t list[kPtThreads / kWave][kPtListLen];  // active cells: row << 10 | x in the x-tile
+};
+// This thread's entry of the table (a global load).
 __device__ __forceinline__ uint32_t pt_table_entry() {
   const uint32_t cfg = key_to_cfg(threadIdx.x);
   return (uint32_t)c_cfg_count[cfg] | (cfg << 16);
 }
-// ... its entry of the second, from it ...
-__device__ __forceinline__ uint32_t pt_table2_entry(uint32_t tab) {
-  const uint32_t cfg = tab >> 16, nv = tab & 0xFu, nq = (uint32_t)__popc((tab >> 8) & 7u);
-  if (cfg == 0u || cfg == 0xFFu) return 0u;
-  return 1u | (nv << 9) | (nq << 20) | ((nv | (nq << 3)) << 24);
-}
-// ... and both tables in LDS (the caller synchronises).
-__device__ __forceinline__ void pt_store_tables(uint32_t *s_tab, uint32_t tab) {
-  s_tab[threadIdx.x] = tab;
-  s_tab[256 + threadIdx.x] = pt_table2_entry(tab);
-}
-__device__ __forceinline__ void pt_init_table(uint32_t *s_tab) { pt_store_tables(s_tab, pt_table_entry()); }
 
 // Zeroes the state the scan expects to start from (first workgroup only).
 __device__ __forceinline__ void zero_scan_state(const ClassifyArgs &a, uint32_t tid, uint32_t nthreads) {
@@ -480,125 +470,75 @@ __device__ __forceinline__ uint32_t cells_in_grid(uint32_t xb, uint32_t cx) {
   return xb >= cx ? 0u : (cx - xb >= 4u ? 0xFu : (1u << (cx - xb)) - 1u);
 }
 
-// One 256-point chunk of a wave: a lane's 4 cells (corner bits w, LDS word
-// widx, lane l of the row's kRowWords) of cell row r, plane cp of the tile.
-struct PtChunk {
-  uint32_t widx, l, xb, x0, xvalid;  // xb: x of the first cell; xvalid: bit q, cell xb + q is in the grid
-  uint32_t y, z, r, cp, seg, grp;    // grp: the 64-cell group of the x-tile
-  uint32_t cnt_a, cnt_v, cnt_q;  // counts of the row before this chunk
-  bool yin, zin, interior;       // interior: every cell and its owned edges' rings lie in the grid
-};
+// Cells of a lane that are active, as 4 bits, from its 20 corner bits w: cell
+// q is when bits q and q + 1 of the four rows are not all alike.
+__device__ __forceinline__ uint32_t active_cells(uint32_t w) {
+  const uint32_t o2 = w | (w >> 16), a2 = w & (w >> 16);
+  const uint32_t o = o2 | (o2 >> 8), n = a2 & (a2 >> 8);
+  return (o | (o >> 1)) & ~(n & (n >> 1)) & 0xFu;
+}
+// Whether any of them can be (all 20 corner bits equal: none is).
+__device__ __forceinline__ bool may_be_active(uint32_t w) { return w != 0u && w != 0x1F1F1F1Fu; }
 
-// Writes the chunk's records and group maps; returns the lane's inclusive
-// scan of the counts (active | vertices << 9 | quads << 20) over the LW lanes
-// that hold one row (64 or more: the wave), 0 when nothing is active.
-template <int LW, uint32_t CAP, uint32_t kRowWords, uint32_t kPlaneWords, int R, int KP>
-__device__ __forceinline__ uint32_t classify_chunk(const ClassifyArgs &a, const PtChunk &ch, uint32_t w,
-                                                   const uint32_t *s_w, const uint32_t *s_tab) {
-  const FieldDesc &g = a.g;
-  const uint32_t lane = lane_id();
-  const uint32_t widx = ch.widx, xb = ch.xb, x0 = ch.x0, y = ch.y, z = ch.z, r = ch.r, cp = ch.cp;
-  const bool yin = ch.yin, zin = ch.zin;
-  // all 20 corner bits equal -> none of the lane's 4 cells is active
-  if (__ballot(w != 0u && w != 0x1F1F1F1Fu) == 0ull) return 0u;
-  // per cell: key, and active (bit 0 of the second table entry)
-  uint32_t keys = 0, lact = 0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const uint32_t tq = (w >> q) & 0x03030303u;
-    const uint32_t key = ((tq * 0x41041u) >> 18) & 0xFFu;
-    keys |= key << (8 * q);
-    lact |= (s_tab[256u + key] & 1u) << q;
+// The second phase of a tile.  Each wave walks its cell rows (append): it finds
+// the active cells of a chunk of 256 from their corner bits, writes the group
+// maps, and appends the cells to a list of its own in LDS; whenever the list
+// holds 64 (and at the end) it classifies 64 of them, a cell per lane (drain):
+// table lookup, 2B/3B check, vertex and quad numbers by one wave scan over the
+// list, records.  A row's cells follow each other in the list, so a record's
+// numbers are the scan minus its value at the row's start.
+//
+// Classifying from the list instead of 4 cells per lane in place is what the
+// list is for: most chunks that hold a surface hold a few active cells, and
+// the lanes' 4 cells in sequence made a chain of some thousand cycles for each
+// such chunk, up to 8 chunks one after the other in a wave (classify of 256^3
+// blobs 33 -> 23 us, 384^3 60 -> 49 us, 603x487x399 142 -> 129 us; the 1024^3
+// gyroid, where every lane has work, 1.50 -> 1.44 ms: 7.0 GB moved).
+template <uint32_t CAP, uint32_t kRowWords, uint32_t kPlaneWords, int R, bool CARRY>
+struct PtList {
+  const ClassifyArgs &a;
+  const uint32_t *s_w;
+  PtShared &sh;
+  uint32_t xt, xoff, k, j0;  // x-tile, first cell of the part in it, first plane and row of the tile
+  uint32_t have = 0, done = 0;     // entries appended, classified
+  uint32_t run = 0, row_run = 0;   // vertices | quads << 16 before the next entry, before its row
+  uint16_t *list;
+
+  __device__ __forceinline__ PtList(const ClassifyArgs &a_, const uint32_t *w, PtShared &s, uint32_t xt_,
+                                    uint32_t xoff_, uint32_t k_, uint32_t j0_)
+      : a(a_), s_w(w), sh(s), xt(xt_), xoff(xoff_), k(k_), j0(j0_), list(s.list[wave_id()]) {}
+
+  static constexpr uint32_t kDivR = (1024u + R - 1u) / R;  // m / R for m < kPtRowsMax
+  __device__ static constexpr bool div_ok() {
+    for (uint32_t m = 0; m < kPtRowsMax; ++m)
+      if (m * kDivR / 1024u != m / R) return false;
+    return true;
   }
-  lact &= ch.xvalid;
-  if (__ballot(lact != 0u) == 0ull) return 0u;
-  // first table entry of each active cell (0 for inactive cells, so they
-  // count nothing)
-  uint32_t e4[4];
-  uint32_t amb = 0;  // bit q: cell q is a 2B/3B configuration
+  static_assert(R >= 1 && R <= 31, "rows of a tile");
+
+  // counts of row m before this part
+  __device__ __forceinline__ uint2 before(uint32_t m) const { return CARRY ? sh.cnt[m] : make_uint2(0u, 0u); }
+
+  // A lane's 4 cells in row m from xl in the x-tile: `act` their active bits,
+  // `incl` the inclusive sum of the active cells over the row's lanes so far,
+  // `pos` the list index of the lane's first.
+  __device__ __forceinline__ void append(uint32_t m, uint32_t xl, uint32_t act, uint32_t pos) {
+    const uint32_t e = m << 10 | xl;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const uint32_t ent = s_tab[(keys >> (8 * q)) & 0xFFu];
-    e4[q] = ((lact >> q) & 1u) ? ent : 0u;
-    amb |= ((e4[q] >> 11) & 1u) << q;
-  }
-  const bool any_amb = __ballot(amb != 0u) != 0ull;
-  // 2B/3B cells (rare): the variant depends on the neighbour across the
-  // listed face.  Inside the tile the neighbour's corner bits are in LDS
-  // (the word one cell or lane over, or of the next row or plane); only a
-  // neighbour outside the tile is read from the field.
-  uint32_t l2m = 0;
-  if (any_amb) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (!((amb >> q) & 1u)) continue;
-      const uint32_t face = (e4[q] >> 12) & 7u;
-      int nx = (int)(xb + q), ny = (int)y, nz = (int)z;
-      bool in_tile;
-      uint32_t nidx = widx, nq = (uint32_t)q;
-      switch (face) {
-        case 0:
-          nx += 1;
-          in_tile = q < 3 || ch.l + 1u < kRowWords;
-          nidx = widx + (q == 3 ? 1u : 0u);
-          nq = (uint32_t)(q + 1) & 3u;
-          break;
-        case 1:
-          nx -= 1;
-          in_tile = q > 0 || ch.l > 0u;
-          nidx = widx - (q == 0 ? 1u : 0u);
-          nq = (uint32_t)(q + 3) & 3u;
-          break;
-        case 2: ny += 1; in_tile = r + 1u < (uint32_t)R; nidx = widx + kRowWords; break;
-        case 3: ny -= 1; in_tile = r > 0u; nidx = widx - kRowWords; break;
-        case 4: nz += 1; in_tile = cp + 1u < (uint32_t)KP; nidx = widx + kPlaneWords; break;
-        default: nz -= 1; in_tile = cp > 0u; nidx = widx - kPlaneWords; break;
+    for (uint32_t q = 0; q < 4; ++q) {
+      if ((act >> q) & 1u) {
+        list[pos & (kPtListLen - 1u)] = (uint16_t)(e + q);
+        ++pos;
       }
-      if (nx < 0 || ny < 0 || nz < 0 || nx >= (int)g.cx || ny >= (int)g.cy || nz >= (int)g.cz) continue;
-      uint32_t ent;
-      if (in_tile) {
-        const uint32_t tq = (s_w[nidx] >> nq) & 0x03030303u;
-        ent = s_tab[((tq * 0x41041u) >> 18) & 0xFFu];
-      } else {
-        ent = c_cfg_count[cell_cfg_global(g, (uint32_t)nx, (uint32_t)ny, (uint32_t)nz)];
-      }
-      l2m |= ((ent >> 11) & 1u) << q;
     }
   }
-  // per cell: variant, vertex count, quad count; per-cell byte: nv (3
-  // bits) | nq (2 bits) << 3 | variant << 5
-  uint32_t pk = 0, info4 = 0, cfgs = 0;
-  if (ch.interior && !any_amb) {
-    // interior chunk (every cell and its owned edges' rings in the grid)
-    // without 2B/3B cells: the second table has it all
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t e2 = s_tab[256u + ((keys >> (8 * q)) & 0xFFu)];
-      cfgs |= (e4[q] >> 16) << (8 * q);
-      pk += e2 & 0x00FFFFFFu;
-      info4 |= (e2 >> 24) << (8 * q);
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t e = e4[q] & 0xFFFFu, l2 = (l2m >> q) & 1u;
-      cfgs |= (e4[q] >> 16) << (8 * q);
-      const uint32_t nv = (e >> (4 * l2)) & 0xFu;
-      const bool xin = xb + q + 1 < g.cx;
-      const uint32_t qmask = (uint32_t)(xin && yin) | ((uint32_t)(xin && zin) << 1) |
-                             ((uint32_t)(yin && zin) << 2);
-      const uint32_t nq = (uint32_t)__popc((e >> 8) & 7u & qmask);
-      info4 |= (nv | (nq << 3) | (l2 << 5)) << (8 * q);
-      pk += ((lact >> q) & 1u) | (nv << 9) | (nq << 20);
-    }
-  }
-  const uint32_t incl = LW >= kWave ? wave_incl_scan_dpp(pk) : row_incl_scan_dpp<LW>(pk);
-  const uint32_t excl = incl - pk;
-  {
-    // Group map: the 16 lanes of a DPP row hold the 64 cells of one group
-    // (4 per lane); OR their nibbles into lane 15 of the row.
-    uint32_t mlo = (lane & 8u) ? 0u : lact << (4u * (lane & 7u));
-    uint32_t mhi = (lane & 8u) ? lact << (4u * (lane & 7u)) : 0u;
+
+  // Group maps of the groups that lanes 16 i .. 16 i + 15 hold; incl: active
+  // cells of the row up to and with this lane.
+  __device__ __forceinline__ void group_maps(uint32_t seg, uint32_t grp, uint32_t act, uint32_t incl) {
+    const uint32_t lane = lane_id();
+    uint32_t mlo = (lane & 8u) ? 0u : act << (4u * (lane & 7u));
+    uint32_t mhi = (lane & 8u) ? act << (4u * (lane & 7u)) : 0u;
     mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 1, 0xF, 0xF, true);
     mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 1, 0xF, 0xF, true);
     mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 2, 0xF, 0xF, true);
@@ -607,38 +547,107 @@ __device__ __forceinline__ uint32_t classify_chunk(const ClassifyArgs &a, const 
     mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 4, 0xF, 0xF, true);
     mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 8, 0xF, 0xF, true);
     mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 8, 0xF, 0xF, true);
-    if ((lane & 15u) == 15u && (mlo | mhi) != 0u) {
-      const uint32_t first = ch.cnt_a + (incl & 0x1FFu) - (uint32_t)(__popc(mlo) + __popc(mhi));
-      a.gmap[(size_t)ch.seg * (CAP / 64u) + ch.grp] = make_uint4(mlo, mhi, first, 0u);
-    }
+    if ((lane & 15u) == 15u && (mlo | mhi) != 0u)
+      a.gmap[(size_t)seg * (CAP / 64u) + grp] =
+          make_uint4(mlo, mhi, incl - (uint32_t)(__popc(mlo) + __popc(mhi)), 0u);
   }
-  if (lact) {
-    uint32_t rank = ch.cnt_a + (excl & 0x1FFu);
-    uint32_t lvb = ch.cnt_v + ((excl >> 9) & 0x7FFu);
-    uint32_t lqb = ch.cnt_q + (excl >> 20);
-    uint64_t *dst = a.slots + (size_t)ch.seg * CAP;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (!((lact >> q) & 1u)) continue;
-      const uint32_t b = (info4 >> (8 * q)) & 0xFFu;
-      dst[rank] = make_record(xb + q - x0, (cfgs >> (8 * q)) & 0xFFu, b >> 5, lvb, lqb);
-      rank += 1;
-      lvb += b & 7u;
-      lqb += (b >> 3) & 3u;
+
+  // Variant-1 test of a 2B/3B cell (its neighbour across the listed face is
+  // 2B/3B too).  Inside the part the neighbour's corner bits are in LDS (the
+  // word one cell or lane over, or of the next row or plane); only a neighbour
+  // outside is read from the field.
+  template <int KP>
+  __device__ __forceinline__ uint32_t variant1(uint32_t ent, uint32_t widx, uint32_t xl, uint32_t cp, uint32_t r) {
+    const FieldDesc &g = a.g;
+    const uint32_t face = (ent >> 12) & 7u, q = xl & 3u, l = (xl - xoff) >> 2;
+    int nx = (int)(xt * CAP + xl), ny = (int)(j0 + r), nz = (int)(k + cp);
+    bool in_part;
+    uint32_t nidx = widx, nq = q;
+    switch (face) {
+      case 0:
+        nx += 1;
+        in_part = q < 3u || l + 1u < kRowWords;
+        nidx = widx + (q == 3u ? 1u : 0u);
+        nq = (q + 1u) & 3u;
+        break;
+      case 1:
+        nx -= 1;
+        in_part = q > 0u || l > 0u;
+        nidx = widx - (q == 0u ? 1u : 0u);
+        nq = (q + 3u) & 3u;
+        break;
+      case 2: ny += 1; in_part = r + 1u < (uint32_t)R; nidx = widx + kRowWords; break;
+      case 3: ny -= 1; in_part = r > 0u; nidx = widx - kRowWords; break;
+      case 4: nz += 1; in_part = cp + 1u < (uint32_t)KP; nidx = widx + kPlaneWords; break;
+      default: nz -= 1; in_part = cp > 0u; nidx = widx - kPlaneWords; break;
     }
+    if (nx < 0 || ny < 0 || nz < 0 || nx >= (int)g.cx || ny >= (int)g.cy || nz >= (int)g.cz) return 0u;
+    uint32_t nent;
+    if (in_part) {
+      const uint32_t tq = (s_w[nidx] >> nq) & 0x03030303u;
+      nent = sh.tab[((tq * 0x41041u) >> 18) & 0xFFu];
+    } else {
+      nent = c_cfg_count[cell_cfg_global(g, (uint32_t)nx, (uint32_t)ny, (uint32_t)nz)];
+    }
+    return (nent >> 11) & 1u;
   }
-  return incl;
-}
+
+  // Classifies the next n (at most 64) entries.
+  template <int KP>
+  __device__ __forceinline__ void drain(uint32_t n) {
+    static_assert(div_ok(), "row index division");
+    const FieldDesc &g = a.g;
+    const uint32_t lane = lane_id();
+    const bool valid = lane < n;
+    const uint32_t e = valid ? list[(done + lane) & (kPtListLen - 1u)] : 0u;
+    const uint32_t m = e >> 10, xl = e & 0x3FFu;
+    const uint2 row = sh.row[m];
+    const uint2 bef = before(m);
+    const uint32_t cp = m * kDivR >> 10, r = m - cp * R, q = xl & 3u;
+    const uint32_t widx = cp * kPlaneWords + (r + 1u) * kRowWords + ((xl - xoff) >> 2);
+    const uint32_t tq = (valid ? s_w[widx] >> q : 0u) & 0x03030303u;
+    const uint32_t ent = sh.tab[((tq * 0x41041u) >> 18) & 0xFFu];
+    uint32_t l2 = 0u;
+    const bool amb = valid && ((ent >> 11) & 1u);
+    if (__ballot(amb) != 0ull) {  // rare
+      if (amb) l2 = variant1<KP>(ent, widx, xl, cp, r);
+    }
+    const uint32_t yin = (row.y >> 16) & 1u, zin = row.y >> 17;
+    const uint32_t xin = xt * CAP + xl + 1u < g.cx ? 1u : 0u;
+    const uint32_t qmask = (xin & yin) | ((xin & zin) << 1) | ((yin & zin) << 2);
+    const uint32_t nv = (l2 ? ent >> 4 : ent) & 0xFu, nq = (uint32_t)__popc((ent >> 8) & qmask);
+    const uint32_t pk = valid ? nv | (nq << 16) : 0u;
+    const uint32_t incl = run + wave_incl_scan_dpp(pk), excl = incl - pk;
+    // the entry's place in its row, and the scan's value at the row's start
+    const uint32_t rank = done + lane - (row.y & 0xFFFFu);
+    const uint32_t at_start = (uint32_t)__shfl((int)excl, (int)((lane - rank) & 63u), kWave);
+    const uint32_t st = rank <= lane ? at_start : row_run;
+    const uint32_t loc = excl - st;
+    if (valid)
+      a.slots[(size_t)row.x * CAP + (bef.x & 0xFFFFu) + rank] =
+          make_record(xl, (ent >> 16) & 0xFFu, l2, bef.y + (loc & 0xFFFFu), (bef.x >> 16) + (loc >> 16));
+    // the row's counts so far (its last entry writes the final ones)
+    const uint32_t next = lane_next(m);
+    if (valid && (lane + 1u == n || next != m)) {
+      const uint32_t tot = incl - st;
+      (CARRY ? sh.cnt2 : sh.cnt)[m] = make_uint2((rank + 1u) | (tot >> 16 << 16), tot & 0xFFFFu);
+    }
+    run = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    row_run = (uint32_t)__builtin_amdgcn_readlane((int)st, (int)(n - 1u));
+    done += n;
+  }
+};
 
 // The tile's row counts leave in one store (a store per row costs more).
-template <int R, int KP>
+template <int R, int KP, bool TWO>
 __device__ __forceinline__ void store_row_counts(const ClassifyArgs &a, uint32_t xt, uint32_t j0, uint32_t k,
-                                                 const uint2 *s_cnt) {
+                                                 const PtShared &sh) {
   __syncthreads();
   if (threadIdx.x < (uint32_t)(KP * R)) {
     const uint32_t m = threadIdx.x, cp = m / R, r = m - cp * R;
     const uint32_t y = j0 + r, z = k + cp;
-    if (y < a.g.cy && z < a.g.cz) a.seg_counts[xt + a.XT * (y + a.g.cy * z)] = s_cnt[m];
+    const uint2 c = sh.cnt[m], c2 = TWO ? sh.cnt2[m] : make_uint2(0u, 0u);
+    if (y < a.g.cy && z < a.g.cz) a.seg_counts[xt + a.XT * (y + a.g.cy * z)] = make_uint2(c.x + c2.x, c.y + c2.y);
   }
 }
 
@@ -730,37 +739,54 @@ struct PtWide {
   }
 
   // each wave classifies cell rows wave, wave+4, ... of the KP*R rows of the
-  // tile; the rows' counts go to s_cnt
+  // tile; the rows' counts go to sh.cnt
   template <uint32_t CAP>
   __device__ static __forceinline__ void classify(const ClassifyArgs &a, uint32_t xt, uint32_t k, uint32_t j0,
-                                                  const uint32_t *s_w, const uint32_t *s_tab, uint2 *s_cnt) {
+                                                  const uint32_t *s_w, PtShared &sh) {
     const FieldDesc &g = a.g;
     const uint32_t lane = lane_id(), wave = wave_id();
-    const uint32_t x0 = xt * CAP;
-    uint32_t xvalid[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) xvalid[c] = cells_in_grid(x0 + 256u * c + 4u * lane, g.cx);
-    for (uint32_t m = wave; m < (uint32_t)(KP * R); m += kPtThreads / kWave) {
+    constexpr int RW = (KP * R + 3) / 4;  // rows of a wave
+    static_assert(RW * C <= 32, "chunks of a wave in one mask");
+    auto word = [&](uint32_t m, int c) {
       const uint32_t cp = m / R, r = m - cp * R;
-      const uint32_t y = j0 + r, z = k + cp;
-      if (y >= g.cy || z >= g.cz) continue;
-      const bool yin = y + 1 < g.cy, zin = z + 1 < g.cz;
-      uint32_t cnt_a = 0, cnt_v = 0, cnt_q = 0;
-      const uint32_t seg = xt + a.XT * (y + g.cy * z);
+      return cp * kPlaneWords + (r + 1u) * kRowWords + c * kWave + lane;
+    };
+    // the chunks that can hold active cells (the words are read together; rows
+    // past the tile read its last row's)
+    uint32_t w[RW][C], live = 0;
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) w[i][c] = s_w[word(min(wave + 4u * i, (uint32_t)(KP * R - 1)), c)];
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) live |= __ballot(may_be_active(w[i][c])) != 0ull ? 1u << (i * C + c) : 0u;
+    }
+    if (live == 0u) return;
+    const uint32_t x0 = xt * CAP;
+    PtList<CAP, kRowWords, kPlaneWords, R, false> L(a, s_w, sh, xt, 0u, k, j0);
+    for (int i = 0; i < RW; ++i) {
+      if (!((live >> (i * C)) & ((1u << C) - 1u))) continue;
+      const uint32_t m = wave + 4u * i, cp = m / R, y = j0 + m - cp * R, z = k + cp;
+      if (m >= (uint32_t)(KP * R) || y >= g.cy || z >= g.cz) continue;
+      const uint32_t seg = xt + a.XT * (y + g.cy * z), start = L.have;
+      if (lane == 0)
+        sh.row[m] = make_uint2(seg, start | (y + 1u < g.cy ? 1u << 16 : 0u) | (z + 1u < g.cz ? 1u << 17 : 0u));
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        const uint32_t widx = cp * kPlaneWords + (r + 1u) * kRowWords + c * kWave + lane;
-        const PtChunk ch{widx, lane + kWave * c, x0 + 256u * c + 4u * lane, x0, xvalid[c], y, z, r, cp, seg,
-                         4u * c + (lane >> 4), cnt_a, cnt_v, cnt_q, yin, zin,
-                         yin && zin && x0 + 256u * (c + 1u) < g.cx};
-        const uint32_t incl = classify_chunk<kWave, CAP, kRowWords, kPlaneWords, R, KP>(a, ch, s_w[widx], s_w, s_tab);
-        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-        cnt_a += tot & 0x1FFu;
-        cnt_v += (tot >> 9) & 0x7FFu;
-        cnt_q += tot >> 20;
+        if (!((live >> (i * C + c)) & 1u)) continue;
+        const uint32_t act = active_cells(s_w[word(m, c)]) & cells_in_grid(x0 + 256u * c + 4u * lane, g.cx);
+        if (__ballot(act != 0u) == 0ull) continue;
+        const uint32_t cnt = (uint32_t)__popc(act), incl = wave_incl_scan_dpp(cnt);
+        L.group_maps(seg, 4u * c + (lane >> 4), act, L.have - start + incl);
+        L.append(m, 256u * c + 4u * lane, act, L.have + incl - cnt);
+        L.have += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        while (L.have - L.done >= (uint32_t)kWave) L.template drain<KP>(kWave);
       }
-      if (lane == 0) s_cnt[m] = make_uint2(cnt_a | (cnt_q << 16), cnt_v);
     }
+    if (L.have != L.done) L.template drain<KP>(L.have - L.done);
   }
 };
 
@@ -828,40 +854,51 @@ struct PtNarrow {
   }
 
   // the part's columns start xoff points into the x-tile; with CARRY the rows'
-  // counts before it are in s_cnt
+  // counts before it are in sh.cnt, and its own go to sh.cnt2
   template <uint32_t CAP, bool CARRY>
   __device__ static __forceinline__ void classify(const ClassifyArgs &a, uint32_t xt, uint32_t xoff, uint32_t k,
-                                                  uint32_t j0, const uint32_t *s_w, const uint32_t *s_tab,
-                                                  uint2 *s_cnt) {
+                                                  uint32_t j0, const uint32_t *s_w, PtShared &sh) {
     const FieldDesc &g = a.g;
     const uint32_t lane = lane_id(), wave = wave_id(), l = lane % LW, sub = lane / LW;
-    const uint32_t x0 = xt * CAP, xb = x0 + xoff + 4u * l, in_x = cells_in_grid(xb, g.cx);
+    const uint32_t in_x = cells_in_grid(xt * CAP + xoff + 4u * l, g.cx);
+    PtList<CAP, (uint32_t)LW, kPlaneWords, R, CARRY> L(a, s_w, sh, xt, xoff, k, j0);
     for (uint32_t m0 = wave * SR; m0 < (uint32_t)(KP * R); m0 += 4u * SR) {
       const uint32_t m = m0 + sub, cp = m / R, r = m - cp * R;
       const uint32_t y = j0 + r, z = k + cp;
-      const bool row_ok = m < (uint32_t)(KP * R), ok = row_ok && y < g.cy && z < g.cz;
-      const uint32_t widx = ok ? cp * kPlaneWords + (r + 1u) * LW + l : 0u;
-      const uint2 before = CARRY && ok ? s_cnt[m] : make_uint2(0u, 0u);
-      const PtChunk ch{widx, l, xb, x0, ok ? in_x : 0u, y, z, r, cp, xt + a.XT * (y + g.cy * z),
-                       (xoff >> 6) + (l >> 4), before.x & 0xFFFFu, before.y, before.x >> 16,
-                       y + 1 < g.cy, z + 1 < g.cz, false};
-      const uint32_t incl =
-          classify_chunk<LW, CAP, (uint32_t)LW, kPlaneWords, R, KP>(a, ch, ok ? s_w[widx] : 0u, s_w, s_tab);
-      if (l == LW - 1 && row_ok)
-        s_cnt[m] = make_uint2(before.x + ((incl & 0x1FFu) | ((incl >> 20) << 16)), before.y + ((incl >> 9) & 0x7FFu));
+      const bool ok = m < (uint32_t)(KP * R) && y < g.cy && z < g.cz;
+      const uint32_t act = ok ? active_cells(s_w[cp * kPlaneWords + (r + 1u) * LW + l]) & in_x : 0u;
+      if (__ballot(act != 0u) == 0ull) continue;
+      const uint32_t cnt = (uint32_t)__popc(act), seg = xt + a.XT * (y + g.cy * z);
+      // active cells of the row up to this lane, and of the rows in the lanes before
+      const uint32_t incl = LW == kWave ? wave_incl_scan_dpp(cnt) : row_incl_scan_dpp<LW>(cnt);
+      uint32_t first = 0u, total = 0u;
+#pragma unroll
+      for (int i = 0; i < SR; ++i) {
+        const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)incl, i * LW + LW - 1);
+        if (sub == (uint32_t)i) first = total;
+        total += t;
+      }
+      const uint32_t start = L.have + first;
+      if (l == 0u && ok)
+        sh.row[m] = make_uint2(seg, start | (y + 1u < g.cy ? 1u << 16 : 0u) | (z + 1u < g.cz ? 1u << 17 : 0u));
+      L.group_maps(seg, (xoff >> 6) + (l >> 4), act, (ok ? L.before(m).x & 0xFFFFu : 0u) + incl);
+      L.append(m, xoff + 4u * l, act, start + incl - cnt);
+      L.have += total;
+      while (L.have - L.done >= (uint32_t)kWave) L.template drain<KP>(kWave);
     }
+    if (L.have != L.done) L.template drain<KP>(L.have - L.done);
   }
 };
 
 // One plane tile with the parts TAIL names (pt_tail).
 template <uint32_t TAIL, uint32_t CAP, int R, int KP>
 __device__ __forceinline__ void classify_pt_parts(const ClassifyArgs &a, uint32_t xt, uint32_t k, uint32_t j0,
-                                                  uint32_t *s_w, uint32_t *s_tab, uint32_t tab_entry,
-                                                  bool store_tab) {
-  uint2 *s_cnt = reinterpret_cast<uint2 *>(s_tab + 512);
+                                                  uint32_t *s_w, PtShared &sh, uint32_t tab_entry, bool store_tab) {
+  static_assert(KP * R <= (int)kPtRowsMax, "row counts are staged in kPtRowsMax LDS entries");
   constexpr bool TINY = TAIL == kPtTailTiny;
   constexpr int C = TAIL == kPtTailFull ? (int)(CAP / 256u) : TINY ? 0 : (int)(TAIL >> 8);
   constexpr int LW = TAIL == kPtTailFull ? 0 : TINY ? 16 : (int)(TAIL & 0xFFu);
+  constexpr bool TWO = C != 0 && LW != 0;
   using W = PtWide<C ? C : 1, R, KP>;
   using N = PtNarrow<LW ? LW : 16, R, KP, TINY>;
   const bool tile_ok = (k < a.g.cz) && (j0 < a.g.cy);  // padding tiles do nothing
@@ -877,24 +914,27 @@ __device__ __forceinline__ void classify_pt_parts(const ClassifyArgs &a, uint32_
   }
   // the table entry was loaded before the field rows; storing it here keeps
   // its wait behind theirs
-  if (store_tab) pt_store_tables(s_tab, tab_entry);
+  if (store_tab) sh.tab[threadIdx.x] = tab_entry;
+  if (threadIdx.x < kPtRowsMax) {
+    sh.cnt[threadIdx.x] = make_uint2(0u, 0u);
+    if (TWO) sh.cnt2[threadIdx.x] = make_uint2(0u, 0u);
+  }
   __syncthreads();
   if (!tile_ok) return;  // uniform over the workgroup
-  if constexpr (C != 0) W::template classify<CAP>(a, xt, k, j0, s_w, s_tab, s_cnt);
+  if constexpr (C != 0) W::template classify<CAP>(a, xt, k, j0, s_w, sh);
   if constexpr (LW != 0) {
     if constexpr (C != 0) __syncthreads();  // the full chunks' counts
-    N::template classify<CAP, C != 0>(a, xt, 256u * C, k, j0, s_n, s_tab, s_cnt);
+    N::template classify<CAP, C != 0>(a, xt, 256u * C, k, j0, s_n, sh);
   }
-  store_row_counts<R, KP>(a, xt, j0, k, s_cnt);
+  store_row_counts<R, KP, TWO>(a, xt, j0, k, sh);
 }
 
 // Single volume: block b -> tile through the XCD mapping (pt_tile_of).
 // TAIL: the parts of the last x-tile.
 template <int W4, int R, int KP, uint32_t TAIL>
-__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >= 4 ? 4 : 8, W4 >= 4 ? 4 : 8))) void k_classify_pt(PtArgs pa) {
-  static_assert(KP * R <= kPtRowsMax, "row counts are staged in kPtRowsMax LDS entries");
+__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >= 4 || R > 7 ? 4 : 8, W4 >= 4 ? 4 : 8))) void k_classify_pt(PtArgs pa) {
   __shared__ uint32_t s_w[PtShape<W4, R, KP>::kLdsWords];
-  __shared__ __align__(16) uint32_t s_tab[kPtTabWords];
+  __shared__ PtShared sh;
   const ClassifyArgs &a = pa.c;
   const uint32_t tab = pt_table_entry();
   if (blockIdx.x == 0) {
@@ -904,9 +944,9 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
   const PtTile t = pt_tile_of(blockIdx.x, a.XT, pa.NRB, pa.NKB, pa.B);
   constexpr uint32_t CAP = 256u * W4;
   if (TAIL != kPtTailFull && t.xt + 1u == a.XT)
-    classify_pt_parts<TAIL, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, s_tab, tab, true);
+    classify_pt_parts<TAIL, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, sh, tab, true);
   else if (TAIL != kPtTailTiny)
-    classify_pt_parts<kPtTailFull, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, s_tab, tab, true);
+    classify_pt_parts<kPtTailFull, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, sh, tab, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -960,8 +1000,8 @@ __device__ __forceinline__ uint32_t volume_of(const uint32_t *off, uint32_t nvol
 template <int W4, int R, int KP>
 __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 == 1 ? 8 : (W4 == 2 ? 6 : 4), W4 == 1 ? 8 : (W4 == 2 ? 6 : 4)))) void k_classify_batch(BatchArgs b) {
   __shared__ uint32_t s_w[PtShape<W4, R, KP>::kLdsWords];
-  __shared__ __align__(16) uint32_t s_tab[kPtTabWords];
-  pt_init_table(s_tab);
+  __shared__ PtShared sh;
+  sh.tab[threadIdx.x] = pt_table_entry();
   if (blockIdx.x == 0) {
     zero_scan_state(b.zero, threadIdx.x, kPtThreads);
     if (threadIdx.x < 4) b.zero.counts_out[threadIdx.x] = 0u;  // the batch's scan counts
@@ -1003,15 +1043,15 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 =
     const uint32_t k = u / nrb * KP, j0 = u % nrb * R, tail = xt + 1u == a.XT ? bv->tail : kPtTailFull;
     constexpr uint32_t CAP = 256u * W4;
     if (W4 <= 2 && tail == kPtTail16)
-      classify_pt_parts<kPtTail16, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+      classify_pt_parts<kPtTail16, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
     else if (W4 <= 2 && tail == kPtTail32)
-      classify_pt_parts<kPtTail32, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+      classify_pt_parts<kPtTail32, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
     else if (W4 == 2 && tail == kPtTail64)
-      classify_pt_parts<kPtTail64, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+      classify_pt_parts<kPtTail64, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
     else if (tail == kPtTailTiny)
-      classify_pt_parts<kPtTailTiny, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+      classify_pt_parts<kPtTailTiny, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
     else
-      classify_pt_parts<kPtTailFull, CAP, R, KP>(a, xt, k, j0, s_w, s_tab, 0u, false);
+      classify_pt_parts<kPtTailFull, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
   }
 }
 
