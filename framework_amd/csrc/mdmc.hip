@@ -347,7 +347,7 @@ int capture_guard(mdmc_ctx *ctx, hipStream_t st) {
 }
 
 struct ScratchLayout {
-  size_t counts, vq, ne, chunk, state, ticket, totals, slots, gmap, coords, total;
+  size_t counts, vq, ne, chunk, state, ticket, totals, slots, slot_q, gmap, coords, total;
 };
 
 ScratchLayout scratch_layout(const Plan &p) {
@@ -366,7 +366,11 @@ ScratchLayout scratch_layout(const Plan &p) {
   L.state = take((size_t)p.ntiles * 4 * sizeof(unsigned long long));
   L.ticket = take(kTicketBytes);
   L.totals = take(sizeof(Totals));
-  L.slots = take(p.nslots * sizeof(uint64_t));
+  // records (4 bytes a slot, two words of slack for pair loads), then the first
+  // quads (2 bytes a slot); the region keeps 8 bytes a slot, so that what a
+  // given scratch size admits does not change
+  L.slots = take(p.nslots * 8);
+  L.slot_q = L.slots + p.nslots * sizeof(uint32_t) + 16;
   L.gmap = take(p.nsegs * (p.cap / 64) * sizeof(uint4));
   L.coords = take(p.ncoord * sizeof(float));
   L.total = off;
@@ -414,7 +418,8 @@ int ensure_scratch(mdmc_ctx *ctx, const Plan &p) {
   s.scan_state = reinterpret_cast<unsigned long long *>(b + o_state);
   s.ticket = reinterpret_cast<uint32_t *>(b + o_ticket);
   s.totals = reinterpret_cast<Totals *>(b + o_totals);
-  s.slots = reinterpret_cast<uint64_t *>(b + o_slots);
+  s.slots = reinterpret_cast<uint32_t *>(b + o_slots);
+  s.slot_q = reinterpret_cast<uint16_t *>(b + lay.slot_q);
   s.gmap = reinterpret_cast<uint4 *>(b + o_gmap);
   s.coords = reinterpret_cast<float *>(b + o_coords);
   ctx->s = s;
@@ -465,6 +470,7 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   ca.Kc = p.Kc;
   ca.seg_counts = s.seg_counts;
   ca.slots = s.slots;
+  ca.slot_q = s.slot_q;
   ca.gmap = s.gmap;
   ca.scan_state = s.scan_state;
   ca.scan_state_words = p.ntiles * 4;
@@ -530,12 +536,16 @@ int launch_emit(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   ea.v.yt_c = s.coords + p.X;
   ea.v.zt_c = s.coords + p.X + p.Y;
   ea.v.XT = p.XT;
+  ea.v.div_xt = fast_div(p.XT);
+  ea.v.div_cy = fast_div(p.cy);
+  ea.v.span = emit_span(p.X, p.XT, p.cap);
   ea.cap = p.cap;
   ea.nsegs = (uint32_t)p.nsegs;
   ea.max_chunks = p.max_chunks;
   ea.seg_counts = s.seg_counts;
   ea.seg_vq = s.seg_vq;
   ea.slots = s.slots;
+  ea.slot_q = s.slot_q;
   ea.gmap = s.gmap;
   ea.ne = s.ne;
   ea.chunk_ne = s.chunk_ne;
@@ -737,6 +747,7 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     b.c.XT = XT;
     b.c.seg_counts = S.seg_counts + seg_off;
     b.c.slots = S.slots + seg_off * cap;
+    b.c.slot_q = S.slot_q + seg_off * cap;
     b.c.gmap = S.gmap + seg_off * (cap / 64);
     b.tile_off = tiles0[v] = (uint32_t)tile_off;
     b.NRB = NRB;
@@ -751,13 +762,26 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     b.rgx = mv.xyz_max[0] - mv.xyz_min[0];
     b.rgy = mv.xyz_max[1] - mv.xyz_min[1];
     b.rgz = mv.xyz_max[2] - mv.xyz_min[2];
-    b.verts = mv.vertices;
-    b.vcap = mv.vertices ? mv.vertex_capacity : 0;
-    b.quads = mv.quads;
-    b.qcap = mv.quads ? mv.quad_capacity : 0;
     b.counts = reinterpret_cast<uint32_t *>(d_counts + v);
     b.coords = empty ? nullptr : S.coords + coord_off;
-    if (!empty) coord_off += (uint64_t)X + Y + Z;
+    if (!empty) {
+      coord_off += (uint64_t)X + Y + Z;
+      b.e.g = b.c.g;
+      b.e.div_xt = fast_div(XT);
+      b.e.div_cy = fast_div(cy);
+      b.e.span = emit_span(X, XT, cap);
+      b.e.xt_c = b.coords;
+      b.e.yt_c = b.coords + X;
+      b.e.zt_c = b.coords + X + Y;
+      b.e.XT = XT;
+      b.e.seg_off = b.seg_off;
+      b.e.verts = mv.vertices;
+      b.e.vcap = mv.vertices ? mv.vertex_capacity : 0;
+      b.e.quads = mv.quads;
+      b.e.qcap = mv.quads ? mv.quad_capacity : 0;
+      b.e.status = b.counts + 3;
+      b.e.kmax = 0xFFFFFFFFu;
+    }
     seg_off += nsegs;
     tile_off += (uint64_t)XT * NRB * NKP;
     cells += (uint64_t)cx * cy * cz;
@@ -948,6 +972,7 @@ int batch_emit(mdmc_ctx *ctx, const mdmc_volume *vols, uint32_t n, mdmc_counts *
   be.a.seg_counts = S.seg_counts;
   be.a.seg_vq = S.seg_vq;
   be.a.slots = S.slots;
+  be.a.slot_q = S.slot_q;
   be.a.gmap = S.gmap;
   be.a.ne = S.ne;
   be.a.chunk_ne = S.chunk_ne;
@@ -1763,6 +1788,9 @@ int mdmc_run_out_of_core(const float *field, const uint32_t dims[3], const float
     ea.v.yt_c = sc.coords + p.X;
     ea.v.zt_c = sc.coords + p.X + p.Y;
     ea.v.XT = p.XT;
+    ea.v.div_xt = fast_div(p.XT);
+    ea.v.div_cy = fast_div(p.cy);
+    ea.v.span = emit_span(p.X, p.XT, p.cap);
     ea.v.vbase = b_lo.x;
     ea.v.qbase = b_lo.y;
     ea.v.kmin = h;
@@ -1774,6 +1802,7 @@ int mdmc_run_out_of_core(const float *field, const uint32_t dims[3], const float
     ea.seg_counts = sc.seg_counts;
     ea.seg_vq = sc.seg_vq;
     ea.slots = sc.slots;
+    ea.slot_q = sc.slot_q;
     ea.gmap = sc.gmap;
     ea.ne = sc.ne;
     ea.chunk_ne = sc.chunk_ne;

@@ -32,7 +32,8 @@ struct Scratch {
   unsigned long long *scan_state;
   uint32_t *ticket;
   Totals *totals;
-  uint64_t *slots;
+  uint32_t *slots;
+  uint16_t *slot_q;
   uint4 *gmap;
   float *coords;
 };

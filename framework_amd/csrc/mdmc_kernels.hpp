@@ -7,7 +7,7 @@
 //               rows staged in LDS as sign bits, uniform 256-cell chunks
 //               skipped with one ballot, active cells found by bit operations
 //               and listed in LDS; listed cells get their 2B/3B table variant,
-//               vertex and quad counts, a DPP-scan rank and a 64-bit record in
+//               vertex and quad counts, a DPP-scan rank and a 32-bit record in
 //               their segment's slot range (segment = one cell row of one
 //               x-tile in one plane), plus a per-64-cell group map (active
 //               mask, first rank).  Workgroups map to tiles XCD by XCD (mdmc_tilemap.h).
@@ -30,6 +30,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "mdmc_tilemap.h"
@@ -64,21 +65,20 @@ struct FieldDesc {
   float iso;
 };
 
-// Record of an active cell (64 bits):
+// Record of an active cell (32 bits):
 //   bits  0-9   x offset inside its x-tile
 //   bits 10-17  configuration
 //   bit  18     uses the variant-1 table (2B/3B correction)
 //   bits 19-31  first vertex, relative to the segment
-//   bits 32-43  first quad, relative to the segment
-__device__ __forceinline__ uint64_t make_record(uint32_t xl, uint32_t cfg, uint32_t lut2,
-                                                uint32_t lvb, uint32_t lqb) {
-  return (uint64_t)(xl | (cfg << 10) | (lut2 << 18) | (lvb << 19)) | ((uint64_t)lqb << 32);
+// Its first quad, relative to the segment, is kept apart (16 bits): only the
+// cell's own emit reads it, while a record is read by up to seven cells.
+__device__ __forceinline__ uint32_t make_record(uint32_t xl, uint32_t cfg, uint32_t lut2, uint32_t lvb) {
+  return xl | (cfg << 10) | (lut2 << 18) | (lvb << 19);
 }
-__device__ __forceinline__ uint32_t rec_x(uint64_t r) { return (uint32_t)r & 0x3FFu; }
-__device__ __forceinline__ uint32_t rec_cfg(uint64_t r) { return ((uint32_t)r >> 10) & 0xFFu; }
-__device__ __forceinline__ uint32_t rec_lut2(uint64_t r) { return ((uint32_t)r >> 18) & 1u; }
-__device__ __forceinline__ uint32_t rec_lvb(uint64_t r) { return ((uint32_t)r >> 19) & 0x1FFFu; }
-__device__ __forceinline__ uint32_t rec_lqb(uint64_t r) { return (uint32_t)(r >> 32) & 0xFFFu; }
+__device__ __forceinline__ uint32_t rec_x(uint32_t r) { return r & 0x3FFu; }
+__device__ __forceinline__ uint32_t rec_cfg(uint32_t r) { return (r >> 10) & 0xFFu; }
+__device__ __forceinline__ uint32_t rec_lut2(uint32_t r) { return (r >> 18) & 1u; }
+__device__ __forceinline__ uint32_t rec_lvb(uint32_t r) { return r >> 19; }
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
@@ -200,7 +200,8 @@ struct ClassifyArgs {
   FieldDesc g;
   uint32_t XT, NRB, NKC, Kc;
   uint2 *seg_counts;      // per segment: {nact | nquad << 16, nvert}
-  uint64_t *slots;        // per segment: 64*W record slots
+  uint32_t *slots;        // per segment: 64*W record slots
+  uint16_t *slot_q;       // per record slot: the cell's first quad
   uint4 *gmap;            // per segment and 64-cell group: {active mask lo, hi, rank of
                           // the group's first active cell, 0}; written for non-empty groups
   unsigned long long *scan_state;  // zeroed here for k_scan
@@ -349,7 +350,8 @@ __global__ __launch_bounds__(64) void k_classify(ClassifyArgs a) {
           const uint32_t rank = cnt_a + mbcnt64(bal);
           const uint32_t lvb = cnt_v + (excl & 0xFFFFu);
           const uint32_t lqb = cnt_q + (excl >> 16);
-          a.slots[(size_t)seg * CAP + rank] = make_record(x - x0, cfg, lut2, lvb, lqb);
+          a.slots[(size_t)seg * CAP + rank] = make_record(x - x0, cfg, lut2, lvb);
+          a.slot_q[(size_t)seg * CAP + rank] = (uint16_t)lqb;
         }
         cnt_a += (uint32_t)__popcll(bal);
         cnt_v += tot & 0xFFFFu;
@@ -623,9 +625,11 @@ struct PtList {
     const uint32_t at_start = (uint32_t)__shfl((int)excl, (int)((lane - rank) & 63u), kWave);
     const uint32_t st = rank <= lane ? at_start : row_run;
     const uint32_t loc = excl - st;
-    if (valid)
-      a.slots[(size_t)row.x * CAP + (bef.x & 0xFFFFu) + rank] =
-          make_record(xl, (ent >> 16) & 0xFFu, l2, bef.y + (loc & 0xFFFFu), (bef.x >> 16) + (loc >> 16));
+    if (valid) {
+      const size_t at = (size_t)row.x * CAP + (bef.x & 0xFFFFu) + rank;
+      a.slots[at] = make_record(xl, (ent >> 16) & 0xFFu, l2, bef.y + (loc & 0xFFFFu));
+      a.slot_q[at] = (uint16_t)((bef.x >> 16) + (loc >> 16));
+    }
     // the row's counts so far (its last entry writes the final ones)
     const uint32_t next = lane_next(m);
     if (valid && (lane + 1u == n || next != m)) {
@@ -957,19 +961,60 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
 
 constexpr uint32_t kMaxBatch = 1024;  // volumes per batch call
 
+// Exact division of 32-bit numbers by a divisor known on the host: a multiply
+// and two shifts (round-up multiplier 2^32 (2^l - d) / d + 1, l = ceil(log2 d);
+// Granlund and Montgomery, "Division by invariant integers using
+// multiplication").
+struct FastDiv {
+  uint32_t mul, sh1, sh2;
+};
+__host__ inline FastDiv fast_div(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32u && (1ull << l) < d) ++l;
+  return FastDiv{(uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1u), l < 1u ? l : 1u, l > 1u ? l - 1u : 0u};
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, FastDiv d) {
+  const uint32_t t = __umulhi(d.mul, n);
+  return (t + ((n - t) >> d.sh1)) >> d.sh2;
+}
+
+// Segments from a wave's first one on whose records, group maps and field rows
+// lie within 2 GB of that segment's (32-bit lane offsets from its bases): a
+// record is 4 bytes, and a segment lies at most 2 * (distance / XT + 1) point
+// rows further on.
+__host__ inline uint32_t emit_span(uint32_t X, uint32_t XT, uint32_t cap) {
+  const uint64_t rec = (1ull << 31) / (4ull * cap) - 1u, rows = (1ull << 31) / (4ull * X);
+  const uint64_t fld = rows > 6u ? (uint64_t)XT * ((rows - 4u) / 2u) : 0u;
+  return (uint32_t)(rec < fld ? rec : fld);
+}
+
+// Per-volume part of the emit arguments.
+struct EmitVol {
+  FieldDesc g;
+  FastDiv div_xt, div_cy;              // division by XT and by cy
+  uint32_t span;                       // emit_span: segments that share 32-bit offsets
+  const float *xt_c, *yt_c, *zt_c;     // coordinate of every point index per axis
+  uint32_t XT, seg_off;                // x-tiles; first segment of the volume
+  uint32_t vbase, qbase;               // global vertex / quad number of its first
+  float *verts;
+  uint64_t vcap;
+  int32_t *quads;
+  uint64_t qcap;
+  uint32_t *status;
+  // emit only cell planes [kmin, kmax); quad entries are vertex numbers plus
+  // vshift (a slab of a larger grid, numbered globally)
+  uint32_t kmin = 0, kmax = 0xFFFFFFFFu, vshift = 0;
+};
+
 struct BatchVol {
   ClassifyArgs c;         // per-volume field and tiling; record pointers start at seg_off
+  EmitVol e;              // for the emit, except vbase and qbase (BatchEmitArgs.base)
   uint32_t NRB, NKP;      // row blocks and plane blocks of the volume
   uint32_t tail;          // parts of the last x-tile (pt_tail)
   uint32_t tile_off;      // first flattened classify tile
   uint32_t seg_off, nsegs;
   float mnx, mny, mnz, rgx, rgy, rgz;
-  float *verts;
-  uint64_t vcap;
-  int32_t *quads;
-  uint64_t qcap;
   uint32_t *counts;       // the volume's mdmc_counts
-  uint32_t vbase, qbase;  // written by k_batch_counts: prefix at seg_off
   float *coords;          // X + Y + Z point coordinates (filled before the emit)
 };
 
@@ -1035,6 +1080,7 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 =
     a.XT = bv->c.XT;
     a.seg_counts = bv->c.seg_counts;
     a.slots = bv->c.slots;
+    a.slot_q = bv->c.slot_q;
     a.gmap = bv->c.gmap;
     const uint32_t nrb = bv->NRB;
     const uint32_t local = t - bv->tile_off;
@@ -1296,29 +1342,14 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(ScanArgs a) {
 
 constexpr int kEmitThreads = 256;
 
-// Per-volume part of the emit arguments.
-struct EmitVol {
-  FieldDesc g;
-  const float *xt_c, *yt_c, *zt_c;     // coordinate of every point index per axis
-  uint32_t XT, seg_off;                // x-tiles; first segment of the volume
-  uint32_t vbase, qbase;               // global vertex / quad number of its first
-  float *verts;
-  uint64_t vcap;
-  int32_t *quads;
-  uint64_t qcap;
-  uint32_t *status;
-  // emit only cell planes [kmin, kmax); quad entries are vertex numbers plus
-  // vshift (a slab of a larger grid, numbered globally)
-  uint32_t kmin = 0, kmax = 0xFFFFFFFFu, vshift = 0;
-};
-
 struct EmitArgs {
   EmitVol v;  // the volume (single-volume launches)
   uint32_t cap, nsegs;
   uint64_t max_chunks;  // capacity of chunk_ne
   const uint2 *seg_counts;
   const uint2 *seg_vq;
-  const uint64_t *slots;
+  const uint32_t *slots;
+  const uint16_t *slot_q;
   const uint4 *gmap;
   const uint2 *ne;
   const uint32_t *chunk_ne;
@@ -1342,66 +1373,112 @@ __device__ __forceinline__ uint32_t const_u2x(const uint2 *p, uint32_t i) {
   return ((const __attribute__((address_space(4))) uint32_t *)p)[2 * i];
 }
 
-// One active cell (segment s, rank within it) of volume vol: its vertices and
-// the quads of its owned edges.
-__device__ __forceinline__ void emit_cell(const EmitArgs &a, const EmitVol &vol, uint32_t s, uint32_t rank,
-                                          const uint64_t *s_lab, float *s_acc) {
+// Kernel arguments and volume descriptors seen through the constant address
+// space; fresh() makes the compiler read the fields used after it again (into
+// scalar registers) instead of keeping them from before.
+typedef const __attribute__((address_space(4))) EmitArgs *EmitArgsK;
+typedef const __attribute__((address_space(4))) EmitVol *EmitVolK;
+__device__ __forceinline__ const EmitArgs &fresh(EmitArgsK p) {
+  asm volatile("" : "+s"(p));
+  return *(const EmitArgs *)p;
+}
+__device__ __forceinline__ const EmitVol &fresh(EmitVolK p) {
+  asm volatile("" : "+s"(p));
+  return *(const EmitVol *)p;
+}
+
+// Address `off` bytes after a wave-uniform base.
+template <class T>
+__device__ __forceinline__ const T *at_off(const void *base, uint32_t off) {
+  return reinterpret_cast<const T *>(static_cast<const char *>(base) + off);
+}
+template <class T>
+__device__ __forceinline__ T *at_off(void *base, uint32_t off) {
+  return reinterpret_cast<T *>(static_cast<char *>(base) + off);
+}
+
+// Two consecutive words or floats, and a vertex, at the alignment of one word.
+typedef uint32_t Word2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float Float2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float Float3 __attribute__((ext_vector_type(3), aligned(4)));
+
+// The active cells of the calling lanes (segment s, rank within it) of volume
+// vol: their vertices and the quads of their owned edges.  s0: the segment of
+// the first of these lanes (uniform); all lanes' segments lie in [s0, s0 +
+// vol.span], so everything a lane addresses is a uniform base, taken for s0,
+// plus a 32-bit lane offset.  base: the volume's first vertex and quad.  (64-bit address arithmetic per lane and load, and
+// the division of a segment number into tile, row and plane on every lane,
+// were a quarter of the kernel's issue slots.)  s_lab: kEmitLab entries.
+__device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base, uint32_t s0, uint32_t s,
+                                           uint32_t rank, const uint64_t *s_lab, float *s_acc) {
+  const EmitArgs &a = fresh(pa);
+  const EmitVol &vol = fresh(pv);
   const FieldDesc &g = vol.g;
   const float iso = g.iso;
-  const size_t sy = g.X, sz = (size_t)g.X * g.Y;
   const uint32_t cap = a.cap;
-  const uint64_t rec = a.slots[(size_t)s * cap + rank];
-  const uint32_t xl = rec_x(rec), cfg = rec_cfg(rec), lut2 = rec_lut2(rec);
-  const uint32_t sl = s - vol.seg_off;
-  const uint32_t xt = sl % vol.XT, row = sl / vol.XT;
-  const uint32_t j = row % g.cy, k = row / g.cy;
-  const uint32_t x = xt * cap + xl;
-  if (x >= g.cx || xl >= cap) { atomicOr(vol.status, kStatusInternal); return; }
-  if (k < vol.kmin || k >= vol.kmax) return;
-  // The lanes of a chunk nearly always share one segment.  What depends only
-  // on the segment (its bases and count, the row's y and z coordinates, the
-  // ring segments' vertex bases below) comes through scalar loads for the
-  // lanes in the wave's first segment and through vector loads for the rest
-  // (these arrays are read-only in the emit).
-  const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
-  // s0u: s0 in a scalar register that the compiler cannot equate with s, so
-  // that on the lanes where s == s0 it does not turn the loads below back
-  // into per-lane vector loads at s
+  const size_t sy = g.X, sz = (size_t)g.X * g.Y;
+  const uint32_t d = s - s0;
+  // this cell's record and the next active one's of its segment
+  const uint32_t *const rec0 = a.slots + (size_t)s0 * cap;
+  const uint32_t roff = d * cap + rank;
+  const Word2 own = *at_off<Word2>(rec0, roff * 4u);
+  const uint32_t lqb = *at_off<uint16_t>(a.slot_q + (size_t)s0 * cap, roff * 2u);
+  // What depends only on the segment (its bases and count, the row's y and z
+  // coordinates) comes through scalar loads for the lanes in s0 and through
+  // vector loads for the rest (these arrays are read-only in the emit).  s0u:
+  // s0 in a scalar register that the compiler cannot equate with s, so that on
+  // the lanes where s == s0 it does not turn the scalar loads back into
+  // per-lane vector loads at s.
   uint32_t s0u = s0;
   asm volatile("" : "+s"(s0u));
-  const uint32_t row0 = (s0u - vol.seg_off) / vol.XT;
-  const uint32_t j0 = row0 % g.cy, k0 = row0 / g.cy;
-  // (scalar loads first, outside any branch on the lane's segment)
+  const uint32_t sl0 = s0u - vol.seg_off;
+  const uint32_t row0 = div_by(sl0, vol.div_xt), xt0 = sl0 - row0 * vol.XT;
+  const uint32_t k0 = div_by(row0, vol.div_cy), j0 = row0 - k0 * g.cy;
   uint2 vq = const_u2(a.seg_vq, s0u);
   uint32_t nact = const_u2x(a.seg_counts, s0u) & 0xFFFFu;
   float Y0 = as_const(vol.yt_c)[j0], Y1 = as_const(vol.yt_c)[j0 + 1];
   float Z0 = as_const(vol.zt_c)[k0], Z1 = as_const(vol.zt_c)[k0 + 1];
-  const bool lead = s == s0;
-  if (!lead) {
-    vq = a.seg_vq[s];
-    nact = a.seg_counts[s].x & 0xFFFFu;
-    Y0 = vol.yt_c[j];
-    Y1 = vol.yt_c[j + 1];
-    Z0 = vol.zt_c[k];
-    Z1 = vol.zt_c[k + 1];
+  uint32_t xt = xt0, j = j0, k = k0, prow = 0;  // prow: point rows after (j0, k0)
+  if (d != 0u) {
+    const uint32_t sl = s - vol.seg_off, row = div_by(sl, vol.div_xt);
+    xt = sl - row * vol.XT;
+    k = div_by(row, vol.div_cy);
+    j = row - k * g.cy;
+    prow = (k - k0) * g.Y + j - j0;
+    vq = *at_off<uint2>(a.seg_vq + s0, d * 8u);
+    nact = at_off<uint2>(a.seg_counts + s0, d * 8u)->x & 0xFFFFu;
+    const Float2 yy = *at_off<Float2>(vol.yt_c, j * 4u), zz = *at_off<Float2>(vol.zt_c, k * 4u);
+    Y0 = yy.x;
+    Y1 = yy.y;
+    Z0 = zz.x;
+    Z1 = zz.y;
   }
-  const uint32_t vb = vq.x + rec_lvb(rec) - vol.vbase;  // volume-local numbers
-  const uint32_t qb = vq.y + rec_lqb(rec) - vol.qbase;
-
-  const float *p = g.f + (size_t)k * sz + (size_t)j * sy + x;
-  float v[8];
-  v[0] = p[0];
-  v[1] = p[1];
-  v[2] = p[sy + 1];
-  v[3] = p[sy];
-  v[4] = p[sz];
-  v[5] = p[sz + 1];
-  v[6] = p[sz + sy + 1];
-  v[7] = p[sz + sy];
-
-  const float X0 = vol.xt_c[x], X1 = vol.xt_c[x + 1];
+  const uint32_t rec = own.x;
+  const uint32_t xl = rec_x(rec), cfg = rec_cfg(rec);
+  const uint32_t x = xt * cap + xl;
   // a rank past the segment's count means inconsistent count-pass data
-  if (rank >= nact) { atomicOr(vol.status, kStatusInternal); return; }
+  if (x >= g.cx || xl >= cap || rank >= nact) { atomicOr(vol.status, kStatusInternal); return; }
+  if (k < vol.kmin || k >= vol.kmax) return;
+
+  // the cell's four point pairs along x
+  const float *const p = g.f + (size_t)k0 * sz + (size_t)j0 * sy + (size_t)xt0 * cap;
+  const uint32_t poff = (prow * g.X + x - xt0 * cap) * 4u;
+  const Float2 v01 = *at_off<Float2>(p, poff), v32 = *at_off<Float2>(p + sy, poff);
+  const Float2 v45 = *at_off<Float2>(p + sz, poff), v76 = *at_off<Float2>(p + sz + sy, poff);
+  const Float2 xx = *at_off<Float2>(vol.xt_c, x * 4u);
+  const float v[8] = {v01.x, v01.y, v32.y, v32.x, v45.x, v45.y, v76.y, v76.x};
+  const float X0 = xx.x, X1 = xx.y;
+
+  // first vertex and quad (numbers of the volume), and as offsets from those of
+  // the first lane: a chunk's cells are consecutive, so the offsets are small
+  const uint32_t vb = vq.x + rec_lvb(rec) - base.x, qb = vq.y + lqb - base.y;
+  const uint32_t vb0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)vb);
+  const uint32_t qb0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)qb);
+  uint32_t dvq = (vb - vb0) | ((qb - qb0) << 16);
+  if (vb - vb0 >= 1024u || qb - qb0 >= 1024u) { atomicOr(vol.status, kStatusInternal); return; }
+  // what the quads need of the position, kept as lane masks over the vertices
+  const bool xin = x + 1 < g.cx, yin = j + 1 < g.cy, zin = k + 1 < g.cz, n0in = rank + 1u < nact;
+  asm volatile("" : "+v"(dvq));  // (one register, not its two halves)
 
   // Edge e runs from corner EF[e] to corner ET[e]: the orientation its
   // owning cell uses (owner edge 6: p2->p6, 9: p5->p6, 10: p6->p7), so the
@@ -1409,14 +1486,15 @@ __device__ __forceinline__ void emit_cell(const EmitArgs &a, const EmitVol &vol,
   constexpr uint8_t EF[12] = {1, 1, 2, 0, 0, 1, 2, 3, 5, 5, 6, 4};
   constexpr uint8_t ET[12] = {0, 2, 3, 3, 4, 5, 6, 7, 4, 6, 7, 7};
   // Owner of each edge lies at a non-positive offset; an edge is skipped
-  // when its owner would be outside the grid (dmc.cu:1539-1545).
-  // bit 0: needs x>0, bit 1: needs y>0, bit 2: needs z>0
-  constexpr uint8_t NEED[12] = {6, 4, 4, 5, 3, 2, 0, 1, 2, 0, 0, 1};
-  const uint32_t have = (x > 0 ? 1u : 0u) | (j > 0 ? 2u : 0u) | (k > 0 ? 4u : 0u);
-
-  const uint64_t labels = s_lab[lut2 * 256 + cfg];
-  const uint16_t info = c_cfg_info[cfg];
-  const uint32_t niso = lut2 ? ((info >> 3) & 7u) : (info & 7u);
+  // when its owner would be outside the grid (dmc.cu:1539-1545): edges that
+  // need a cell at -x (0x898), -y (0x131), -z (0x00F)
+  const uint64_t labels = s_lab[(rec >> 10) & 0x1FFu];
+  const uint32_t lab_hi = (uint32_t)(labels >> 32);
+  const uint32_t niso = (lab_hi >> 16) & 0xFu;
+  uint32_t use = lab_hi >> 20;  // crossed edges whose owner is in the grid
+  if (x == 0u) use &= ~0x898u;
+  if (j == 0u) use &= ~0x131u;
+  if (k == 0u) use &= ~0x00Fu;
   // Group sums live in LDS, component c of group q at s_acc[(3q + c) * T]
   // (T = threads per block; the caller offsets s_acc by the thread index).
   // They start at -0.0, so the first addition yields the point itself
@@ -1434,8 +1512,9 @@ __device__ __forceinline__ void emit_cell(const EmitArgs &a, const EmitVol &vol,
   float ex[3] = {0, 0, 0}, ey[3] = {0, 0, 0}, ez[3] = {0, 0, 0};
 #pragma unroll
   for (int e = 0; e < 12; ++e) {
-    const uint32_t lab = (uint32_t)(labels >> (4 * e)) & 0xFu;
-    if (lab == 0xFu) continue;
+    // (edges 6, 9, 10 are the cell's own: used whenever crossed)
+    if (!((use >> e) & 1u)) continue;
+    const uint32_t lab = (e < 8 ? (uint32_t)labels >> (4 * e) : lab_hi >> (4 * e - 32)) & 0xFu;
     const int f = EF[e], to = ET[e];
     const float vf = v[f], vt = v[to];
     const float tt = (iso - vf) / (vt - vf);
@@ -1452,130 +1531,157 @@ __device__ __forceinline__ void emit_cell(const EmitArgs &a, const EmitVol &vol,
     if (e == 6) { ex[0] = px; ey[0] = py; ez[0] = pz; }
     if (e == 9) { ex[1] = px; ey[1] = py; ez[1] = pz; }
     if (e == 10) { ex[2] = px; ey[2] = py; ez[2] = pz; }
-    if ((NEED[e] & have) != NEED[e]) continue;
     float *acc = s_acc + 3 * lab * T;
     acc[0] = acc[0] + px;
     acc[T] = acc[T] + py;
     acc[2 * T] = acc[2 * T] + pz;
     cnt += 1u << (8 * lab);
   }
-  const uint32_t b6 = ((cfg >> 2) ^ (cfg >> 6)) & 1u;
-  const uint32_t b9 = ((cfg >> 5) ^ (cfg >> 6)) & 1u;
-  const uint32_t b10 = ((cfg >> 7) ^ (cfg >> 6)) & 1u;
+  const uint32_t b6 = (use >> 6) & 1u, b9 = (use >> 9) & 1u, b10 = (use >> 10) & 1u;
   const uint32_t nv = niso + b6 + b9 + b10;
-  if ((uint64_t)vb + nv <= vol.vcap) {
-    float *out = vol.verts + 3ull * vb;
+  if ((uint64_t)vb0 + (dvq & 0xFFFFu) + nv <= vol.vcap) {
+    float *const out = vol.verts + 3ull * vb0;
+    uint32_t o = (dvq & 0xFFFFu) * 12u;
     const float qnan = __int_as_float(0x7FC00000);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if ((uint32_t)q < niso) {
         const uint32_t n = (cnt >> (8 * q)) & 0xFFu;
-        const float d = (float)n;
-        out[3 * q + 0] = n ? s_acc[(3 * q + 0) * T] / d : qnan;
-        out[3 * q + 1] = n ? s_acc[(3 * q + 1) * T] / d : qnan;
-        out[3 * q + 2] = n ? s_acc[(3 * q + 2) * T] / d : qnan;
+        const float dn = (float)n;
+        Float3 r;
+        r.x = n ? s_acc[(3 * q + 0) * T] / dn : qnan;
+        r.y = n ? s_acc[(3 * q + 1) * T] / dn : qnan;
+        r.z = n ? s_acc[(3 * q + 2) * T] / dn : qnan;
+        *at_off<Float3>(out, o + 12u * q) = r;
       }
     }
-    uint32_t wv = niso;
-    if (b6) { out[3 * wv] = ex[0]; out[3 * wv + 1] = ey[0]; out[3 * wv + 2] = ez[0]; ++wv; }
-    if (b9) { out[3 * wv] = ex[1]; out[3 * wv + 1] = ey[1]; out[3 * wv + 2] = ez[1]; ++wv; }
-    if (b10) { out[3 * wv] = ex[2]; out[3 * wv + 1] = ey[2]; out[3 * wv + 2] = ez[2]; ++wv; }
+    o += niso * 12u;
+    if (b6) { *at_off<Float3>(out, o) = Float3{ex[0], ey[0], ez[0]}; o += 12u; }
+    if (b9) { *at_off<Float3>(out, o) = Float3{ex[1], ey[1], ez[1]}; o += 12u; }
+    if (b10) *at_off<Float3>(out, o) = Float3{ex[2], ey[2], ez[2]};
   } else {
     atomicOr(vol.status, kStatusVertexOverflow);
   }
 
   // Quads (dmc.cu:1983-2047): rings in ccw order, reversed (0,3,2,1) when
-  // the owned edge's first corner is not above iso.
-  const bool xin = x + 1 < g.cx, yin = j + 1 < g.cy, zin = k + 1 < g.cz;
+  // the owned edge's first corner is not above iso.  The arguments are read
+  // again (scalar loads that hit the cache) instead of staying in registers
+  // over the vertices.
+  const EmitArgs &aq = fresh(pa);
+  const EmitVol &vq_ = fresh(pv);
   const bool e6 = b6 && xin && yin, e9 = b9 && xin && zin, e10 = b10 && yin && zin;
   if (!(e6 || e9 || e10)) return;
-  const uint32_t nq = (uint32_t)e6 + (uint32_t)e9 + (uint32_t)e10;
-  if ((uint64_t)qb + nq > vol.qcap) { atomicOr(vol.status, kStatusQuadOverflow); return; }
+  const uint32_t nq = (uint32_t)e6 + (uint32_t)e9 + (uint32_t)e10, dq = dvq >> 16;
+  if ((uint64_t)qb0 + dq + nq > vq_.qcap) { atomicOr(vq_.status, kStatusQuadOverflow); return; }
   // Ring cells n = 0 (+1,0,0), 1 (0,+1,0), 2 (0,0,+1), 3 (+1,+1,0),
   // 4 (+1,0,+1), 5 (0,+1,+1).  A ring cell contains the crossing edge, so it
   // is active.  Cells 1, 2 and 5 are found through their segments' group
   // maps.  Cells 0, 3 and 4 follow from this cell, 1 and 2: a ring cell and
   // its -x neighbour in the ring are both active, so the +x one is the next
-  // active cell of its row (the first of the next x-tile's segment when x is
-  // the tile's last cell).  Each record's x field confirms the cell found.
-  // A lookup the quads do not need reads this cell's segment instead, so that
-  // every load is in bounds.
-  const uint32_t need = (e6 ? 0x0Bu : 0u) | (e9 ? 0x15u : 0u) | (e10 ? 0x26u : 0u);
-  const bool wrap = xl + 1u == cap;  // +x lies in the next x-tile's segment
-  const uint32_t xl1 = wrap ? 0u : xl + 1u;
-  const uint32_t dy = vol.XT, dz = vol.XT * g.cy;
-  const uint32_t s1 = (need & 0x0Au) ? s + dy : s, s2 = (need & 0x14u) ? s + dz : s;
-  const uint32_t s5 = (need & 0x20u) ? s + dy + dz : s;
-  const uint32_t G = cap >> 6;
-  const uint4 g1 = a.gmap[(size_t)s1 * G + (xl >> 6)], g2 = a.gmap[(size_t)s2 * G + (xl >> 6)];
-  const uint4 g5 = a.gmap[(size_t)s5 * G + (xl >> 6)];
-  // the first segment's ring segments (clamped: a lane that needs one has it
-  // in the grid), scalar loads first as above
-  const uint32_t last = a.nsegs - 1u;
-  uint32_t vq0[6];
-  vq0[1] = const_u2x(a.seg_vq, min(s0u + dy, last));
-  vq0[2] = const_u2x(a.seg_vq, min(s0u + dz, last));
-  vq0[5] = const_u2x(a.seg_vq, min(s0u + dy + dz, last));
-  if (!lead) {
-    vq0[1] = a.seg_vq[s1].x;
-    vq0[2] = a.seg_vq[s2].x;
-    vq0[5] = a.seg_vq[s5].x;
+  // active cell of its row, read with it (the first of the next x-tile's
+  // segment when x is the tile's last cell).  Each record's x field confirms
+  // the cell found.  A lookup the quads do not need reads at offset 0 of a
+  // segment in range, so that every load is in bounds.
+  const bool need1 = e6 || e10, need2 = e9 || e10, need5 = e10;
+  const uint32_t capq = aq.cap, G = capq >> 6, dy = vq_.XT, dz = vq_.XT * vq_.g.cy, last = aq.nsegs - 1u;
+  const uint32_t b1 = min(s0u + dy, last), b2 = min(s0u + dz, last), b5 = min(s0u + dy + dz, last);
+  const uint32_t goff = (d * G + (xl >> 6)) * 16u;
+  const uint4 g1 = *at_off<uint4>(aq.gmap + (size_t)b1 * G, need1 ? goff : 0u);
+  const uint4 g2 = *at_off<uint4>(aq.gmap + (size_t)b2 * G, need2 ? goff : 0u);
+  const uint4 g5 = *at_off<uint4>(aq.gmap + (size_t)b5 * G, need5 ? goff : 0u);
+  uint32_t vq1 = const_u2x(aq.seg_vq, b1), vq2 = const_u2x(aq.seg_vq, b2), vq5 = const_u2x(aq.seg_vq, b5);
+  if (d != 0u) {
+    vq1 = at_off<uint2>(aq.seg_vq + b1, need1 ? d * 8u : 0u)->x;
+    vq2 = at_off<uint2>(aq.seg_vq + b2, need2 ? d * 8u : 0u)->x;
+    vq5 = at_off<uint2>(aq.seg_vq + b5, need5 ? d * 8u : 0u)->x;
   }
-  vq0[0] = vq.x;
-  vq0[3] = vq0[1];
-  vq0[4] = vq0[2];
-  if (wrap && (need & 0x19u)) {  // the next x-tile's segments of rows y, y+1 and plane z+1
-    vq0[0] = a.seg_vq[s + 1u].x;
-    vq0[3] = a.seg_vq[s1 + 1u].x;
-    vq0[4] = a.seg_vq[s2 + 1u].x;
-  }
-  const uint32_t bit = xl & 63u;
-  const uint64_t below = (1ull << bit) - 1ull;
-  const uint64_t m1 = (uint64_t)g1.x | ((uint64_t)g1.y << 32), m2 = (uint64_t)g2.x | ((uint64_t)g2.y << 32);
-  const uint64_t m5 = (uint64_t)g5.x | ((uint64_t)g5.y << 32);
-  const uint32_t r1 = g1.z + (uint32_t)__popcll(m1 & below), r2 = g2.z + (uint32_t)__popcll(m2 & below);
-  const uint32_t r5 = g5.z + (uint32_t)__popcll(m5 & below);
-  const uint32_t ns[6] = {wrap ? s + 1u : s, s1, s2, wrap ? s1 + 1u : s1, wrap ? s2 + 1u : s2, s5};
-  const uint32_t nr[6] = {wrap ? 0u : rank + 1u, r1, r2, wrap ? 0u : r1 + 1u, wrap ? 0u : r2 + 1u, r5};
-  const uint32_t nx[6] = {xl1, xl, xl, xl1, xl1, xl};
-  const bool inmask[6] = {true, ((m1 >> bit) & 1ull) != 0, ((m2 >> bit) & 1ull) != 0, true, true,
-                          ((m5 >> bit) & 1ull) != 0};
-  const uint32_t *slot_lo = reinterpret_cast<const uint32_t *>(a.slots);  // record bits 0..31
-  uint32_t nrec[6];
-  bool act[6];
-#pragma unroll
-  for (int n = 0; n < 6; ++n) {
-    const bool ok_r = ((need >> n) & 1u) && inmask[n] && nr[n] < cap;
-    nrec[n] = ok_r ? slot_lo[2 * ((size_t)ns[n] * cap + nr[n])] : 0u;
-    act[n] = ok_r && rec_x(nrec[n]) == nx[n];
-  }
-  bool ok = true;
-  // vertex of ring cell n for its local edge e
-  auto vtx = [&](int n, int e, bool used) -> int32_t {
-    const uint32_t m2 = nrec[n];
-    const uint32_t lab = (uint32_t)(s_lab[rec_lut2(m2) * 256 + rec_cfg(m2)] >> (4 * e)) & 0xFu;
-    if (used && (!act[n] || lab == 0xFu)) ok = false;
-    return (int32_t)(vq0[n] + rec_lvb(m2) + lab - vol.vbase + vol.vshift);
+  const uint32_t bit = xl & 63u, blo = bit < 32u ? (1u << bit) - 1u : ~0u, bhi = bit < 32u ? 0u : (1u << (bit - 32u)) - 1u;
+  auto rank_of = [&](const uint4 &gm) {  // (clamped: a group map may be stale where the lane needs no lookup)
+    return min(gm.z + (uint32_t)__popc(gm.x & blo) + (uint32_t)__popc(gm.y & bhi), capq - 1u);
   };
-  int4 *qo = reinterpret_cast<int4 *>(vol.quads) + qb;
-  uint32_t qn = 0;
-  const int32_t self = (int32_t)(vb + vol.vshift);
+  auto in_map = [&](const uint4 &gm) { return (((bit < 32u ? gm.x : gm.y) >> (bit & 31u)) & 1u) != 0u; };
+  const uint32_t r1 = rank_of(g1), r2 = rank_of(g2), r5 = rank_of(g5);
+  const Word2 c13 = *at_off<Word2>(aq.slots + (size_t)b1 * capq, need1 ? (d * capq + r1) * 4u : 0u);
+  const Word2 c24 = *at_off<Word2>(aq.slots + (size_t)b2 * capq, need2 ? (d * capq + r2) * 4u : 0u);
+  const uint32_t c5 = *at_off<uint32_t>(aq.slots + (size_t)b5 * capq, need5 ? (d * capq + r5) * 4u : 0u);
+  uint32_t c0 = own.y, c3 = c13.y, c4 = c24.y, vq0 = vq.x, vq3 = vq1, vq4 = vq2, xn = xl + 1u;
+  // the next active cell of a row is in the segment only if its count says so
+  bool n0 = n0in, n3 = r1 + 1u < capq, n4 = r2 + 1u < capq;
+  if (xn == capq) {  // +x lies in the next x-tile's segments of this row, row y + 1 and plane z + 1
+    xn = 0u;
+    n0 = n3 = n4 = true;
+    uint32_t sn = s0 + d + 1u;
+    asm volatile("" : "+v"(sn));  // (keeps the addresses below out of the lanes' common path)
+    if (e6 || e9) {
+      c0 = aq.slots[(size_t)sn * capq];
+      vq0 = aq.seg_vq[sn].x;
+    }
+    if (e6) {
+      c3 = aq.slots[(size_t)(sn + dy) * capq];
+      vq3 = aq.seg_vq[sn + dy].x;
+    }
+    if (e9) {
+      c4 = aq.slots[(size_t)(sn + dz) * capq];
+      vq4 = aq.seg_vq[sn + dz].x;
+    }
+  }
+  const bool ok0 = n0 && rec_x(c0) == xn, ok3 = n3 && rec_x(c3) == xn, ok4 = n4 && rec_x(c4) == xn;
+  const bool ok1 = in_map(g1) && rec_x(c13.x) == xl, ok2 = in_map(g2) && rec_x(c24.x) == xl;
+  const bool ok5 = in_map(g5) && rec_x(c5) == xl;
+  bool ok = true;
+  // vertex of a ring cell (record m, its segment's first vertex vqn) for its local edge e
+  const uint32_t *const s_lab32 = reinterpret_cast<const uint32_t *>(s_lab);
+  const uint32_t shift = vq_.vshift - base.x;
+  auto vtx = [&](uint32_t m, uint32_t vqn, int e, bool found) -> int32_t {
+    const uint32_t lab = (s_lab32[2u * ((m >> 10) & 0x1FFu) + (e >> 3)] >> (4 * (e & 7))) & 0xFu;
+    if (!found || lab == 0xFu) ok = false;
+    return (int32_t)(vqn + rec_lvb(m) + lab + shift);
+  };
+  int32_t *const qout = vq_.quads + 4ull * qb0;
+  uint32_t qo = dq * 16u;
+  const int32_t self = (int32_t)(vb0 + (dvq & 0xFFFFu) + vq_.vshift);
   if (e6) {
-    const int32_t m0 = self + (int32_t)((labels >> 24) & 0xFu);
-    const int32_t m1 = vtx(0, 7, true), m2 = vtx(3, 4, true), m3 = vtx(1, 5, true);
-    qo[qn++] = v[2] <= iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
+    const int32_t m0 = self + (int32_t)(((uint32_t)labels >> 24) & 0xFu);
+    const int32_t m1 = vtx(c0, vq0, 7, ok0), m2 = vtx(c3, vq3, 4, ok3), m3 = vtx(c13.x, vq1, 5, ok1);
+    *at_off<int4>(qout, qo) = v[2] <= vq_.g.iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
+    qo += 16u;
   }
   if (e9) {
-    const int32_t m0 = self + (int32_t)((labels >> 36) & 0xFu);
-    const int32_t m1 = vtx(2, 1, true), m2 = vtx(4, 3, true), m3 = vtx(0, 11, true);
-    qo[qn++] = v[5] <= iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
+    const int32_t m0 = self + (int32_t)((lab_hi >> 4) & 0xFu);
+    const int32_t m1 = vtx(c24.x, vq2, 1, ok2), m2 = vtx(c4, vq4, 3, ok4), m3 = vtx(c0, vq0, 11, ok0);
+    *at_off<int4>(qout, qo) = v[5] <= vq_.g.iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
+    qo += 16u;
   }
   if (e10) {
-    const int32_t m0 = self + (int32_t)((labels >> 40) & 0xFu);
-    const int32_t m1 = vtx(1, 8, true), m2 = vtx(5, 0, true), m3 = vtx(2, 2, true);
-    qo[qn++] = v[7] <= iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
+    const int32_t m0 = self + (int32_t)((lab_hi >> 8) & 0xFu);
+    const int32_t m1 = vtx(c13.x, vq1, 8, ok1), m2 = vtx(c5, vq5, 0, ok5), m3 = vtx(c24.x, vq2, 2, ok2);
+    *at_off<int4>(qout, qo) = v[7] <= vq_.g.iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
   }
-  if (!ok) atomicOr(vol.status, kStatusLookup);
+  if (!ok) atomicOr(vq_.status, kStatusLookup);
+}
+
+// The lanes with a cell (todo), in runs whose segments lie within vol.span of
+// their first lane's (nearly always one run).
+__device__ __forceinline__ void emit_lanes(EmitArgsK pa, EmitVolK pv, uint2 base, bool todo, uint32_t s, uint32_t rank,
+                                           const uint64_t *s_lab, float *s_acc) {
+  for (uint64_t left = __ballot(todo); left != 0ull; left = __ballot(todo)) {
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)s, __ffsll((long long)left) - 1);
+    const bool mine = todo && s - s0 <= fresh(pv).span;
+    if (mine) emit_cells(pa, pv, base, s0, s, rank, s_lab, s_acc);
+    todo = todo && !mine;
+  }
+}
+
+// Entry i of the emit's table in LDS, by configuration and variant: the label
+// nibbles of edges 0..11, the number of iso vertices (bits 48-51) and the
+// crossed edges (bits 52-63).
+__device__ __forceinline__ uint64_t emit_label(uint32_t i) {
+  const uint64_t l = (&c_label[0][0])[i];
+  const uint32_t info = c_cfg_info[i & 255u], n = i >= 256u ? (info >> 3) & 7u : info & 7u;
+  uint64_t cross = 0;
+#pragma unroll
+  for (int e = 0; e < 12; ++e) cross |= (uint64_t)(((l >> (4 * e)) & 0xFu) != 0xFu) << e;
+  return (l & 0xFFFFFFFFFFFFull) | ((uint64_t)n << 48) | (cross << 52);
 }
 
 // Segment and rank of active cell ch*64 + lane: the chunk's first entry of
@@ -1671,11 +1777,13 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
   const EmitTickets et = emit_tickets(num_chunks, blockIdx.x & 7u, gridDim.x, wpb);
   uint64_t first = emit_ticket_chunk(et, blockIdx.x >> 3, wpb);
   if (first >= et.hi) return;  // (uniform: before the barrier)
-  for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = (&c_label[0][0])[i];
+  for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = emit_label(i);
   uint32_t *ctr = a.emit_ctr + kEmitCtr * ((blockIdx.x & 7u) + 1u);
   __syncthreads();
   const uint32_t lane = lane_id(), wave = wave_id();
   const uint32_t num_ne = min(tot.num_nonempty, a.nsegs);
+  const EmitArgsK pa = (EmitArgsK)__builtin_amdgcn_kernarg_segment_ptr();  // a
+  const uint2 base = make_uint2(a.v.vbase, a.v.qbase);
   for (uint32_t it = 0;; ++it) {
     // the next ticket is asked for before this one's chunks run and published
     // after them; two slots, because thread 0 writes the next iteration's
@@ -1684,8 +1792,9 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
     if (et.dynamic && threadIdx.x == 0) next = atomicAdd(ctr, 1u);
     const uint64_t ch = first + wave;
     if (ch < et.hi) {
-      uint32_t s, rank;
-      if (locate_cell(a, tot, num_ne, (uint32_t)ch, lane, s, rank)) emit_cell(a, a.v, s, rank, s_lab, s_acc + threadIdx.x);
+      uint32_t s = 0, rank = 0;
+      const bool found = locate_cell(a, tot, num_ne, (uint32_t)ch, lane, s, rank);
+      emit_lanes(pa, &pa->v, base, found, s, rank, s_lab, s_acc + threadIdx.x);
     }
     if (!et.dynamic) break;
     if (threadIdx.x == 0) s_ticket[it & 1u] = next;
@@ -1725,7 +1834,7 @@ struct CellPos {
 // row's coordinates) comes through scalar loads for the lanes in the wave's
 // first segment and through vector loads for the others.
 __device__ __forceinline__ CellPos cell_pos(const EmitArgs &a, const EmitVol &vol, uint32_t s, uint32_t rank,
-                                            uint64_t &rec) {
+                                            uint32_t &rec) {
   CellPos c;
   rec = a.slots[(size_t)s * a.cap + rank];
   c.xl = rec_x(rec);
@@ -1754,7 +1863,7 @@ __device__ __forceinline__ CellPos cell_pos(const EmitArgs &a, const EmitVol &vo
   c.y1 = y1;
   c.z1 = z1;
   c.vb = vq.x + rec_lvb(rec) - vol.vbase;
-  c.qb = vq.y + rec_lqb(rec) - vol.qbase;
+  c.qb = vq.y + a.slot_q[(size_t)s * a.cap + rank] - vol.qbase;
   return c;
 }
 
@@ -1823,7 +1932,7 @@ __device__ __forceinline__ void smooth_chunk(const EmitArgs &a, const EmitVol &v
   uint32_t has = 0, bip = 0, qb = 0, ev0 = 0;
   float x1 = 0.0f, y1 = 0.0f, z1 = 0.0f;
   if (found) {
-    uint64_t rec;
+    uint32_t rec;
     const CellPos c = cell_pos(a, vol, s, rank, rec);
     if (c.x >= g.cx || rank >= c.nact) {
       atomicOr(vol.status, kStatusInternal);
@@ -1937,7 +2046,7 @@ __device__ __forceinline__ void smooth_chunk(const EmitArgs &a, const EmitVol &v
 // value.
 __device__ __forceinline__ void reaverage_cell(const EmitArgs &a, const EmitVol &vol, uint32_t s, uint32_t rank,
                                                const uint64_t *s_lab, const uint16_t *s_info, float *s_acc) {
-  uint64_t rec;
+  uint32_t rec;
   const CellPos c = cell_pos(a, vol, s, rank, rec);
   const FieldDesc &g = vol.g;
   const uint32_t cap = a.cap;
@@ -2007,14 +2116,13 @@ __device__ __forceinline__ void reaverage_cell(const EmitArgs &a, const EmitVol 
     }
   }
   const uint32_t nx[6] = {xlm, c.xl, c.xl, xlm, xlm, c.xl};
-  const uint32_t *slot_lo = reinterpret_cast<const uint32_t *>(a.slots);
   uint32_t own_base[8], own_bip[8];  // first edge point of each owner, its bipolar bits
   bool ok = true;
 #pragma unroll
   for (int n = 0; n < 6; ++n) {
     const bool use = (need >> n) & 1u;
     const bool ok_r = use && inmask[n] && nr[n] < cap;
-    const uint32_t m = slot_lo[2 * ((size_t)(ok_r ? ns[n] : s) * cap + (ok_r ? nr[n] : rank))];
+    const uint32_t m = a.slots[(size_t)(ok_r ? ns[n] : s) * cap + (ok_r ? nr[n] : rank)];
     if (use && !(ok_r && rec_x(m) == nx[n])) ok = false;
     own_base[n] = vq0[n] + rec_lvb(m) - vol.vbase + iso_count_lds(s_info, rec_cfg(m), rec_lut2(m));
     own_bip[n] = owned_bipolar(rec_cfg(m));
@@ -2215,18 +2323,20 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
   // kMaxBatch entries keep the workgroup's LDS at 20 KB, 8 workgroups per CU)
   __shared__ uint32_t s_soff[kMaxBatch];
   const EmitArgs &a = b.a;
+  static_assert(offsetof(BatchEmitArgs, a) == 0, "the kernel's arguments start with a");
+  const EmitArgsK pa = (EmitArgsK)__builtin_amdgcn_kernarg_segment_ptr();  // b.a
   const Totals tot = *a.totals;
   const uint32_t num_chunks = (uint32_t)min((uint64_t)tot.num_chunks, a.max_chunks);
   if (!workgroup_has_chunks(num_chunks)) return;  // (uniform: before the barrier)
-  for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = (&c_label[0][0])[i];
+  for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = emit_label(i);
   for (uint32_t i = threadIdx.x; i < b.nvol; i += kEmitThreads) s_soff[i] = b.seg_off[i];
   __syncthreads();
   const uint32_t lane = lane_id(), wave = wave_id();
   const uint32_t num_ne = min(tot.num_nonempty, a.nsegs);
   const ChunkIter it = chunk_iter(num_chunks, wave);
   for (uint32_t ch = it.next; ch < it.end; ch += it.step) {
-    uint32_t s, rank;
-    if (!locate_cell(a, tot, num_ne, ch, lane, s, rank)) continue;
+    uint32_t s = 0, rank = 0;
+    bool todo = locate_cell(a, tot, num_ne, ch, lane, s, rank);
     // the last volume whose first segment is <= s (empty volumes share it)
     uint32_t lo = 0, hi = b.nvol;
     while (hi - lo > 1) {
@@ -2236,36 +2346,11 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
     // the lanes of one volume at a time (64 consecutive active cells rarely
     // span two volumes), so that the volume's descriptor is wave-uniform and
     // comes in through scalar loads instead of occupying vector registers
-    for (;;) {
-      const uint32_t v = __builtin_amdgcn_readfirstlane(lo);
-      if (lo != v) continue;
+    for (uint64_t left = __ballot(todo); left != 0ull; left = __ballot(todo)) {
+      const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)lo, __ffsll((long long)left) - 1);
       const __attribute__((address_space(4))) BatchVol *bv = (const __attribute__((address_space(4))) BatchVol *)b.vols + v;
-      const __attribute__((address_space(4))) uint2 *bb = (const __attribute__((address_space(4))) uint2 *)b.base + v;
-      EmitVol e;
-      e.g.f = bv->c.g.f;
-      e.g.X = bv->c.g.X;
-      e.g.Y = bv->c.g.Y;
-      e.g.Z = bv->c.g.Z;
-      e.g.cx = bv->c.g.cx;
-      e.g.cy = bv->c.g.cy;
-      e.g.cz = bv->c.g.cz;
-      e.g.iso = bv->c.g.iso;
-      float *const co = bv->coords;
-      e.xt_c = co;
-      e.yt_c = co + e.g.X;
-      e.zt_c = co + e.g.X + e.g.Y;
-      e.XT = bv->c.XT;
-      e.seg_off = bv->seg_off;
-      e.vbase = bb->x;
-      e.qbase = bb->y;
-      e.verts = bv->verts;
-      e.vcap = e.verts ? bv->vcap : 0;
-      e.quads = bv->quads;
-      e.qcap = e.quads ? bv->qcap : 0;
-      uint32_t *const cnt = bv->counts;
-      e.status = cnt ? cnt + 3 : a.v.status;
-      emit_cell(a, e, s, rank, s_lab, s_acc + threadIdx.x);
-      break;
+      emit_lanes(pa, &bv->e, const_u2(b.base, v), todo && lo == v, s, rank, s_lab, s_acc + threadIdx.x);
+      todo = todo && lo != v;
     }
   }
 }
@@ -2277,7 +2362,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
 struct CellsArgs {
   uint32_t XT, cap, cx, nsegs;
   const uint2 *seg_counts;
-  const uint64_t *slots;
+  const uint32_t *slots;
   const uint2 *seg_vq;
   const uint2 *ne;
   const Totals *totals;
@@ -2300,7 +2385,7 @@ __global__ __launch_bounds__(256) void k_cells(CellsArgs a) {
     for (uint32_t r = threadIdx.x; r < n; r += blockDim.x) {
       const uint64_t pos = (uint64_t)e.y + r;
       if (pos >= a.capacity) break;
-      const uint64_t rec = a.slots[(size_t)sg * a.cap + r];
+      const uint32_t rec = a.slots[(size_t)sg * a.cap + r];
       a.cell_index[pos] = xt * a.cap + rec_x(rec) + a.cx * row;
       a.cfg[pos] = (uint8_t)rec_cfg(rec);
       a.flags[pos] = (uint8_t)rec_lut2(rec);
