@@ -371,7 +371,7 @@ ScratchLayout scratch_layout(const Plan &p) {
   // given scratch size admits does not change
   L.slots = take(p.nslots * 8);
   L.slot_q = L.slots + p.nslots * sizeof(uint32_t) + 16;
-  L.gmap = take(p.nsegs * (p.cap / 64) * sizeof(uint4));
+  L.gmap = take(p.nsegs * (p.cap / 16) * sizeof(uint32_t));
   L.coords = take(p.ncoord * sizeof(float));
   L.total = off;
   return L;
@@ -420,7 +420,7 @@ int ensure_scratch(mdmc_ctx *ctx, const Plan &p) {
   s.totals = reinterpret_cast<Totals *>(b + o_totals);
   s.slots = reinterpret_cast<uint32_t *>(b + o_slots);
   s.slot_q = reinterpret_cast<uint16_t *>(b + lay.slot_q);
-  s.gmap = reinterpret_cast<uint4 *>(b + o_gmap);
+  s.gmap = reinterpret_cast<uint32_t *>(b + o_gmap);
   s.coords = reinterpret_cast<float *>(b + o_coords);
   ctx->s = s;
   return MDMC_OK;
@@ -748,7 +748,7 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     b.c.seg_counts = S.seg_counts + seg_off;
     b.c.slots = S.slots + seg_off * cap;
     b.c.slot_q = S.slot_q + seg_off * cap;
-    b.c.gmap = S.gmap + seg_off * (cap / 64);
+    b.c.gmap = S.gmap + seg_off * (cap / 16);
     b.tile_off = tiles0[v] = (uint32_t)tile_off;
     b.NRB = NRB;
     b.NKP = NKP;

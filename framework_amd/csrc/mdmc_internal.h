@@ -34,7 +34,7 @@ struct Scratch {
   Totals *totals;
   uint32_t *slots;
   uint16_t *slot_q;
-  uint4 *gmap;
+  uint32_t *gmap;
   float *coords;
 };
 

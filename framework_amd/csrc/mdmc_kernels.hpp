@@ -9,7 +9,7 @@
 //               and listed in LDS; listed cells get their 2B/3B table variant,
 //               vertex and quad counts, a DPP-scan rank and a 32-bit record in
 //               their segment's slot range (segment = one cell row of one
-//               x-tile in one plane), plus a per-64-cell group map (active
+//               x-tile in one plane), plus a per-16-cell group map (active
 //               mask, first rank).  Workgroups map to tiles XCD by XCD (mdmc_tilemap.h).
 //               k_classify is the z-marching form for any row length.
 //   k_scan      single-pass decoupled look-back scan (ticketed tiles) over the
@@ -202,8 +202,8 @@ struct ClassifyArgs {
   uint2 *seg_counts;      // per segment: {nact | nquad << 16, nvert}
   uint32_t *slots;        // per segment: 64*W record slots
   uint16_t *slot_q;       // per record slot: the cell's first quad
-  uint4 *gmap;            // per segment and 64-cell group: {active mask lo, hi, rank of
-                          // the group's first active cell, 0}; written for non-empty groups
+  uint32_t *gmap;         // per segment and 16-cell group: active mask | rank of the group's
+                          // first active cell << 16; written for non-empty groups
   unsigned long long *scan_state;  // zeroed here for k_scan
   uint32_t scan_state_words;
   uint2 *seg_pad;         // segment totals past the last segment, up to a whole scan tile
@@ -328,8 +328,11 @@ __global__ __launch_bounds__(64) void k_classify(ClassifyArgs a) {
         const bool active = (x < g.cx) && (cfg != 0u) && (cfg != 0xFFu);
         const uint64_t bal = __ballot(active);
         if (bal == 0ull) continue;
-        if (lane == 0)
-          a.gmap[(size_t)seg * W + c] = make_uint4((uint32_t)bal, (uint32_t)(bal >> 32), cnt_a, 0u);
+        if (lane < 4u) {
+          const uint32_t m16 = (uint32_t)(bal >> (16u * lane)) & 0xFFFFu;
+          const uint32_t before = (uint32_t)__popcll(bal & ((1ull << (16u * lane)) - 1ull));
+          if (m16) a.gmap[(size_t)seg * (4u * W) + 4u * c + lane] = m16 | ((cnt_a + before) << 16);
+        }
         uint32_t nv = 0, nq = 0, lut2 = 0;
         if (active) {
           const uint32_t info = s_info[cfg];
@@ -535,23 +538,15 @@ struct PtList {
     }
   }
 
-  // Group maps of the groups that lanes 16 i .. 16 i + 15 hold; incl: active
-  // cells of the row up to and with this lane.
+  // Group maps of the groups that lanes 4 i .. 4 i + 3 hold, from lane 4 i + 3
+  // (grp: its group); incl: active cells of the row up to and with this lane.
   __device__ __forceinline__ void group_maps(uint32_t seg, uint32_t grp, uint32_t act, uint32_t incl) {
     const uint32_t lane = lane_id();
-    uint32_t mlo = (lane & 8u) ? 0u : act << (4u * (lane & 7u));
-    uint32_t mhi = (lane & 8u) ? act << (4u * (lane & 7u)) : 0u;
-    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 1, 0xF, 0xF, true);
-    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 1, 0xF, 0xF, true);
-    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 2, 0xF, 0xF, true);
-    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 2, 0xF, 0xF, true);
-    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 4, 0xF, 0xF, true);
-    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 4, 0xF, 0xF, true);
-    mlo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mlo, kDppRowShr + 8, 0xF, 0xF, true);
-    mhi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mhi, kDppRowShr + 8, 0xF, 0xF, true);
-    if ((lane & 15u) == 15u && (mlo | mhi) != 0u)
-      a.gmap[(size_t)seg * (CAP / 64u) + grp] =
-          make_uint4(mlo, mhi, incl - (uint32_t)(__popc(mlo) + __popc(mhi)), 0u);
+    uint32_t m = act << (4u * (lane & 3u));
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, kDppRowShr + 1, 0xF, 0xF, true);
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, kDppRowShr + 2, 0xF, 0xF, true);
+    // (lanes other than 4 i + 3 hold bits of the group before)
+    if ((lane & 3u) == 3u && m != 0u) a.gmap[(size_t)seg * (CAP / 16u) + grp] = m | ((incl - (uint32_t)__popc(m)) << 16);
   }
 
   // Variant-1 test of a 2B/3B cell (its neighbour across the listed face is
@@ -784,7 +779,7 @@ struct PtWide {
         const uint32_t act = active_cells(s_w[word(m, c)]) & cells_in_grid(x0 + 256u * c + 4u * lane, g.cx);
         if (__ballot(act != 0u) == 0ull) continue;
         const uint32_t cnt = (uint32_t)__popc(act), incl = wave_incl_scan_dpp(cnt);
-        L.group_maps(seg, 4u * c + (lane >> 4), act, L.have - start + incl);
+        L.group_maps(seg, 16u * c + (lane >> 2), act, L.have - start + incl);
         L.append(m, 256u * c + 4u * lane, act, L.have + incl - cnt);
         L.have += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
         while (L.have - L.done >= (uint32_t)kWave) L.template drain<KP>(kWave);
@@ -885,7 +880,7 @@ struct PtNarrow {
       const uint32_t start = L.have + first;
       if (l == 0u && ok)
         sh.row[m] = make_uint2(seg, start | (y + 1u < g.cy ? 1u << 16 : 0u) | (z + 1u < g.cz ? 1u << 17 : 0u));
-      L.group_maps(seg, (xoff >> 6) + (l >> 4), act, (ok ? L.before(m).x & 0xFFFFu : 0u) + incl);
+      L.group_maps(seg, (xoff >> 4) + (l >> 2), act, (ok ? L.before(m).x & 0xFFFFu : 0u) + incl);
       L.append(m, xoff + 4u * l, act, start + incl - cnt);
       L.have += total;
       while (L.have - L.done >= (uint32_t)kWave) L.template drain<KP>(kWave);
@@ -1341,6 +1336,9 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(ScanArgs a) {
 // active mask below x.
 
 constexpr int kEmitThreads = 256;
+// Words of LDS of an emit wave: 12 sums a lane, then its vertices (up to 4 of
+// 3 words a cell) or quads (up to 3 of 4 words) on their way out.
+constexpr uint32_t kEmitStage = 12 * kWave;
 
 struct EmitArgs {
   EmitVol v;  // the volume (single-volume launches)
@@ -1350,7 +1348,7 @@ struct EmitArgs {
   const uint2 *seg_vq;
   const uint32_t *slots;
   const uint16_t *slot_q;
-  const uint4 *gmap;
+  const uint32_t *gmap;
   const uint2 *ne;
   const uint32_t *chunk_ne;
   const Totals *totals;
@@ -1368,7 +1366,11 @@ __device__ __forceinline__ uint2 const_u2(const uint2 *p, uint32_t i) {
   const __attribute__((address_space(4))) uint32_t *w = (const __attribute__((address_space(4))) uint32_t *)p;
   return make_uint2(w[2 * i], w[2 * i + 1]);
 }
-// Its first word only.
+// Entry i of an array of words.
+__device__ __forceinline__ uint32_t const_u1(const uint32_t *p, uint32_t i) {
+  return ((const __attribute__((address_space(4))) uint32_t *)p)[i];
+}
+// First word of entry i of an array of uint2.
 __device__ __forceinline__ uint32_t const_u2x(const uint2 *p, uint32_t i) {
   return ((const __attribute__((address_space(4))) uint32_t *)p)[2 * i];
 }
@@ -1400,7 +1402,10 @@ __device__ __forceinline__ T *at_off(void *base, uint32_t off) {
 // Two consecutive words or floats, and a vertex, at the alignment of one word.
 typedef uint32_t Word2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef float Float2 __attribute__((ext_vector_type(2), aligned(4)));
-typedef float Float3 __attribute__((ext_vector_type(3), aligned(4)));
+struct Float3 {  // (a 3-vector type would be stored as 4 words)
+  float x, y, z;
+};
+typedef int Int4 __attribute__((ext_vector_type(4)));
 
 // The active cells of the calling lanes (segment s, rank within it) of volume
 // vol: their vertices and the quads of their owned edges.  s0: the segment of
@@ -1410,7 +1415,7 @@ typedef float Float3 __attribute__((ext_vector_type(3), aligned(4)));
 // the division of a segment number into tile, row and plane on every lane,
 // were a quarter of the kernel's issue slots.)  s_lab: kEmitLab entries.
 __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base, uint32_t s0, uint32_t s,
-                                           uint32_t rank, const uint64_t *s_lab, float *s_acc) {
+                                           uint32_t rank, const uint64_t *s_lab, float *s_wave) {
   const EmitArgs &a = fresh(pa);
   const EmitVol &vol = fresh(pv);
   const FieldDesc &g = vol.g;
@@ -1495,11 +1500,12 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
   if (x == 0u) use &= ~0x898u;
   if (j == 0u) use &= ~0x131u;
   if (k == 0u) use &= ~0x00Fu;
-  // Group sums live in LDS, component c of group q at s_acc[(3q + c) * T]
-  // (T = threads per block; the caller offsets s_acc by the thread index).
-  // They start at -0.0, so the first addition yields the point itself
-  // bitwise, as the reference's "assign the first, add the rest" does.
-  constexpr uint32_t T = kEmitThreads;
+  // Group sums live in the wave's part of LDS, component c of group q of a lane
+  // at s_acc[(3q + c) * T].  They start at -0.0, so the first addition yields
+  // the point itself bitwise, as the reference's "assign the first, add the
+  // rest" does.
+  constexpr uint32_t T = kWave;
+  float *const s_acc = s_wave + lane_id();
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     if ((uint32_t)q < niso) {
@@ -1538,11 +1544,31 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
     cnt += 1u << (8 * lab);
   }
   const uint32_t b6 = (use >> 6) & 1u, b9 = (use >> 9) & 1u, b10 = (use >> 10) & 1u;
-  const uint32_t nv = niso + b6 + b9 + b10;
-  if ((uint64_t)vb0 + (dvq & 0xFFFFu) + nv <= vol.vcap) {
-    float *const out = vol.verts + 3ull * vb0;
-    uint32_t o = (dvq & 0xFFFFu) * 12u;
-    const float qnan = __int_as_float(0x7FC00000);
+  const uint32_t nv = niso + b6 + b9 + b10, dv = dvq & 0xFFFFu;
+  const uint64_t lanes = __ballot(true);
+  const uint32_t idx = mbcnt64(lanes), nlanes = (uint32_t)__popcll(lanes);
+  float *const out = vol.verts + 3ull * vb0;
+  const float qnan = __int_as_float(0x7FC00000);
+  const bool vfit = (uint64_t)vb0 + dv + nv <= vol.vcap;
+  if (__ballot(niso != 1u || dv + nv > kEmitStage / 3u) == 0ull) {
+    // One iso vertex in every cell (nearly all chunks): the vertices are put
+    // in order in the wave's part of LDS and leave as whole lines.  A store
+    // per lane and vertex touches a dozen lines each time, four times over.
+    const uint32_t n = cnt & 0xFFu;
+    const float dn = (float)n;
+    const Float3 r{n ? s_acc[0] / dn : qnan, n ? s_acc[T] / dn : qnan, n ? s_acc[2 * T] / dn : qnan};
+    if (vfit) {
+      Float3 *st = reinterpret_cast<Float3 *>(s_wave + 3u * dv);
+      *st++ = r;
+      if (b6) *st++ = Float3{ex[0], ey[0], ez[0]};
+      if (b9) *st++ = Float3{ex[1], ey[1], ez[1]};
+      if (b10) *st = Float3{ex[2], ey[2], ez[2]};
+    }
+    const uint64_t fits = __ballot(vfit);
+    const uint32_t total = fits ? (uint32_t)__builtin_amdgcn_readlane((int)(dv + nv), 63 - __builtin_clzll(fits)) : 0u;
+    for (uint32_t i = idx; i < total; i += nlanes) *at_off<Float3>(out, i * 12u) = *reinterpret_cast<const Float3 *>(s_wave + 3u * i);
+  } else if (vfit) {
+    uint32_t o = dv * 12u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if ((uint32_t)q < niso) {
@@ -1559,9 +1585,8 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
     if (b6) { *at_off<Float3>(out, o) = Float3{ex[0], ey[0], ez[0]}; o += 12u; }
     if (b9) { *at_off<Float3>(out, o) = Float3{ex[1], ey[1], ez[1]}; o += 12u; }
     if (b10) *at_off<Float3>(out, o) = Float3{ex[2], ey[2], ez[2]};
-  } else {
-    atomicOr(vol.status, kStatusVertexOverflow);
   }
+  if (!vfit) atomicOr(vol.status, kStatusVertexOverflow);
 
   // Quads (dmc.cu:1983-2047): rings in ccw order, reversed (0,3,2,1) when
   // the owned edge's first corner is not above iso.  The arguments are read
@@ -1570,9 +1595,8 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
   const EmitArgs &aq = fresh(pa);
   const EmitVol &vq_ = fresh(pv);
   const bool e6 = b6 && xin && yin, e9 = b9 && xin && zin, e10 = b10 && yin && zin;
-  if (!(e6 || e9 || e10)) return;
+  if (__ballot(e6 || e9 || e10) == 0ull) return;
   const uint32_t nq = (uint32_t)e6 + (uint32_t)e9 + (uint32_t)e10, dq = dvq >> 16;
-  if ((uint64_t)qb0 + dq + nq > vq_.qcap) { atomicOr(vq_.status, kStatusQuadOverflow); return; }
   // Ring cells n = 0 (+1,0,0), 1 (0,+1,0), 2 (0,0,+1), 3 (+1,+1,0),
   // 4 (+1,0,+1), 5 (0,+1,+1).  A ring cell contains the crossing edge, so it
   // is active.  Cells 1, 2 and 5 are found through their segments' group
@@ -1583,23 +1607,23 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
   // the cell found.  A lookup the quads do not need reads at offset 0 of a
   // segment in range, so that every load is in bounds.
   const bool need1 = e6 || e10, need2 = e9 || e10, need5 = e10;
-  const uint32_t capq = aq.cap, G = capq >> 6, dy = vq_.XT, dz = vq_.XT * vq_.g.cy, last = aq.nsegs - 1u;
+  const uint32_t capq = aq.cap, G = capq >> 4, dy = vq_.XT, dz = vq_.XT * vq_.g.cy, last = aq.nsegs - 1u;
   const uint32_t b1 = min(s0u + dy, last), b2 = min(s0u + dz, last), b5 = min(s0u + dy + dz, last);
-  const uint32_t goff = (d * G + (xl >> 6)) * 16u;
-  const uint4 g1 = *at_off<uint4>(aq.gmap + (size_t)b1 * G, need1 ? goff : 0u);
-  const uint4 g2 = *at_off<uint4>(aq.gmap + (size_t)b2 * G, need2 ? goff : 0u);
-  const uint4 g5 = *at_off<uint4>(aq.gmap + (size_t)b5 * G, need5 ? goff : 0u);
+  const uint32_t goff = (d * G + (xl >> 4)) * 4u;
+  const uint32_t g1 = *at_off<uint32_t>(aq.gmap + (size_t)b1 * G, need1 ? goff : 0u);
+  const uint32_t g2 = *at_off<uint32_t>(aq.gmap + (size_t)b2 * G, need2 ? goff : 0u);
+  const uint32_t g5 = *at_off<uint32_t>(aq.gmap + (size_t)b5 * G, need5 ? goff : 0u);
   uint32_t vq1 = const_u2x(aq.seg_vq, b1), vq2 = const_u2x(aq.seg_vq, b2), vq5 = const_u2x(aq.seg_vq, b5);
   if (d != 0u) {
     vq1 = at_off<uint2>(aq.seg_vq + b1, need1 ? d * 8u : 0u)->x;
     vq2 = at_off<uint2>(aq.seg_vq + b2, need2 ? d * 8u : 0u)->x;
     vq5 = at_off<uint2>(aq.seg_vq + b5, need5 ? d * 8u : 0u)->x;
   }
-  const uint32_t bit = xl & 63u, blo = bit < 32u ? (1u << bit) - 1u : ~0u, bhi = bit < 32u ? 0u : (1u << (bit - 32u)) - 1u;
-  auto rank_of = [&](const uint4 &gm) {  // (clamped: a group map may be stale where the lane needs no lookup)
-    return min(gm.z + (uint32_t)__popc(gm.x & blo) + (uint32_t)__popc(gm.y & bhi), capq - 1u);
+  const uint32_t bit = xl & 15u, below = (1u << bit) - 1u;
+  auto rank_of = [&](uint32_t gm) {  // (clamped: a group map may be stale where the lane needs no lookup)
+    return min((gm >> 16) + (uint32_t)__popc(gm & below), capq - 1u);
   };
-  auto in_map = [&](const uint4 &gm) { return (((bit < 32u ? gm.x : gm.y) >> (bit & 31u)) & 1u) != 0u; };
+  auto in_map = [&](uint32_t gm) { return ((gm >> bit) & 1u) != 0u; };
   const uint32_t r1 = rank_of(g1), r2 = rank_of(g2), r5 = rank_of(g5);
   const Word2 c13 = *at_off<Word2>(aq.slots + (size_t)b1 * capq, need1 ? (d * capq + r1) * 4u : 0u);
   const Word2 c24 = *at_off<Word2>(aq.slots + (size_t)b2 * capq, need2 ? (d * capq + r2) * 4u : 0u);
@@ -1637,37 +1661,41 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
     if (!found || lab == 0xFu) ok = false;
     return (int32_t)(vqn + rec_lvb(m) + lab + shift);
   };
-  int32_t *const qout = vq_.quads + 4ull * qb0;
-  uint32_t qo = dq * 16u;
+  // in order in the wave's part of LDS (like the vertices, 3 quads a cell fit)
+  const bool qfit = (uint64_t)qb0 + dq + nq <= vq_.qcap && dq + nq <= kEmitStage / 4u;
+  Int4 *st = reinterpret_cast<Int4 *>(s_wave) + (qfit ? dq : 0u);
   const int32_t self = (int32_t)(vb0 + (dvq & 0xFFFFu) + vq_.vshift);
   if (e6) {
     const int32_t m0 = self + (int32_t)(((uint32_t)labels >> 24) & 0xFu);
     const int32_t m1 = vtx(c0, vq0, 7, ok0), m2 = vtx(c3, vq3, 4, ok3), m3 = vtx(c13.x, vq1, 5, ok1);
-    *at_off<int4>(qout, qo) = v[2] <= vq_.g.iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
-    qo += 16u;
+    if (qfit) *st++ = v[2] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
   }
   if (e9) {
     const int32_t m0 = self + (int32_t)((lab_hi >> 4) & 0xFu);
     const int32_t m1 = vtx(c24.x, vq2, 1, ok2), m2 = vtx(c4, vq4, 3, ok4), m3 = vtx(c0, vq0, 11, ok0);
-    *at_off<int4>(qout, qo) = v[5] <= vq_.g.iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
-    qo += 16u;
+    if (qfit) *st++ = v[5] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
   }
   if (e10) {
     const int32_t m0 = self + (int32_t)((lab_hi >> 8) & 0xFu);
     const int32_t m1 = vtx(c13.x, vq1, 8, ok1), m2 = vtx(c5, vq5, 0, ok5), m3 = vtx(c24.x, vq2, 2, ok2);
-    *at_off<int4>(qout, qo) = v[7] <= vq_.g.iso ? make_int4(m0, m1, m2, m3) : make_int4(m0, m3, m2, m1);
+    if (qfit) *st++ = v[7] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
   }
+  const uint64_t fits = __ballot(qfit);
+  const uint32_t total = fits ? (uint32_t)__builtin_amdgcn_readlane((int)(dq + nq), 63 - __builtin_clzll(fits)) : 0u;
+  int32_t *const qout = vq_.quads + 4ull * qb0;
+  for (uint32_t i = idx; i < total; i += nlanes) *at_off<Int4>(qout, i * 16u) = reinterpret_cast<const Int4 *>(s_wave)[i];
+  if (!qfit && nq) atomicOr(vq_.status, kStatusQuadOverflow);
   if (!ok) atomicOr(vq_.status, kStatusLookup);
 }
 
 // The lanes with a cell (todo), in runs whose segments lie within vol.span of
 // their first lane's (nearly always one run).
 __device__ __forceinline__ void emit_lanes(EmitArgsK pa, EmitVolK pv, uint2 base, bool todo, uint32_t s, uint32_t rank,
-                                           const uint64_t *s_lab, float *s_acc) {
+                                           const uint64_t *s_lab, float *s_wave) {
   for (uint64_t left = __ballot(todo); left != 0ull; left = __ballot(todo)) {
     const uint32_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)s, __ffsll((long long)left) - 1);
     const bool mine = todo && s - s0 <= fresh(pv).span;
-    if (mine) emit_cells(pa, pv, base, s0, s, rank, s_lab, s_acc);
+    if (mine) emit_cells(pa, pv, base, s0, s, rank, s_lab, s_wave);
     todo = todo && !mine;
   }
 }
@@ -1691,7 +1719,7 @@ __device__ __forceinline__ uint64_t emit_label(uint32_t i) {
 __device__ __forceinline__ bool locate_cell(const EmitArgs &a, const Totals &tot, uint32_t num_ne,
                                             uint32_t ch, uint32_t lane, uint32_t &s, uint32_t &rank) {
   const uint32_t act = ch * 64u + lane;
-  const uint32_t u0 = a.chunk_ne[ch];
+  const uint32_t u0 = const_u1(a.chunk_ne, (uint32_t)__builtin_amdgcn_readfirstlane((int)ch));  // (ch is uniform)
   const uint2 wl = (u0 < num_ne && u0 + lane <= num_ne) ? a.ne[u0 + lane] : make_uint2(0u, 0xFFFFFFFFu);
   uint32_t m = 0;
 #pragma unroll
@@ -1768,7 +1796,7 @@ constexpr int kEmitPersistPerCu = 8;
 __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_emit(EmitArgs a) {
   constexpr uint32_t wpb = kEmitThreads / kWave;
   __shared__ uint64_t s_lab[2 * 256];
-  __shared__ float s_acc[12 * kEmitThreads];
+  __shared__ __align__(16) float s_acc[kEmitStage * wpb];
   __shared__ uint32_t s_ticket[2];
   const Totals tot = *a.totals;
   // Counts are clamped to buffer capacities so that no access can leave the
@@ -1794,7 +1822,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
     if (ch < et.hi) {
       uint32_t s = 0, rank = 0;
       const bool found = locate_cell(a, tot, num_ne, (uint32_t)ch, lane, s, rank);
-      emit_lanes(pa, &pa->v, base, found, s, rank, s_lab, s_acc + threadIdx.x);
+      emit_lanes(pa, &pa->v, base, found, s, rank, s_lab, s_acc + kEmitStage * wave);
     }
     if (!et.dynamic) break;
     if (threadIdx.x == 0) s_ticket[it & 1u] = next;
@@ -2082,36 +2110,31 @@ __device__ __forceinline__ void reaverage_cell(const EmitArgs &a, const EmitVol 
   const uint32_t need1 = need & 0x0Au, need2 = need & 0x14u, need5 = need & 0x20u, needw = need & 0x19u;
   const uint32_t ns[6] = {wrap ? s - 1u : s, need1 ? s - dy : s, need2 ? s - dz : s,
                           wrap ? s - 1u - dy : s - dy, wrap ? s - 1u - dz : s - dz, need5 ? s - dy - dz : s};
-  const uint32_t G = cap >> 6;
-  const uint4 g1 = a.gmap[(size_t)ns[1] * G + (c.xl >> 6)], g2 = a.gmap[(size_t)ns[2] * G + (c.xl >> 6)];
-  const uint4 g5 = a.gmap[(size_t)ns[5] * G + (c.xl >> 6)];
+  const uint32_t G = cap >> 4;
+  const uint32_t g1 = a.gmap[(size_t)ns[1] * G + (c.xl >> 4)], g2 = a.gmap[(size_t)ns[2] * G + (c.xl >> 4)];
+  const uint32_t g5 = a.gmap[(size_t)ns[5] * G + (c.xl >> 4)];
   uint32_t vq0[6];
   vq0[1] = a.seg_vq[ns[1]].x;
   vq0[2] = a.seg_vq[ns[2]].x;
   vq0[5] = a.seg_vq[ns[5]].x;
-  const uint32_t bit = c.xl & 63u;
-  const uint64_t below = (1ull << bit) - 1ull;
-  const uint64_t m1 = (uint64_t)g1.x | ((uint64_t)g1.y << 32), m2 = (uint64_t)g2.x | ((uint64_t)g2.y << 32);
-  const uint64_t m5 = (uint64_t)g5.x | ((uint64_t)g5.y << 32);
-  const uint32_t r1 = g1.z + (uint32_t)__popcll(m1 & below), r2 = g2.z + (uint32_t)__popcll(m2 & below);
-  const uint32_t r5 = g5.z + (uint32_t)__popcll(m5 & below);
+  const uint32_t bit = c.xl & 15u, below = (1u << bit) - 1u;
+  const uint32_t r1 = (g1 >> 16) + (uint32_t)__popc(g1 & below), r2 = (g2 >> 16) + (uint32_t)__popc(g2 & below);
+  const uint32_t r5 = (g5 >> 16) + (uint32_t)__popc(g5 & below);
   uint32_t nr[6] = {rank - 1u, r1, r2, r1 - 1u, r2 - 1u, r5};
-  bool inmask[6] = {rank > 0u, ((m1 >> bit) & 1ull) != 0, ((m2 >> bit) & 1ull) != 0, r1 > 0u, r2 > 0u,
-                    ((m5 >> bit) & 1ull) != 0};
+  bool inmask[6] = {rank > 0u, ((g1 >> bit) & 1u) != 0, ((g2 >> bit) & 1u) != 0, r1 > 0u, r2 > 0u,
+                    ((g5 >> bit) & 1u) != 0};
   vq0[0] = c.seg_vb;
   vq0[3] = vq0[1];
   vq0[4] = vq0[2];
   if (wrap && needw) {  // owners 0, 3, 4: the last cells of the previous x-tile's segments
-    const uint32_t gw = (cap - 1u) >> 6, bw = (cap - 1u) & 63u;
-    const uint64_t bwl = (1ull << bw) - 1ull;
+    const uint32_t gw = (cap - 1u) >> 4;
 #pragma unroll
     for (int n = 0; n < 6; ++n) {
       if (n != 0 && n != 3 && n != 4) continue;
       const uint32_t sn = ((need >> n) & 1u) ? ns[n] : s;  // in bounds when not needed
-      const uint4 gx = a.gmap[(size_t)sn * G + gw];
-      const uint64_t mx = (uint64_t)gx.x | ((uint64_t)gx.y << 32);
-      nr[n] = gx.z + (uint32_t)__popcll(mx & bwl);
-      inmask[n] = ((mx >> bw) & 1ull) != 0;
+      const uint32_t gx = a.gmap[(size_t)sn * G + gw];
+      nr[n] = (gx >> 16) + (uint32_t)__popc(gx & 0x7FFFu);
+      inmask[n] = ((gx >> 15) & 1u) != 0;
       vq0[n] = a.seg_vq[sn].x;
     }
   }
@@ -2318,7 +2341,7 @@ struct BatchEmitArgs {
 // binary search over the volumes' first segments.
 __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_emit_batch(BatchEmitArgs b) {
   __shared__ uint64_t s_lab[2 * 256];
-  __shared__ float s_acc[12 * kEmitThreads];
+  __shared__ __align__(16) float s_acc[kEmitStage * (kEmitThreads / kWave)];
   // first segment of each volume (the search below reads entries 1 .. nvol-1;
   // kMaxBatch entries keep the workgroup's LDS at 20 KB, 8 workgroups per CU)
   __shared__ uint32_t s_soff[kMaxBatch];
@@ -2349,7 +2372,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(8,
     for (uint64_t left = __ballot(todo); left != 0ull; left = __ballot(todo)) {
       const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)lo, __ffsll((long long)left) - 1);
       const __attribute__((address_space(4))) BatchVol *bv = (const __attribute__((address_space(4))) BatchVol *)b.vols + v;
-      emit_lanes(pa, &bv->e, const_u2(b.base, v), todo && lo == v, s, rank, s_lab, s_acc + threadIdx.x);
+      emit_lanes(pa, &bv->e, const_u2(b.base, v), todo && lo == v, s, rank, s_lab, s_acc + kEmitStage * wave);
       todo = todo && lo != v;
     }
   }
