@@ -215,6 +215,11 @@ int plan_tiling(const uint32_t dims[3], Plan *p, const int *opt) {
   p->band = band_opt > 0 && band_opt <= 64 ? (uint32_t)band_opt : 1u;
   p->NRBp = nrb;
   p->NKBp = (p->cz + p->ptKP - 1) / p->ptKP;
+  // the scan by whole planes, if a workgroup holds one (a plane's segments and
+  // the sums are 32-bit counts well within range)
+  const uint64_t plane_segs = (uint64_t)p->XT * p->cy, parts = (uint64_t)p->XT * nrb * p->cz;
+  p->scan_planes = !p->zmarch && plane_segs <= kPlaneScanSegs && parts <= kPlaneScanParts
+                       ? (uint32_t)(kPlaneScanSegs / plane_segs) : 0u;
   // 8 XCDs, each at most ceil(NKB * groups / 8) group tiles of `band` columns
   const uint64_t ng = ((uint64_t)p->XT * nrb + p->band - 1) / p->band;
   p->pt_blocks = 8ull * p->band * (((uint64_t)p->NKBp * ng + 7) / 8);
@@ -347,7 +352,7 @@ int capture_guard(mdmc_ctx *ctx, hipStream_t st) {
 }
 
 struct ScratchLayout {
-  size_t counts, vq, ne, chunk, state, ticket, totals, slots, slot_q, gmap, coords, total;
+  size_t counts, vq, ne, chunk, state, ticket, totals, slots, slot_q, part, gmap, coords, total;
 };
 
 ScratchLayout scratch_layout(const Plan &p) {
@@ -367,10 +372,12 @@ ScratchLayout scratch_layout(const Plan &p) {
   L.ticket = take(kTicketBytes);
   L.totals = take(sizeof(Totals));
   // records (4 bytes a slot, two words of slack for pair loads), then the first
-  // quads (2 bytes a slot); the region keeps 8 bytes a slot, so that what a
-  // given scratch size admits does not change
+  // quads (2 bytes a slot), then the classify's sums for the scan (8 bytes per
+  // row block of a plane, less than a byte a slot); the region keeps 8 bytes a
+  // slot, so that what a given scratch size admits does not change
   L.slots = take(p.nslots * 8);
   L.slot_q = L.slots + p.nslots * sizeof(uint32_t) + 16;
+  L.part = align256(L.slot_q + p.nslots * sizeof(uint16_t));
   L.gmap = take(p.nsegs * (p.cap / 16) * sizeof(uint32_t));
   L.coords = take(p.ncoord * sizeof(float));
   L.total = off;
@@ -420,6 +427,7 @@ int ensure_scratch(mdmc_ctx *ctx, const Plan &p) {
   s.totals = reinterpret_cast<Totals *>(b + o_totals);
   s.slots = reinterpret_cast<uint32_t *>(b + o_slots);
   s.slot_q = reinterpret_cast<uint16_t *>(b + lay.slot_q);
+  s.part = reinterpret_cast<uint2 *>(b + lay.part);
   s.gmap = reinterpret_cast<uint32_t *>(b + o_gmap);
   s.coords = reinterpret_cast<float *>(b + o_coords);
   ctx->s = s;
@@ -472,10 +480,15 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   ca.slots = s.slots;
   ca.slot_q = s.slot_q;
   ca.gmap = s.gmap;
-  ca.scan_state = s.scan_state;
-  ca.scan_state_words = p.ntiles * 4;
-  ca.seg_pad = s.seg_counts + p.nsegs;
-  ca.seg_pad_n = (uint32_t)((uint64_t)p.ntiles * kScanTile - p.nsegs);
+  if (p.scan_planes) {
+    ca.part = s.part;
+    ca.NRB = p.NRBp;
+  } else {  // what the look-back scan starts from
+    ca.scan_state = s.scan_state;
+    ca.scan_state_words = p.ntiles * 4;
+    ca.seg_pad = s.seg_counts + p.nsegs;
+    ca.seg_pad_n = (uint32_t)((uint64_t)p.ntiles * kScanTile - p.nsegs);
+  }
   ca.scan_ticket = s.ticket;
   ca.totals = s.totals;
   ca.counts_out = reinterpret_cast<uint32_t *>(d_counts);
@@ -514,7 +527,12 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   }
   {
     ProfScope ps(ctx, 1, st);
-    hipLaunchKernelGGL(k_scan, dim3(p.ntiles), dim3(kScanThreads), 0, st, sa);
+    if (p.scan_planes) {
+      const PlaneScanArgs pa{sa, s.part, p.XT * p.cy, p.XT * p.NRBp, p.scan_planes};
+      hipLaunchKernelGGL(k_scan_planes, dim3((p.cz + p.scan_planes - 1) / p.scan_planes), dim3(kScanThreads), 0, st, pa);
+    } else {
+      hipLaunchKernelGGL(k_scan, dim3(p.ntiles), dim3(kScanThreads), 0, st, sa);
+    }
   }
   HIP_TRY(hipGetLastError());
   return MDMC_OK;

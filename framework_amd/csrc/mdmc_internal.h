@@ -22,6 +22,7 @@ struct Plan {
   uint32_t ptR, ptKP;        // plane tiles: cell rows, cell planes
   uint32_t band, NKBp, NRBp; // plane tiles: columns per group, plane blocks, row blocks
   uint64_t pt_blocks;        // plane-tile grid
+  uint32_t scan_planes;      // cell planes per workgroup of the plane scan (0: look-back scan)
 };
 
 struct Scratch {
@@ -34,6 +35,7 @@ struct Scratch {
   Totals *totals;
   uint32_t *slots;
   uint16_t *slot_q;
+  uint2 *part;
   uint32_t *gmap;
   float *coords;
 };

@@ -206,6 +206,8 @@ struct ClassifyArgs {
                           // first active cell << 16; written for non-empty groups
   unsigned long long *scan_state;  // zeroed here for k_scan
   uint32_t scan_state_words;
+  uint2 *part;            // per plane, row block and x-tile: the sums of its segments' totals
+                          // {active | quads << 16, vertices | non-empty << 16} (null: not wanted)
   uint2 *seg_pad;         // segment totals past the last segment, up to a whole scan tile
   uint32_t seg_pad_n;     // (zeroed here, read by the scan)
   uint32_t *scan_ticket;  // the ticket region, zeroed here
@@ -647,6 +649,19 @@ __device__ __forceinline__ void store_row_counts(const ClassifyArgs &a, uint32_t
     const uint32_t y = j0 + r, z = k + cp;
     const uint2 c = sh.cnt[m], c2 = TWO ? sh.cnt2[m] : make_uint2(0u, 0u);
     if (y < a.g.cy && z < a.g.cz) a.seg_counts[xt + a.XT * (y + a.g.cy * z)] = make_uint2(c.x + c2.x, c.y + c2.y);
+  }
+  // their sums per plane, for the scan (by another wave; rows past the grid
+  // have no counts)
+  const uint32_t cp = threadIdx.x - (uint32_t)kWave;
+  if (a.part != nullptr && cp < (uint32_t)KP && k + cp < a.g.cz) {
+    uint2 sum = make_uint2(0u, 0u);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint2 c = sh.cnt[cp * R + r], c2 = TWO ? sh.cnt2[cp * R + r] : make_uint2(0u, 0u);
+      sum.x += c.x + c2.x;
+      sum.y += c.y + c2.y + (((c.x + c2.x) & 0xFFFFu) != 0u ? 1u << 16 : 0u);
+    }
+    a.part[((size_t)(k + cp) * a.NRB + j0 / R) * a.XT + xt] = sum;
   }
 }
 
@@ -1311,6 +1326,139 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(ScanArgs a) {
     tot.num_chunks = (pa + 63u) >> 6;
     tot.pad0 = tot.pad1 = tot.pad2 = 0;
     *a.totals = tot;
+    if (pe <= a.nsegs) a.ne[pe] = make_uint2(a.nsegs, pa); else bad = true;
+    if (a.counts_out) {
+      a.counts_out[0] = pa;
+      a.counts_out[1] = pv;
+      a.counts_out[2] = pq;
+    }
+  }
+  if (bad && a.counts_out) atomicOr(a.counts_out + 3, kStatusInternal);
+  if (a.fill_coords) coords_fill(a.co, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+
+// The scan of a small or medium single volume, without look-back: a workgroup
+// takes whole cell planes of at most kPlaneScanSegs segments and finds what
+// precedes them by summing the sums the classify left per plane, row block and
+// x-tile (1/7 of the totals, contiguous in scan order), so that no workgroup
+// waits for another: a look-back's hops between the XCDs' caches cost more
+// than reading them.  HIP events around the scan: 64^3 10.0 -> 6.7 us, 128^3
+// 10.2 -> 7.4, 256^3 9.9 -> 9.1, 384^3 12.0 -> 10.5.  The reading grows with
+// the square of the sums: at 512^3 (37,000 sums) it costs what the look-back
+// does, so kPlaneScanParts ends there.
+constexpr uint32_t kPlaneScanSegs = kScanTile;
+constexpr uint32_t kPlaneScanParts = 1u << 15;
+
+struct PlaneScanArgs {
+  ScanArgs s;           // (state and ticket unused)
+  const uint2 *part;
+  uint32_t plane_segs;  // segments per cell plane
+  uint32_t plane_parts; // sums per cell plane
+  uint32_t planes;      // cell planes per workgroup
+};
+
+__global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
+  constexpr int kWaves = kScanThreads / kWave;
+  __shared__ uint4 s_before[kWaves], s_wave[kWaves];
+  const ScanArgs &a = p.s;
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const uint32_t first = blockIdx.x * p.planes * p.plane_segs;
+  const uint32_t end = min(first + p.planes * p.plane_segs, a.nsegs);
+  const uint32_t base = first + tid * kScanIpt;
+  // this thread's segments (the totals array is padded to whole tiles)
+  uint2 c[kScanIpt];
+  {
+    typedef uint32_t Word4 __attribute__((ext_vector_type(4), aligned(8)));
+    const Word4 *src = reinterpret_cast<const Word4 *>(a.seg_counts + (base < end ? base : first));
+#pragma unroll
+    for (int i = 0; i < kScanIpt / 2; ++i) {
+      const Word4 w = src[i];
+      c[2 * i] = base + 2 * i < end ? make_uint2(w.x, w.y) : make_uint2(0u, 0u);
+      c[2 * i + 1] = base + 2 * i + 1 < end ? make_uint2(w.z, w.w) : make_uint2(0u, 0u);
+    }
+  }
+  // sums of everything before the workgroup's planes
+  const uint32_t nbefore = blockIdx.x * p.planes * p.plane_parts;
+  uint4 bef = make_uint4(0, 0, 0, 0);
+  const uint4 *parts2 = reinterpret_cast<const uint4 *>(p.part);
+#pragma unroll 8
+  for (uint32_t i = tid; i < nbefore / 2u; i += kScanThreads) {
+    const uint4 q = parts2[i];
+    bef.x += (q.x & 0xFFFFu) + (q.z & 0xFFFFu);
+    bef.y += (q.y & 0xFFFFu) + (q.w & 0xFFFFu);
+    bef.z += (q.x >> 16) + (q.z >> 16);
+    bef.w += (q.y >> 16) + (q.w >> 16);
+  }
+  if ((nbefore & 1u) && tid == 0) {
+    const uint2 q = p.part[nbefore - 1u];
+    bef.x += q.x & 0xFFFFu;
+    bef.y += q.y & 0xFFFFu;
+    bef.z += q.x >> 16;
+    bef.w += q.y >> 16;
+  }
+  uint4 sum = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < kScanIpt; ++i) {
+    sum.x += c[i].x & 0xFFFFu;
+    sum.y += c[i].y;
+    sum.z += c[i].x >> 16;
+    sum.w += (c[i].x & 0xFFFFu) ? 1u : 0u;
+  }
+  const uint4 inc = make_uint4(wave_incl_scan_dpp(sum.x), wave_incl_scan_dpp(sum.y), wave_incl_scan_dpp(sum.z),
+                               wave_incl_scan_dpp(sum.w));
+  const uint4 binc = make_uint4(wave_incl_scan_dpp(bef.x), wave_incl_scan_dpp(bef.y), wave_incl_scan_dpp(bef.z),
+                                wave_incl_scan_dpp(bef.w));
+  if (lane == kWave - 1) {
+    s_wave[wave] = inc;
+    s_before[wave] = binc;
+  }
+  __syncthreads();
+  uint32_t pa = inc.x - sum.x, pv = inc.y - sum.y, pq = inc.z - sum.z, pe = inc.w - sum.w;
+  uint64_t tot_v = 0, tot_q = 0;  // a total past 2^32 - 1 is reported
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint4 v = s_wave[w], b = s_before[w];
+    pa += b.x;
+    pv += b.y;
+    pq += b.z;
+    pe += b.w;
+    tot_v += (uint64_t)b.y + v.y;
+    tot_q += (uint64_t)b.z + v.z;
+    if ((uint32_t)w < wave) {
+      pa += v.x;
+      pv += v.y;
+      pq += v.z;
+      pe += v.w;
+    }
+  }
+  if (tid == 0 && ((tot_v | tot_q) >> 32) != 0u && a.counts_out) atomicOr(a.counts_out + 3, kStatusIndexRange);
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < kScanIpt; ++i) {
+    const uint32_t sg = base + i, n = c[i].x & 0xFFFFu;
+    if (sg < end) a.seg_vq[sg] = make_uint2(pv, pq);
+    if (n) {
+      if (pe < a.nsegs) a.ne[pe] = make_uint2(sg, pa); else bad = true;
+      for (uint32_t gch = (pa + 63u) >> 6; (gch << 6) < pa + n; ++gch) {
+        if (gch < a.max_chunks) a.chunk_ne[gch] = pe; else bad = true;
+      }
+      ++pe;
+    }
+    pa += n;
+    pv += c[i].y;
+    pq += c[i].x >> 16;
+  }
+  if (end == a.nsegs && tid == kScanThreads - 1) {
+    // pa/pv/pq/pe now hold the grand totals
+    Totals tot;
+    tot.num_active = pa;
+    tot.num_vertices = pv;
+    tot.num_quads = pq;
+    tot.num_nonempty = pe;
+    tot.num_chunks = (pa + 63u) >> 6;
+    tot.pad0 = tot.pad1 = tot.pad2 = 0;
+    *a.totals = tot;
+    a.seg_vq[a.nsegs] = make_uint2(pv, pq);
     if (pe <= a.nsegs) a.ne[pe] = make_uint2(a.nsegs, pa); else bad = true;
     if (a.counts_out) {
       a.counts_out[0] = pa;
