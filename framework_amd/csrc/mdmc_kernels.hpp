@@ -2004,6 +2004,14 @@ __global__ void k_zero_tickets(uint32_t *t) { zero_tickets(t, threadIdx.x); }
 // k_reaverage recomputes iso vertices from the stored edge points (reading
 // edge points only), so neither reads what it writes.
 //
+// Each pass rewrites every other vertex of the mesh, so it moves all of its
+// lines twice: on 3.4 M cells (256x240x272 gyroid) k_smooth has 240 MB to move
+// (52 us at a large copy's rate) and takes 84 us with its vector units 90%
+// busy (92 us with two differences, products and a root per corner instead of
+// per edge and integer divisions for the position); k_reaverage has 200 MB
+// (43 us) and takes 68 us, bound by its chain of lookups (83 us with a gather
+// for each of the 12 edges, a third of the address units' work for nothing).
+//
 // The split of a convex ring is at the corner of the largest angle, taken as
 // the smallest cosine (a.b) / (sqrt(a.a) sqrt(b.b)) with IEEE sqrt and
 // division, first smallest wins (the reference takes acosf of rsqrtf-
@@ -2029,17 +2037,17 @@ __device__ __forceinline__ CellPos cell_pos(const EmitArgs &a, const EmitVol &vo
   c.cfg = rec_cfg(rec);
   c.lut2 = rec_lut2(rec);
   const uint32_t sl = s - vol.seg_off;
-  const uint32_t xt = sl % vol.XT, row = sl / vol.XT;
-  c.j = row % vol.g.cy;
-  c.k = row / vol.g.cy;
+  const uint32_t row = div_by(sl, vol.div_xt), xt = sl - row * vol.XT;
+  c.k = div_by(row, vol.div_cy);
+  c.j = row - c.k * vol.g.cy;
   c.x = xt * a.cap + c.xl;
   const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
   uint32_t s0u = s0;
   asm volatile("" : "+s"(s0u));
-  const uint32_t row0 = (s0u - vol.seg_off) / vol.XT;
+  const uint32_t row0 = div_by(s0u - vol.seg_off, vol.div_xt), k0 = div_by(row0, vol.div_cy);
   uint2 vq = const_u2(a.seg_vq, s0u);
   uint32_t nact = const_u2x(a.seg_counts, s0u) & 0xFFFFu;
-  float y1 = as_const(vol.yt_c)[row0 % vol.g.cy + 1u], z1 = as_const(vol.zt_c)[row0 / vol.g.cy + 1u];
+  float y1 = as_const(vol.yt_c)[row0 - k0 * vol.g.cy + 1u], z1 = as_const(vol.zt_c)[k0 + 1u];
   if (s != s0) {
     vq = a.seg_vq[s];
     nact = a.seg_counts[s].x & 0xFFFFu;
@@ -2053,12 +2061,6 @@ __device__ __forceinline__ CellPos cell_pos(const EmitArgs &a, const EmitVol &vo
   c.vb = vq.x + rec_lvb(rec) - vol.vbase;
   c.qb = vq.y + a.slot_q[(size_t)s * a.cap + rank] - vol.qbase;
   return c;
-}
-
-// the same from a copy of c_cfg_info in LDS
-__device__ __forceinline__ uint32_t iso_count_lds(const uint16_t *s_info, uint32_t cfg, uint32_t lut2) {
-  const uint32_t info = s_info[cfg];
-  return lut2 ? ((info >> 3) & 7u) : (info & 7u);
 }
 
 __device__ __forceinline__ uint32_t iso_count(uint32_t cfg, uint32_t lut2) {
@@ -2076,18 +2078,6 @@ struct P2 {
   float x, y;
 };
 
-// calc_cross_z_sign (dmc.cu:1741-1747)
-__device__ __forceinline__ bool cross_nonneg(P2 l, P2 m, P2 r) {
-  const float dx1 = r.x - m.x, dy1 = r.y - m.y, dx2 = l.x - m.x, dy2 = l.y - m.y;
-  return dx1 * dy2 - dx2 * dy1 >= 0.0f;
-}
-
-__device__ __forceinline__ float corner_cos(P2 l, P2 m, P2 r) {
-  const float ax = l.x - m.x, ay = l.y - m.y, bx = r.x - m.x, by = r.y - m.y;
-  const float num = ax * bx + ay * by;
-  return num / (sqrtf(ax * ax + ay * ay) * sqrtf(bx * bx + by * by));
-}
-
 // is_inside_triangle (dmc.cu:1894-1912)
 __device__ __forceinline__ bool inside_tri(P2 p0, P2 p1, P2 p2, P2 t, float &al, float &be, float &ga) {
   const float v0x = p1.x - p0.x, v0y = p1.y - p0.y, v1x = p2.x - p0.x, v1y = p2.y - p0.y;
@@ -2098,7 +2088,10 @@ __device__ __forceinline__ bool inside_tri(P2 p0, P2 p1, P2 p2, P2 t, float &al,
   be = (d11 * d20 - d10 * d21) * inv;
   ga = (d00 * d21 - d10 * d20) * inv;
   al = 1.0f - be - ga;
-  return (-1e-4 < (double)be) && (-1e-4 < (double)ga) && ((double)(be + ga) < 1.0 + 1e-4);
+  // The reference compares with the doubles -1e-4 and 1 + 1e-4.  Both lie just
+  // below the float nearest to them, so these comparisons decide alike.
+  static_assert((double)-1e-4f > -1e-4 && (double)1.0001f > 1.0 + 1e-4, "float thresholds");
+  return be >= -1e-4f && ga >= -1e-4f && be + ga < 1.0001f;
 }
 
 // v[t] for t in 0..3 by selects (no indexed register array)
@@ -2185,22 +2178,35 @@ __device__ __forceinline__ void smooth_chunk(const EmitArgs &a, const EmitVol &v
       P[p].y = l == 0u ? vy[p] : vz[p];
     }
     if (bad) { atomicOr(vol.status, kStatusInternal); continue; }
+    // Edge vectors E_p = P_p+1 - P_p.  With a = P_p-1 - P_p = -E_p-1 and b = E_p
+    // the reference's cross product (calc_cross_z_sign, dmc.cu:1741-1747) and
+    // dot product at corner p come out of E_p-1 and E_p up to signs, which
+    // change no rounding, and each length serves two corners: 8 differences
+    // and 4 square roots instead of 32 and 8.
+    P2 E[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) E[p] = P2{P[(p + 1) & 3].x - P[p].x, P[(p + 1) & 3].y - P[p].y};
     // calc_quadrilateral_signs (dmc.cu:1749-1780)
     uint32_t npos = 0, ipos = 0, ineg = 0;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-      if (cross_nonneg(P[(p + 3) & 3], P[p], P[(p + 1) & 3])) { ++npos; ipos = p; }
+      const P2 e = E[p], f = E[(p + 3) & 3];
+      if (f.x * e.y - e.x * f.y >= 0.0f) { ++npos; ipos = p; }
       else ineg = p;
     }
     if (npos == 2) continue;  // self-crossing ring (dmc.cu:1783-1786)
     uint32_t s0;
     if (npos == 0 || npos == 4) {
-      float best = corner_cos(P[3], P[0], P[1]);
+      // (the smallest cosine is the largest of f.e / (|f| |e|))
+      float len[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) len[p] = sqrtf(E[p].x * E[p].x + E[p].y * E[p].y);
+      float best = (E[3].x * E[0].x + E[3].y * E[0].y) / (len[3] * len[0]);
       s0 = 0;
 #pragma unroll
       for (int p = 1; p < 4; ++p) {
-        const float cs = corner_cos(P[(p + 3) & 3], P[p], P[(p + 1) & 3]);
-        if (cs < best) { best = cs; s0 = p; }
+        const float c = (E[p - 1].x * E[p].x + E[p - 1].y * E[p].y) / (len[p - 1] * len[p]);
+        if (c > best) { best = c; s0 = p; }
       }
     } else {
       s0 = npos < 2 ? ipos : ineg;  // the concave corner
@@ -2216,13 +2222,13 @@ __device__ __forceinline__ void smooth_chunk(const EmitArgs &a, const EmitVol &v
     } else {
       continue;
     }
-    float *E = vol.verts + 3ull * e_vtx;
+    float *out = vol.verts + 3ull * e_vtx;
     const float r0 = al * sel4(ta, vx) + be * sel4(tb, vx) + ga * sel4(tc, vx);
     const float r1 = al * sel4(ta, vy) + be * sel4(tb, vy) + ga * sel4(tc, vy);
     const float r2 = al * sel4(ta, vz) + be * sel4(tb, vz) + ga * sel4(tc, vz);
-    E[0] = r0;
-    E[1] = r1;
-    E[2] = r2;
+    out[0] = r0;
+    out[1] = r1;
+    out[2] = r2;
   }
 }
 
@@ -2233,7 +2239,7 @@ __device__ __forceinline__ void smooth_chunk(const EmitArgs &a, const EmitVol &v
 // group from -0.0 and divided by the count; groups with no point keep their
 // value.
 __device__ __forceinline__ void reaverage_cell(const EmitArgs &a, const EmitVol &vol, uint32_t s, uint32_t rank,
-                                               const uint64_t *s_lab, const uint16_t *s_info, float *s_acc) {
+                                               const uint64_t *s_lab, uint32_t *s_idx) {
   uint32_t rec;
   const CellPos c = cell_pos(a, vol, s, rank, rec);
   const FieldDesc &g = vol.g;
@@ -2242,19 +2248,19 @@ __device__ __forceinline__ void reaverage_cell(const EmitArgs &a, const EmitVol 
     atomicOr(vol.status, kStatusInternal);
     return;
   }
+  const uint32_t *const s_lab32 = reinterpret_cast<const uint32_t *>(s_lab);
   const uint64_t labels = s_lab[c.lut2 * 256 + c.cfg];
-  const uint32_t niso = iso_count_lds(s_info, c.cfg, c.lut2);
-  // owner cell (7 = this cell) and the owner's edge shift (0: e6, 1: e9, 2: e10)
-  constexpr uint8_t OWN_N[12] = {5, 2, 2, 4, 3, 1, 7, 0, 1, 7, 7, 0};
-  constexpr uint8_t OWN_L[12] = {2, 1, 2, 1, 0, 0, 0, 0, 2, 1, 2, 1};
-  constexpr uint8_t NEED[12] = {6, 4, 4, 5, 3, 2, 0, 1, 2, 0, 0, 1};  // bit 0: x>0, 1: y>0, 2: z>0
-  const uint32_t have = (c.x > 0 ? 1u : 0u) | (c.j > 0 ? 2u : 0u) | (c.k > 0 ? 4u : 0u);
+  const uint32_t lab_hi = (uint32_t)(labels >> 32), niso = (lab_hi >> 16) & 0xFu;
+  // crossed edges whose owner is in the grid, as in the emit
+  uint32_t use = lab_hi >> 20;
+  if (c.x == 0u) use &= ~0x898u;
+  if (c.j == 0u) use &= ~0x131u;
+  if (c.k == 0u) use &= ~0x00Fu;
+  // owner n's edges: 0: 7, 11; 1: 5, 8; 2: 1, 2; 3: 4; 4: 3; 5: 0
+  constexpr uint32_t OWNED[6] = {0x880u, 0x120u, 0x006u, 0x010u, 0x008u, 0x001u};
   uint32_t need = 0;
 #pragma unroll
-  for (int e = 0; e < 12; ++e) {
-    const uint32_t lab = (uint32_t)(labels >> (4 * e)) & 0xFu;
-    if (lab != 0xFu && (NEED[e] & have) == NEED[e] && OWN_N[e] < 7) need |= 1u << OWN_N[e];
-  }
+  for (int n = 0; n < 6; ++n) need |= (use & OWNED[n]) ? 1u << n : 0u;
   // Owners 1 (0,-1,0), 2 (0,0,-1) and 5 (0,-1,-1) are found through their
   // segments' group maps.  An owner needed here contains a crossing edge, so
   // it is active, and so are the other cells around that edge: owners 0
@@ -2299,76 +2305,92 @@ __device__ __forceinline__ void reaverage_cell(const EmitArgs &a, const EmitVol 
     }
   }
   const uint32_t nx[6] = {xlm, c.xl, c.xl, xlm, xlm, c.xl};
-  uint32_t own_base[8], own_bip[8];  // first edge point of each owner, its bipolar bits
+  // Each edge's point (its owner's first edge point and the owner's crossed
+  // edges before it) in column e of the lane's part of LDS.
+  constexpr uint32_t T = kEmitThreads;
+  constexpr int kOwnerEdges[7][3] = {{7, 11, -1}, {5, -1, 8}, {-1, 1, 2}, {4, -1, -1}, {-1, 3, -1}, {-1, -1, 0}, {6, 9, 10}};
   bool ok = true;
+  auto put = [&](int n, uint32_t first, uint32_t bip) {
+    const uint32_t i1 = first + (bip & 1u), i2 = i1 + ((bip >> 1) & 1u);
+    const uint32_t at[3] = {first, i1, i2};
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const int e = kOwnerEdges[n][l];
+      if (e < 0) continue;
+      s_idx[e * T] = at[l];
+      // (a point its owner does not have, or past the capacity, is left out)
+      if (((use >> e) & 1u) && (!((bip >> l) & 1u) || (uint64_t)at[l] >= vol.vcap)) {
+        ok = false;
+        use &= ~(1u << e);
+      }
+    }
+  };
+  uint32_t m[6];  // (all six in flight before the first is used)
+  bool ok_r[6];
 #pragma unroll
   for (int n = 0; n < 6; ++n) {
-    const bool use = (need >> n) & 1u;
-    const bool ok_r = use && inmask[n] && nr[n] < cap;
-    const uint32_t m = a.slots[(size_t)(ok_r ? ns[n] : s) * cap + (ok_r ? nr[n] : rank)];
-    if (use && !(ok_r && rec_x(m) == nx[n])) ok = false;
-    own_base[n] = vq0[n] + rec_lvb(m) - vol.vbase + iso_count_lds(s_info, rec_cfg(m), rec_lut2(m));
-    own_bip[n] = owned_bipolar(rec_cfg(m));
+    const bool used = (need >> n) & 1u;
+    ok_r[n] = used && inmask[n] && nr[n] < cap;
+    m[n] = a.slots[(size_t)(ok_r[n] ? ns[n] : s) * cap + (ok_r[n] ? nr[n] : rank)];
+    if (used && !ok_r[n]) ok = false;
   }
-  own_base[6] = 0;
-  own_bip[6] = 0;
-  own_base[7] = c.vb + niso;
-  own_bip[7] = owned_bipolar(c.cfg);
-  constexpr uint32_t T = kEmitThreads;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if ((uint32_t)q < niso) {
-      s_acc[(3 * q + 0) * T] = -0.0f;
-      s_acc[(3 * q + 1) * T] = -0.0f;
-      s_acc[(3 * q + 2) * T] = -0.0f;
-    }
+  for (int n = 0; n < 6; ++n) {
+    if (ok_r[n] && rec_x(m[n]) != nx[n]) ok = false;
+    const uint32_t miso = (s_lab32[2u * ((m[n] >> 10) & 0x1FFu) + 1u] >> 16) & 0xFu;
+    put(n, vq0[n] + rec_lvb(m[n]) - vol.vbase + miso, owned_bipolar(rec_cfg(m[n])));
   }
+  put(6, c.vb + niso, owned_bipolar(c.cfg));
   if ((uint64_t)c.vb + niso > vol.vcap) { atomicOr(vol.status, kStatusVertexOverflow); return; }
-  // every edge point's index first, then all the loads (vertex 0, which
-  // exists, for edges that do not contribute), then the sums in edge order:
-  // the loads are in flight together instead of one edge at a time
-  uint32_t use = 0, pidx[12];
+  // The points are gathered three of a lane's own edges at a time, in edge
+  // order: a cell crosses 4 of the 12 on average and the most of 64 lanes is
+  // 5 to 6, so two rounds (a gather costs its 64 lanes' addresses whether or
+  // not they contribute; a load the lane does not need reads vertex 0).
+  Float3 *const out = reinterpret_cast<Float3 *>(vol.verts + 3ull * c.vb);
+  auto walk = [&](auto add) {
+    for (uint32_t left = use; left != 0u;) {
+      const uint32_t l1 = left & (left - 1u), l2 = l1 & (l1 - 1u);
+      const uint32_t e0 = (uint32_t)__builtin_ctz(left), e1 = l1 ? (uint32_t)__builtin_ctz(l1) : 12u;
+      const uint32_t e2 = l2 ? (uint32_t)__builtin_ctz(l2) : 12u;
+      const uint32_t i0 = s_idx[e0 * T], i1 = s_idx[e1 * T], i2 = s_idx[e2 * T];
+      const Float3 *const pts = reinterpret_cast<const Float3 *>(vol.verts);
+      const Float3 p0 = pts[i0], p1 = pts[i1], p2 = pts[i2];
+      add(e0, p0);
+      if (l1) add(e1, p1);
+      if (l2) add(e2, p2);
+      left = l2 & (l2 - 1u);
+    }
+  };
+  s_idx[12 * T] = 0u;
+  if (__ballot(niso != 1u) == 0ull) {
+    const uint32_t n = (uint32_t)__popc(use);
+    float sx = -0.0f, sy = -0.0f, sz = -0.0f;
+    walk([&](uint32_t, const Float3 &p) {
+      sx = sx + p.x;
+      sy = sy + p.y;
+      sz = sz + p.z;
+    });
+    const float d = (float)n;
+    if (n) *out = Float3{sx / d, sy / d, sz / d};
+  } else {
+    float sx[4] = {-0.0f, -0.0f, -0.0f, -0.0f}, sy[4] = {-0.0f, -0.0f, -0.0f, -0.0f}, sz[4] = {-0.0f, -0.0f, -0.0f, -0.0f};
+    uint32_t cnt = 0;  // 8 bits per group
+    walk([&](uint32_t e, const Float3 &p) {
+      const uint32_t lab = (uint32_t)(labels >> (4u * e)) & 0xFu;
+      cnt += 1u << (8u * lab);
 #pragma unroll
-  for (int e = 0; e < 12; ++e) {
-    pidx[e] = 0;
-    const uint32_t lab = (uint32_t)(labels >> (4 * e)) & 0xFu;
-    if (lab == 0xFu || (NEED[e] & have) != NEED[e]) continue;
-    const uint32_t on = OWN_N[e], ol = OWN_L[e];
-    if (!((own_bip[on] >> ol) & 1u)) { ok = false; continue; }
-    const uint32_t idx = own_base[on] + (uint32_t)__popc(own_bip[on] & ((1u << ol) - 1u));
-    if ((uint64_t)idx >= vol.vcap) { ok = false; continue; }
-    pidx[e] = idx;
-    use |= 1u << e;
-  }
-  float px[12], py[12], pz[12];
+      for (int q = 0; q < 4; ++q) {
+        sx[q] = lab == (uint32_t)q ? sx[q] + p.x : sx[q];
+        sy[q] = lab == (uint32_t)q ? sy[q] + p.y : sy[q];
+        sz[q] = lab == (uint32_t)q ? sz[q] + p.z : sz[q];
+      }
+    });
 #pragma unroll
-  for (int e = 0; e < 12; ++e) {
-    const float *pnt = vol.verts + 3ull * pidx[e];
-    px[e] = pnt[0];
-    py[e] = pnt[1];
-    pz[e] = pnt[2];
-  }
-  uint32_t cnt = 0;
-#pragma unroll
-  for (int e = 0; e < 12; ++e) {
-    if (!((use >> e) & 1u)) continue;
-    const uint32_t lab = (uint32_t)(labels >> (4 * e)) & 0xFu;
-    float *acc = s_acc + 3 * lab * T;
-    acc[0] = acc[0] + px[e];
-    acc[T] = acc[T] + py[e];
-    acc[2 * T] = acc[2 * T] + pz[e];
-    cnt += 1u << (8 * lab);
-  }
-  float *out = vol.verts + 3ull * c.vb;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if ((uint32_t)q < niso) {
-      const uint32_t n = (cnt >> (8 * q)) & 0xFFu;
-      if (n) {
+    for (int q = 0; q < 4; ++q) {
+      if ((uint32_t)q < niso) {
+        const uint32_t n = (cnt >> (8 * q)) & 0xFFu;
         const float d = (float)n;
-        out[3 * q + 0] = s_acc[(3 * q + 0) * T] / d;
-        out[3 * q + 1] = s_acc[(3 * q + 1) * T] / d;
-        out[3 * q + 2] = s_acc[(3 * q + 2) * T] / d;
+        if (n) out[q] = Float3{sx[q] / d, sy[q] / d, sz[q] / d};
       }
     }
   }
@@ -2390,13 +2412,11 @@ __global__ __launch_bounds__(kEmitThreads) void k_smooth(EmitArgs a) {
 
 __global__ __launch_bounds__(kEmitThreads) void k_reaverage(EmitArgs a) {
   __shared__ uint64_t s_lab[2 * 256];
-  __shared__ uint16_t s_info[256];  // c_cfg_info: seven lookups per cell
-  __shared__ float s_acc[12 * kEmitThreads];
+  __shared__ uint32_t s_idx[13 * kEmitThreads];
   const Totals tot = *a.totals;
   const uint32_t num_chunks = (uint32_t)min((uint64_t)tot.num_chunks, a.max_chunks);
   if (!workgroup_has_chunks(num_chunks)) return;  // (uniform: before the barrier)
-  for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = (&c_label[0][0])[i];
-  for (uint32_t i = threadIdx.x; i < 256; i += kEmitThreads) s_info[i] = c_cfg_info[i];
+  for (uint32_t i = threadIdx.x; i < 512; i += kEmitThreads) s_lab[i] = emit_label(i);
   __syncthreads();
   const uint32_t lane = lane_id(), wave = wave_id();
   const uint32_t num_ne = min(tot.num_nonempty, a.nsegs);
@@ -2404,7 +2424,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_reaverage(EmitArgs a) {
   for (uint32_t ch = it.next; ch < it.end; ch += it.step) {
     uint32_t s, rank;
     if (!locate_cell(a, tot, num_ne, ch, lane, s, rank)) continue;
-    reaverage_cell(a, a.v, s, rank, s_lab, s_info, s_acc + threadIdx.x);
+    reaverage_cell(a, a.v, s, rank, s_lab, s_idx + threadIdx.x);
   }
 }
 
