@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -272,6 +273,9 @@ struct mdmc_ctx {
   uint32_t batch_n = 0, batch_W4 = 0, batch_KP = 0, batch_tiles = 0;
   uint64_t batch_key = 0;
   mdmc::Plan batch_plan{};
+  // mdmc_counts_read: pinned words that k_publish writes, and its last number
+  uint32_t *pub = nullptr;
+  uint32_t pub_seq = 0;
   // batched field generation: pinned staging + device copy of GenVol table and
   // the per-axis tables
   void *gdev = nullptr;
@@ -1225,6 +1229,7 @@ void mdmc_ctx_destroy(mdmc_ctx *ctx) {
   if (ctx->bdev) (void)hipFree(ctx->bdev);
   if (ctx->gdev) (void)hipFree(ctx->gdev);
   if (ctx->ghost) (void)hipHostFree(ctx->ghost);
+  if (ctx->pub) (void)hipHostFree(ctx->pub);
   if (ctx->ghost_ev) (void)hipEventDestroy(ctx->ghost_ev);
   for (int i = 0; i < 2; ++i) {
     if (ctx->bhost[i]) (void)hipHostFree(ctx->bhost[i]);
@@ -1270,6 +1275,40 @@ int mdmc_emit_device(mdmc_ctx *ctx, const float *d_field, const float xyz_min[3]
   if (grc != MDMC_OK) return grc;
   return launch_emit(ctx, ctx->plan, d_field, ctx->iso, xyz_min, xyz_max, d_vertices, vertex_capacity,
                      d_quads, quad_capacity, d_counts, static_cast<hipStream_t>(stream));
+}
+
+int mdmc_counts_read(mdmc_ctx *ctx, const mdmc_counts *d_counts, uint32_t n, mdmc_counts *counts, void *stream) {
+  if (!ctx || !d_counts || !counts) return fail(MDMC_ERR_INVALID, "null argument");
+  if (n == 0 || n > kMaxBatch) return fail(MDMC_ERR_INVALID, "1..1024 counts can be read");
+  static_assert(sizeof(mdmc_counts) == 4 * sizeof(uint32_t), "counts are four words");
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const int grc = capture_guard(ctx, st);
+  if (grc != MDMC_OK) return grc;
+  if (ctx->capturing_now) return fail(MDMC_ERR_INVALID, "counts cannot be read under stream capture");
+  if (!ctx->pub) {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, (kPublishHead + 4u * kMaxBatch) * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(MDMC_ERR_NOMEM, "pinned counts allocation failed");
+    }
+    ctx->pub = static_cast<uint32_t *>(p);
+    ctx->pub[0] = 0;
+  }
+  const uint32_t seq = ++ctx->pub_seq;
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(256), 0, st, reinterpret_cast<const uint32_t *>(d_counts), 4u * n, ctx->pub,
+                     seq);
+  HIP_TRY(hipGetLastError());
+  // watched for as long as small and medium extractions take; then the
+  // stream's own wait, which also reports what went wrong on it
+  const auto give_up = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+  bool there = false;
+  for (uint32_t i = 1; !(there = __atomic_load_n(ctx->pub, __ATOMIC_ACQUIRE) == seq); ++i) {
+    if ((i & 63u) == 0u && std::chrono::steady_clock::now() > give_up) break;
+  }
+  if (!there) HIP_TRY(hipStreamSynchronize(st));
+  if (__atomic_load_n(ctx->pub, __ATOMIC_ACQUIRE) != seq) return fail(MDMC_ERR_HIP, "the counts did not arrive");
+  std::memcpy(counts, ctx->pub + kPublishHead, n * sizeof(mdmc_counts));
+  return MDMC_OK;
 }
 
 int mdmc_extract_device(mdmc_ctx *ctx, const float *d_field, const uint32_t dims[3],

@@ -970,6 +970,7 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
 // numbers are the global ones minus the prefix at its first segment.
 
 constexpr uint32_t kMaxBatch = 1024;  // volumes per batch call
+constexpr uint32_t kPublishHead = 16;  // words before the counts of k_publish
 
 // Exact division of 32-bit numbers by a divisor known on the host: a multiply
 // and two shifts (round-up multiplier 2^32 (2^l - d) / d + 1, l = ceil(log2 d);
@@ -2484,6 +2485,18 @@ __global__ __launch_bounds__(256) void k_batch_counts(BatchCountArgs b) {
     bv.counts[2] = v1.y - v0.y;
     bv.counts[3] = b.batch_counts[3];
   }
+}
+
+// Counts to pinned host memory, then the call's number in its first word: the
+// host, which watches that word, has them 2-3 us after the kernels before this
+// one end.  The stream's own completion and a copy out of device memory cost
+// it 15-20 us (one workgroup).
+__global__ __launch_bounds__(256) void k_publish(const uint32_t *src, uint32_t words, uint32_t *host, uint32_t seq) {
+  for (uint32_t i = threadIdx.x; i < words; i += 256u)
+    __hip_atomic_store(host + kPublishHead + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // After a batch emit: status bits the emit could only attribute to the batch

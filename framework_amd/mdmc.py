@@ -136,6 +136,8 @@ def lib():
     L.mdmc_count_device.restype = ctypes.c_int
     L.mdmc_emit_device.argtypes = [_VP, _VP, _F3, _F3, _VP, ctypes.c_uint64, _VP, ctypes.c_uint64, _VP, _VP]
     L.mdmc_emit_device.restype = ctypes.c_int
+    L.mdmc_counts_read.argtypes = [_VP, _VP, ctypes.c_uint32, _VP, _VP]
+    L.mdmc_counts_read.restype = ctypes.c_int
     L.mdmc_extract_device.argtypes = [_VP, _VP, _U3, _F3, _F3, ctypes.c_float, _VP, ctypes.c_uint64, _VP,
                                       ctypes.c_uint64, _VP, _VP]
     L.mdmc_extract_device.restype = ctypes.c_int
@@ -341,6 +343,13 @@ class Context:
         c = self._counts.cpu().numpy().view(np.uint32)
         return {"num_active": int(c[0]), "num_vertices": int(c[1]), "num_quads": int(c[2]), "status": int(c[3])}
 
+    def _wait_counts(self, counts, n, stream):
+        """Waits for the stream; the n counts as (n, 4) uint32 in host memory."""
+        c = np.empty((n, 4), dtype=np.uint32)
+        _check(lib().mdmc_counts_read(self._h, _VP(counts.data_ptr()), n, c.ctypes.data_as(_VP), self._stream(stream)),
+               "mdmc_counts_read")
+        return c
+
     def count(self, field, iso: float, counts=None, stream=None) -> None:
         if field.dtype != self._torch.float32 or not field.is_contiguous() or not field.is_cuda:
             raise ValueError("field must be a contiguous float32 CUDA tensor")
@@ -377,18 +386,16 @@ class Context:
         iterations).  Returns (vertices (V,3), quads (Q,4), counts)."""
         torch = self._torch
         self.count(field, iso, stream=stream)
-        (stream or torch.cuda.current_stream()).synchronize()
-        cnt = self.read_counts()
-        if cnt["status"]:
-            raise MDMCError(-7, f"count status {cnt['status']}")
-        V, Q = cnt["num_vertices"], cnt["num_quads"]
+        _, V, Q, status = self._wait_counts(self._counts, 1, stream)[0].tolist()
+        if status:
+            raise MDMCError(-7, f"count status {status}")
         verts = torch.empty((V, 3), dtype=torch.float32, device=field.device)
         quads = torch.empty((Q, 4), dtype=torch.int32, device=field.device)
         self.emit(field, verts, quads, xyz_min, xyz_max, stream=stream)
         if num_smooth:
             self.smooth(verts, quads, num_smooth, stream=stream)
-        (stream or torch.cuda.current_stream()).synchronize()
-        cnt = self.read_counts()
+        cnt = dict(zip(("num_active", "num_vertices", "num_quads", "status"),
+                       self._wait_counts(self._counts, 1, stream)[0].tolist()))
         if cnt["status"]:
             raise MDMCError(-7, f"emit status {cnt['status']}: " +
                             ", ".join(n for b, n in STATUS_NAMES.items() if cnt["status"] & b))
@@ -492,8 +499,7 @@ class Context:
             return []
         counts = self.batch_counts_tensor(n)
         self.batch_count(fields, isos, counts, stream=stream, _table=table)
-        (stream or torch.cuda.current_stream()).synchronize()
-        c = counts.cpu().numpy().view(np.uint32)
+        c = self._wait_counts(counts, n, stream)
         nv = c[:, 1].astype(np.int64)
         nq = c[:, 2].astype(np.int64)
         all_v = torch.empty((int(nv.sum()), 3), dtype=torch.float32, device="cuda")
@@ -505,8 +511,7 @@ class Context:
         table["quads"] = np.where(nq > 0, np.uint64(all_q.data_ptr()) + np.uint64(16) * qoff, 0)
         table["quad_capacity"] = nq
         self.batch_emit(fields, isos, None, counts, stream=stream, _table=table)
-        (stream or torch.cuda.current_stream()).synchronize()
-        c = counts.cpu().numpy().view(np.uint32)
+        c = self._wait_counts(counts, n, stream)
         bad = np.nonzero(c[:, 3])[0]
         if len(bad):
             raise MDMCError(-7, f"volume {int(bad[0])}: status {int(c[bad[0], 3])}")

@@ -200,6 +200,10 @@ int mdmc_emit_device(mdmc_ctx *ctx, const float *d_field, const float xyz_min[3]
                      int32_t *d_quads, uint64_t quad_capacity, mdmc_counts *d_counts,
                      void *stream);
 
+/* Waits for what `stream` holds so far and copies the n counts (n <= 1024) in
+ * device memory `d_counts` to `counts` in host memory.  Not under capture. */
+int mdmc_counts_read(mdmc_ctx *ctx, const mdmc_counts *d_counts, uint32_t n, mdmc_counts *counts, void *stream);
+
 /* mdmc_count_device followed by mdmc_emit_device. */
 int mdmc_extract_device(mdmc_ctx *ctx, const float *d_field, const uint32_t dims[3],
                         const float xyz_min[3], const float xyz_max[3], float iso,
