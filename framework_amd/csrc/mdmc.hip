@@ -216,14 +216,26 @@ int plan_tiling(const uint32_t dims[3], Plan *p, const int *opt) {
   p->band = band_opt > 0 && band_opt <= 64 ? (uint32_t)band_opt : 1u;
   p->NRBp = nrb;
   p->NKBp = (p->cz + p->ptKP - 1) / p->ptKP;
+  // Narrow last x-tiles (only the default shapes have kernels for them; every
+  // shape has one for rows of less than 4 points) are columns of their own.
+  p->tail = pt_tail(p->X, p->XT, p->cap);
+  if (p->tail != kPtTailTiny && (rows != pt_rows(W / 4) || p->ptKP != pt_planes(W / 4))) p->tail = kPtTailFull;
+  const uint32_t xt_full = p->tail == kPtTailFull ? p->XT : p->XT - 1u;
+  p->tall = pt_tall_when(p->tail, rows, p->ptKP, p->XT, (uint64_t)p->XT * nrb * p->NKBp) != kTallNever;
+  const uint32_t kp_tail = p->tall ? pt_tall(p->tail, rows, p->ptKP) : p->ptKP;
+  p->NKBt = (p->cz + kp_tail - 1) / kp_tail;
   // the scan by whole planes, if a workgroup holds one (a plane's segments and
   // the sums are 32-bit counts well within range)
   const uint64_t plane_segs = (uint64_t)p->XT * p->cy, parts = (uint64_t)p->XT * nrb * p->cz;
   p->scan_planes = !p->zmarch && plane_segs <= kPlaneScanSegs && parts <= kPlaneScanParts
                        ? (uint32_t)(kPlaneScanSegs / plane_segs) : 0u;
   // 8 XCDs, each at most ceil(NKB * groups / 8) group tiles of `band` columns
-  const uint64_t ng = ((uint64_t)p->XT * nrb + p->band - 1) / p->band;
-  p->pt_blocks = 8ull * p->band * (((uint64_t)p->NKBp * ng + 7) / 8);
+  auto blocks = [&](uint64_t cols, uint64_t nkb) {
+    const uint64_t ng = (cols + p->band - 1) / p->band;
+    return 8ull * p->band * ((nkb * ng + 7) / 8);
+  };
+  p->tail_block = blocks((uint64_t)xt_full * nrb, p->NKBp);
+  p->pt_blocks = p->tail_block + (p->tail == kPtTailFull ? 0 : blocks(nrb, p->NKBt));
   return MDMC_OK;
 }
 
@@ -500,8 +512,8 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   {
     ProfScope ps(ctx, 0, st);
     if (!p.zmarch) {
-      PtArgs pa{ca, p.band, p.NKBp, p.NRBp};
-      rc = launch_classify_pt(p.W, p.ptR, p.ptKP, pt_tail(p.X, p.XT, p.cap), pa, (uint32_t)p.pt_blocks, st);
+      PtArgs pa{ca, p.band, p.NKBp, p.NRBp, (uint32_t)p.tail_block, p.NKBt, p.tall};
+      rc = launch_classify_pt(p.W, p.ptR, p.ptKP, p.tail, pa, (uint32_t)p.pt_blocks, st);
     } else {
       rc = launch_classify(p.W, p.R, ca, (uint32_t)p.classify_blocks, st);
     }
@@ -753,7 +765,12 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
                      uint32_t *tiles_total) {
   const uint32_t cap = 256u * W4;
   uint32_t *const tiles0 = batch_tile_off(ctx->bhost[slot], n), *const segs0 = batch_seg_off(ctx->bhost[slot], n);
-  uint64_t seg_off = 0, tile_off = 0, cells = 0, coord_off = 0;
+  uint64_t seg_off = 0, tile_off = 0, cells = 0, coord_off = 0, tiles = 0;
+  for (uint32_t v = 0; v < n; ++v) {  // (tiles of KP planes)
+    const uint32_t *const d = vols[v].dims;
+    if (d[0] < 2 || d[1] < 2 || d[2] < 2) continue;
+    tiles += (uint64_t)((d[0] - 1 + cap - 1) / cap) * ((d[1] - 1 + kBatchRows - 1) / kBatchRows) * ((d[2] - 1 + KP - 1) / KP);
+  }
   for (uint32_t v = 0; v < n; ++v) {
     const mdmc_volume &mv = vols[v];
     BatchVol &b = ctx->bhost[slot][v];
@@ -763,7 +780,9 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     const uint32_t cx = empty ? 0 : X - 1, cy = empty ? 0 : Y - 1, cz = empty ? 0 : Z - 1;
     const uint32_t XT = empty ? 1 : (cx + cap - 1) / cap;
     const uint32_t NRB = empty ? 0 : (cy + kBatchRows - 1) / kBatchRows;
-    const uint32_t NKP = empty ? 0 : (cz + KP - 1) / KP;
+    const uint32_t tail = empty ? kPtTailFull : pt_tail(X, XT, cap);
+    const uint32_t tall = pt_tall_when(tail, kBatchRows, KP, XT, tiles), kp = tall == kTallAll ? pt_tall(tail, kBatchRows, KP) : KP;
+    const uint32_t NKP = empty ? 0 : (cz + kp - 1) / kp;
     const uint64_t nsegs = (uint64_t)XT * cy * cz;
     b.c.g = FieldDesc{mv.field, X, Y, Z, cx, cy, cz, mv.iso};
     b.c.XT = XT;
@@ -774,7 +793,8 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     b.tile_off = tiles0[v] = (uint32_t)tile_off;
     b.NRB = NRB;
     b.NKP = NKP;
-    b.tail = empty ? kPtTailFull : pt_tail(X, XT, cap);
+    b.tail = tail;
+    b.tall = tall;
     b.seg_off = segs0[v] = (uint32_t)seg_off;
     b.nsegs = (uint32_t)nsegs;
     b.mnx = mv.xyz_min[0];

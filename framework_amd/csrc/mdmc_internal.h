@@ -21,7 +21,9 @@ struct Plan {
   int zmarch;  // use the z-marching classify kernel
   uint32_t ptR, ptKP;        // plane tiles: cell rows, cell planes
   uint32_t band, NKBp, NRBp; // plane tiles: columns per group, plane blocks, row blocks
-  uint64_t pt_blocks;        // plane-tile grid
+  uint32_t tail;             // parts of the last x-tile (pt_tail); if narrow: its plane blocks,
+  uint32_t NKBt, tall;       // and whether they are tall
+  uint64_t pt_blocks, tail_block;  // plane-tile grid, first block of the narrow x-tiles
   uint32_t scan_planes;      // cell planes per workgroup of the plane scan (0: look-back scan)
 };
 

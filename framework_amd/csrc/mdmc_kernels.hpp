@@ -411,6 +411,13 @@ struct PtArgs {
   uint32_t B;    // columns per group
   uint32_t NKB;  // plane blocks
   uint32_t NRB;  // row blocks
+  // The last x-tiles, where they are narrow, are in the blocks from tail_block
+  // on (a multiple of 8) as columns of their own.  Among the others' columns
+  // they fell to the same XCDs throughout: with two x-tiles four XCDs got all
+  // the full ones (603x487x399: 129 us, 107 apart).
+  uint32_t tail_block;
+  uint32_t NKBT;  // their plane blocks
+  uint32_t tall;  // of pt_tall planes
 };
 
 // Cell rows per plane tile (R + 1 point rows, 2 per wave) and cell planes per
@@ -433,6 +440,28 @@ __host__ __device__ constexpr uint32_t pt_tail(uint32_t X, uint32_t XT, uint32_t
   if (np <= 128u) return kPtTail32;
   if (cap == 256u) return kPtTailFull;
   return np <= 256u ? kPtTail64 : np <= 320u ? kPtTail256_16 : np <= 384u ? kPtTail256_32 : kPtTailFull;
+}
+
+// Cell planes of a narrow last x-tile's workgroup where it takes more than KP of
+// them (a tall tile): as many as fill the LDS words and registers of a full
+// tile.  A narrow tile of KP planes holds a quarter of a full one's points or
+// less, but its loads, barriers and list rounds follow each other just as
+// slowly, and it keeps its place on the CU for half as long (256 volumes of 32
+// to 256 points a side: classify 701 us, with tall tiles 584).
+__host__ __device__ constexpr uint32_t pt_tall(uint32_t tail, uint32_t R, uint32_t KP) {
+  const bool narrow = tail == kPtTail16 || tail == kPtTail32 || tail == kPtTail64;
+  const uint32_t most = tail == kPtTail64 ? 4u : 8u;
+  return narrow && R == 7u && most >= KP ? most / KP * KP : KP;
+}
+// Narrow tiles are tall where rows have full x-tiles as well (in a batch, whose
+// tiles are in memory order, every pt_tall / KP-th plane block's narrow tile
+// works and the others leave: kTallSome), and where a row is one narrow tile
+// if enough tiles remain to fill the chip twice (kTallAll; 24 volumes of 32 to
+// 128 points, 4,000 tiles: 31.0 us tall or not).
+constexpr uint32_t kTallNever = 0u, kTallSome = 1u, kTallAll = 2u;
+constexpr uint64_t kTallTiles = 8192;  // of KP planes
+__host__ __device__ constexpr uint32_t pt_tall_when(uint32_t tail, uint32_t R, uint32_t KP, uint64_t XT, uint64_t tiles) {
+  return pt_tall(tail, R, KP) == KP ? kTallNever : XT > 1u ? kTallSome : tiles >= kTallTiles ? kTallAll : kTallNever;
 }
 
 template <int W4, int R, int KP>
@@ -955,12 +984,18 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
     zero_scan_state(a, threadIdx.x, kPtThreads);
     if (a.counts_out != nullptr && threadIdx.x < 4) a.counts_out[threadIdx.x] = 0u;
   }
-  const PtTile t = pt_tile_of(blockIdx.x, a.XT, pa.NRB, pa.NKB, pa.B);
+  constexpr uint32_t KPT = pt_tall(TAIL, R, KP);
   constexpr uint32_t CAP = 256u * W4;
-  if (TAIL != kPtTailFull && t.xt + 1u == a.XT)
-    classify_pt_parts<TAIL, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, sh, tab, true);
-  else if (TAIL != kPtTailTiny)
+  if (TAIL != kPtTailFull && blockIdx.x >= pa.tail_block) {
+    const PtTile t = pt_tile_of(blockIdx.x - pa.tail_block, 1u, pa.NRB, pa.NKBT, pa.B);
+    if (KPT != KP && pa.tall)
+      classify_pt_parts<TAIL, CAP, R, (int)KPT>(a, a.XT - 1u, t.kb * KPT, t.rb * R, s_w, sh, tab, true);
+    else
+      classify_pt_parts<TAIL, CAP, R, KP>(a, a.XT - 1u, t.kb * KP, t.rb * R, s_w, sh, tab, true);
+  } else if (TAIL != kPtTailTiny) {
+    const PtTile t = pt_tile_of(blockIdx.x, TAIL != kPtTailFull ? a.XT - 1u : a.XT, pa.NRB, pa.NKB, pa.B);
     classify_pt_parts<kPtTailFull, CAP, R, KP>(a, t.xt, t.kb * KP, t.rb * R, s_w, sh, tab, true);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1021,6 +1056,7 @@ struct BatchVol {
   ClassifyArgs c;         // per-volume field and tiling; record pointers start at seg_off
   EmitVol e;              // for the emit, except vbase and qbase (BatchEmitArgs.base)
   uint32_t NRB, NKP;      // row blocks and plane blocks of the volume
+  uint32_t tall;          // kTall*
   uint32_t tail;          // parts of the last x-tile (pt_tail)
   uint32_t tile_off;      // first flattened classify tile
   uint32_t seg_off, nsegs;
@@ -1096,10 +1132,20 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 =
     const uint32_t nrb = bv->NRB;
     const uint32_t local = t - bv->tile_off;
     const uint32_t xt = local % a.XT, u = local / a.XT;
-    __syncthreads();  // the previous tile's LDS words are no longer read
-    const uint32_t k = u / nrb * KP, j0 = u % nrb * R, tail = xt + 1u == a.XT ? bv->tail : kPtTailFull;
+    const uint32_t kb = u / nrb, k = kb * KP, j0 = (u - kb * nrb) * R;
+    const uint32_t tail = xt + 1u == a.XT ? bv->tail : kPtTailFull, tall = tail == kPtTailFull ? kTallNever : bv->tall;
     constexpr uint32_t CAP = 256u * W4;
-    if (W4 <= 2 && tail == kPtTail16)
+    const uint32_t kpt = pt_tall(tail, R, KP);
+    if (tall == kTallSome && kb % (kpt / KP) != 0u) continue;  // (uniform) another's planes
+    __syncthreads();  // the previous tile's LDS words are no longer read
+    const uint32_t kt = tall == kTallSome ? k : kb * kpt;
+    if (W4 <= 2 && tail == kPtTail16 && tall != kTallNever)
+      classify_pt_parts<kPtTail16, CAP, R, (int)pt_tall(kPtTail16, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
+    else if (W4 <= 2 && tail == kPtTail32 && tall != kTallNever)
+      classify_pt_parts<kPtTail32, CAP, R, (int)pt_tall(kPtTail32, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
+    else if (W4 == 2 && tail == kPtTail64 && tall != kTallNever)
+      classify_pt_parts<kPtTail64, CAP, R, (int)pt_tall(kPtTail64, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
+    else if (W4 <= 2 && tail == kPtTail16)
       classify_pt_parts<kPtTail16, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
     else if (W4 <= 2 && tail == kPtTail32)
       classify_pt_parts<kPtTail32, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);

@@ -63,3 +63,32 @@ def test_batch_of_row_widths(fa_mod, widths):
             (ref["num_active"], ref["num_vertices"], ref["num_quads"]), f.shape
         assert_same_mesh(v.cpu().numpy(), q.cpu().numpy(), ref)
     ctx.close()
+
+
+def _tall_field(X, Y, Z):
+    """Mostly empty: noise in a box in the middle and at the far corner."""
+    rng = np.random.default_rng(X)
+    f = np.ones((Z, Y, X), np.float32)
+    for k, j in ((Z // 2, Y // 2), (Z - 9, Y - 9)):
+        f[k:k + 10, j:j + 9, :] = rng.standard_normal(f[k:k + 10, j:j + 9, :].shape)
+    return f
+
+
+@pytest.mark.parametrize("shape", [(5, 645, 365), (64, 645, 362), (70, 645, 365), (128, 641, 367)])
+def test_narrow_rows_many_tiles(fa_mod, shape):
+    """Rows of one narrow x-tile in a grid of over 8192 tiles: tiles of 8 planes."""
+    import torch
+
+    ctx = fa_mod.Context()
+    check_against_oracle(ctx, torch.from_numpy(_tall_field(*shape)).cuda(), 0.1)
+    ctx.close()
+
+
+def test_batch_of_narrow_rows_many_tiles(fa_mod):
+    import torch
+
+    ctx = fa_mod.Context()
+    host = [_tall_field(*s) for s in ((60, 330, 365), (100, 331, 363), (300, 40, 39), (257, 9, 6), (3, 50, 40))]
+    for f, (v, q, c) in zip(host, ctx.batch_extract([torch.from_numpy(f).cuda() for f in host], [0.1] * len(host))):
+        assert_same_mesh(v.cpu().numpy(), q.cpu().numpy(), oracle.run(f, 0.1))
+    ctx.close()
