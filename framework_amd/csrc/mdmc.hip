@@ -472,6 +472,19 @@ uint32_t emit_blocks(const mdmc_ctx *ctx, uint64_t max_chunks) {
   return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(8, (b + 7) / 8 * 8), 0x7FFFFFF8ull);
 }
 
+// The scan over segment totals that no whole-plane sums cover.  The sums of the
+// scan tiles lie where the look-back keeps its state (32 bytes a tile).
+static void launch_scan(const ScanArgs &sa, hipStream_t st) {
+  const uint32_t tiles = (sa.nsegs + kScanTile - 1u) / kScanTile;
+  if (tiles < kTileScanMin || tiles > kTileScanMax) {
+    hipLaunchKernelGGL(k_scan, dim3(sa.ntiles), dim3(kScanThreads), 0, st, sa);
+    return;
+  }
+  uint4 *const sums = reinterpret_cast<uint4 *>(sa.state);
+  hipLaunchKernelGGL(k_scan_sums, dim3(tiles), dim3(kScanThreads), 0, st, sa, sums);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(kScanThreads), 0, st, sa, static_cast<const uint4 *>(sums));
+}
+
 // box (optional): xyz_min, xyz_max; with it the scan also fills the
 // coordinate tables the emit reads.
 int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
@@ -547,7 +560,7 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
       const PlaneScanArgs pa{sa, s.part, p.XT * p.cy, p.XT * p.NRBp, p.scan_planes};
       hipLaunchKernelGGL(k_scan_planes, dim3((p.cz + p.scan_planes - 1) / p.scan_planes), dim3(kScanThreads), 0, st, pa);
     } else {
-      hipLaunchKernelGGL(k_scan, dim3(p.ntiles), dim3(kScanThreads), 0, st, sa);
+      launch_scan(sa, st);
     }
   }
   HIP_TRY(hipGetLastError());
@@ -962,7 +975,7 @@ int batch_count(mdmc_ctx *ctx, const mdmc_volume *vols, uint32_t n, mdmc_counts 
   sa.counts_out = bcounts;
   {
     ProfScope ps(ctx, 1, st);
-    hipLaunchKernelGGL(k_scan, dim3(agg.ntiles), dim3(kScanThreads), 0, st, sa);
+    launch_scan(sa, st);
   }
   HIP_TRY(hipGetLastError());
   BatchCountArgs bc{};
@@ -976,7 +989,7 @@ int batch_count(mdmc_ctx *ctx, const mdmc_volume *vols, uint32_t n, mdmc_counts 
   bc.batch_counts = bcounts;
   {
     ProfScope ps(ctx, 3, st);
-    hipLaunchKernelGGL(k_batch_counts, dim3((n + 255) / 256), dim3(256), 0, st, bc);
+    hipLaunchKernelGGL(k_batch_counts, dim3((n + 3) / 4), dim3(256), 0, st, bc);
   }
   HIP_TRY(hipGetLastError());
   agg.nsegs = nsegs;

@@ -12,9 +12,12 @@
 //               x-tile in one plane), plus a per-16-cell group map (active
 //               mask, first rank).  Workgroups map to tiles XCD by XCD (mdmc_tilemap.h).
 //               k_classify is the z-marching form for any row length.
-//   k_scan      single-pass decoupled look-back scan (ticketed tiles) over the
-//               segment totals: vertex/quad bases per segment, the non-empty
-//               segment list and where each 64-cell chunk starts.
+//   k_scan_planes, k_scan_tiles, k_scan   scan over the segment totals:
+//               vertex/quad bases per segment, the non-empty segment list and
+//               where each 64-cell chunk starts.  From sums per plane that the
+//               classify left, from sums per 2048 segments, or (the smallest
+//               batches, the largest volumes, the z-marching classify's small
+//               grids) single-pass with decoupled look-back.
 //   k_emit      one wave per chunk of 64 active cells: edge crossing points
 //               in the owner's orientation, dual vertices (FP32, reference
 //               operation order) and quads; ring cells are found through the
@@ -1404,45 +1407,21 @@ struct PlaneScanArgs {
   uint32_t planes;      // cell planes per workgroup
 };
 
-__global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
-  constexpr int kWaves = kScanThreads / kWave;
-  __shared__ uint4 s_before[kWaves], s_wave[kWaves];
-  const ScanArgs &a = p.s;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-  const uint32_t first = blockIdx.x * p.planes * p.plane_segs;
-  const uint32_t end = min(first + p.planes * p.plane_segs, a.nsegs);
-  const uint32_t base = first + tid * kScanIpt;
-  // this thread's segments (the totals array is padded to whole tiles)
-  uint2 c[kScanIpt];
-  {
-    typedef uint32_t Word4 __attribute__((ext_vector_type(4), aligned(8)));
-    const Word4 *src = reinterpret_cast<const Word4 *>(a.seg_counts + (base < end ? base : first));
+// A thread's kScanIpt segment totals from `base`, zeros from `end` on (the
+// totals array is padded to whole tiles).
+__device__ __forceinline__ void scan_load(const uint2 *seg_counts, uint32_t first, uint32_t base, uint32_t end,
+                                          uint2 (&c)[kScanIpt]) {
+  typedef uint32_t Word4 __attribute__((ext_vector_type(4), aligned(8)));
+  const Word4 *src = reinterpret_cast<const Word4 *>(seg_counts + (base < end ? base : first));
 #pragma unroll
-    for (int i = 0; i < kScanIpt / 2; ++i) {
-      const Word4 w = src[i];
-      c[2 * i] = base + 2 * i < end ? make_uint2(w.x, w.y) : make_uint2(0u, 0u);
-      c[2 * i + 1] = base + 2 * i + 1 < end ? make_uint2(w.z, w.w) : make_uint2(0u, 0u);
-    }
+  for (int i = 0; i < kScanIpt / 2; ++i) {
+    const Word4 w = src[i];
+    c[2 * i] = base + 2 * i < end ? make_uint2(w.x, w.y) : make_uint2(0u, 0u);
+    c[2 * i + 1] = base + 2 * i + 1 < end ? make_uint2(w.z, w.w) : make_uint2(0u, 0u);
   }
-  // sums of everything before the workgroup's planes
-  const uint32_t nbefore = blockIdx.x * p.planes * p.plane_parts;
-  uint4 bef = make_uint4(0, 0, 0, 0);
-  const uint4 *parts2 = reinterpret_cast<const uint4 *>(p.part);
-#pragma unroll 8
-  for (uint32_t i = tid; i < nbefore / 2u; i += kScanThreads) {
-    const uint4 q = parts2[i];
-    bef.x += (q.x & 0xFFFFu) + (q.z & 0xFFFFu);
-    bef.y += (q.y & 0xFFFFu) + (q.w & 0xFFFFu);
-    bef.z += (q.x >> 16) + (q.z >> 16);
-    bef.w += (q.y >> 16) + (q.w >> 16);
-  }
-  if ((nbefore & 1u) && tid == 0) {
-    const uint2 q = p.part[nbefore - 1u];
-    bef.x += q.x & 0xFFFFu;
-    bef.y += q.y & 0xFFFFu;
-    bef.z += q.x >> 16;
-    bef.w += q.y >> 16;
-  }
+}
+// {active cells, vertices, quads, non-empty segments}
+__device__ __forceinline__ uint4 scan_sum(const uint2 (&c)[kScanIpt]) {
   uint4 sum = make_uint4(0, 0, 0, 0);
 #pragma unroll
   for (int i = 0; i < kScanIpt; ++i) {
@@ -1451,13 +1430,29 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
     sum.z += c[i].x >> 16;
     sum.w += (c[i].x & 0xFFFFu) ? 1u : 0u;
   }
-  const uint4 inc = make_uint4(wave_incl_scan_dpp(sum.x), wave_incl_scan_dpp(sum.y), wave_incl_scan_dpp(sum.z),
-                               wave_incl_scan_dpp(sum.w));
-  const uint4 binc = make_uint4(wave_incl_scan_dpp(bef.x), wave_incl_scan_dpp(bef.y), wave_incl_scan_dpp(bef.z),
-                                wave_incl_scan_dpp(bef.w));
+  return sum;
+}
+__device__ __forceinline__ uint4 scan_incl(uint4 v) {
+  return make_uint4(wave_incl_scan_dpp(v.x), wave_incl_scan_dpp(v.y), wave_incl_scan_dpp(v.z), wave_incl_scan_dpp(v.w));
+}
+
+// A workgroup's segments [first, end): their bases and the lists, given the
+// thread's share `bef` of the sums of everything before them.
+__device__ __forceinline__ void scan_write(const ScanArgs &a, uint32_t first, uint32_t end, const uint2 (&c)[kScanIpt],
+                                           uint4 bef) {
+  constexpr int kWaves = kScanThreads / kWave;
+  __shared__ uint4 s_before[kWaves], s_wave[kWaves];
+  __shared__ uint2 s_high[kWaves];  // upper words of s_before's vertices and quads
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id(), base = first + tid * kScanIpt;
+  const uint4 sum = scan_sum(c), inc = scan_incl(sum);
+  // (vertices and quads may pass 2^32, which is reported: summed in halves)
+  const uint32_t act = wave_incl_scan_dpp(bef.x), ne = wave_incl_scan_dpp(bef.w);
+  const uint64_t bv = ((uint64_t)wave_incl_scan_dpp(bef.y >> 16) << 16) + wave_incl_scan_dpp(bef.y & 0xFFFFu);
+  const uint64_t bq = ((uint64_t)wave_incl_scan_dpp(bef.z >> 16) << 16) + wave_incl_scan_dpp(bef.z & 0xFFFFu);
   if (lane == kWave - 1) {
     s_wave[wave] = inc;
-    s_before[wave] = binc;
+    s_before[wave] = make_uint4(act, (uint32_t)bv, (uint32_t)bq, ne);
+    s_high[wave] = make_uint2((uint32_t)(bv >> 32), (uint32_t)(bq >> 32));
   }
   __syncthreads();
   uint32_t pa = inc.x - sum.x, pv = inc.y - sum.y, pq = inc.z - sum.z, pe = inc.w - sum.w;
@@ -1469,8 +1464,9 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
     pv += b.y;
     pq += b.z;
     pe += b.w;
-    tot_v += (uint64_t)b.y + v.y;
-    tot_q += (uint64_t)b.z + v.z;
+    const uint2 h = s_high[w];
+    tot_v += ((uint64_t)h.x << 32) + b.y + v.y;
+    tot_q += ((uint64_t)h.y << 32) + b.z + v.z;
     if ((uint32_t)w < wave) {
       pa += v.x;
       pv += v.y;
@@ -1514,6 +1510,76 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
     }
   }
   if (bad && a.counts_out) atomicOr(a.counts_out + 3, kStatusInternal);
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
+  const ScanArgs &a = p.s;
+  const uint32_t tid = threadIdx.x;
+  const uint32_t first = blockIdx.x * p.planes * p.plane_segs;
+  const uint32_t end = min(first + p.planes * p.plane_segs, a.nsegs);
+  uint2 c[kScanIpt];
+  scan_load(a.seg_counts, first, first + tid * kScanIpt, end, c);
+  // sums of everything before the workgroup's planes
+  const uint32_t nbefore = blockIdx.x * p.planes * p.plane_parts;
+  uint4 bef = make_uint4(0, 0, 0, 0);
+  const uint4 *parts2 = reinterpret_cast<const uint4 *>(p.part);
+#pragma unroll 8
+  for (uint32_t i = tid; i < nbefore / 2u; i += kScanThreads) {
+    const uint4 q = parts2[i];
+    bef.x += (q.x & 0xFFFFu) + (q.z & 0xFFFFu);
+    bef.y += (q.y & 0xFFFFu) + (q.w & 0xFFFFu);
+    bef.z += (q.x >> 16) + (q.z >> 16);
+    bef.w += (q.y >> 16) + (q.w >> 16);
+  }
+  if ((nbefore & 1u) && tid == 0) {
+    const uint2 q = p.part[nbefore - 1u];
+    bef.x += q.x & 0xFFFFu;
+    bef.y += q.y & 0xFFFFu;
+    bef.z += q.x >> 16;
+    bef.w += q.y >> 16;
+  }
+  scan_write(a, first, end, c, bef);
+  if (a.fill_coords) coords_fill(a.co, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+
+// The scan of larger volumes and of batches, in two launches and again without
+// look-back: k_scan_sums leaves the sums of every scan tile, and a workgroup of
+// k_scan_tiles adds up those before its own.  HIP events around both launches:
+// 512^3 (128 tiles) 13.3 -> 11.6 us, 603x487x399 (190) 13.3 -> 12.0, 1024^3
+// gyroid (1024) 62.8 -> 44.9, 256 volumes of 32 to 256 points (1,460) 66.7 ->
+// 40.2; with 24 volumes of 32 to 128 points (57 tiles) the look-back is ahead,
+// 9.9 to 11.3.  The reading grows with the square of the tiles.
+constexpr uint32_t kTileScanMin = 96, kTileScanMax = 4096;
+
+__global__ __launch_bounds__(kScanThreads) void k_scan_sums(ScanArgs a, uint4 *sums) {
+  __shared__ uint4 s_wave[kScanThreads / kWave];
+  const uint32_t first = blockIdx.x * kScanTile, end = min(first + kScanTile, a.nsegs);
+  uint2 c[kScanIpt];
+  scan_load(a.seg_counts, first, first + threadIdx.x * kScanIpt, end, c);
+  const uint4 inc = scan_incl(scan_sum(c));
+  if (lane_id() == kWave - 1) s_wave[wave_id()] = inc;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  uint4 t = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int w = 0; w < kScanThreads / kWave; ++w) {
+    const uint4 v = s_wave[w];
+    t = make_uint4(t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w);
+  }
+  sums[blockIdx.x] = t;
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(ScanArgs a, const uint4 *sums) {
+  const uint32_t first = blockIdx.x * kScanTile, end = min(first + kScanTile, a.nsegs);
+  uint2 c[kScanIpt];
+  scan_load(a.seg_counts, first, first + threadIdx.x * kScanIpt, end, c);
+  uint4 bef = make_uint4(0, 0, 0, 0);
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) {
+    const uint4 v = sums[i];
+    bef = make_uint4(bef.x + v.x, bef.y + v.y, bef.z + v.z, bef.w + v.w);
+  }
+  scan_write(a, first, end, c, bef);
   if (a.fill_coords) coords_fill(a.co, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
@@ -2516,17 +2582,35 @@ __global__ void k_slab_info(const uint2 *seg_vq, const uint2 *ne, const Totals *
   out[8] = actives_before(ne, num_ne, s_hi) - actives_before(ne, num_ne, s_lo);
 }
 
-// One thread per volume: its totals and the bases of its numbering.
+// The same by a whole wave: 64 entries a round, so 4 rounds of loads for 16 M
+// segments instead of 24 one after the other.
+__device__ __forceinline__ uint32_t actives_before_wave(const uint2 *ne, uint32_t num_ne, uint32_t s) {
+  uint32_t lo = 0, n = num_ne;  // the first entry at or after s is in [lo, lo + n]
+  while (n != 0u) {
+    const uint32_t step = (n + kWave - 1u) / kWave, i = lane_id() * step;
+    const uint32_t less = (uint32_t)__popcll(__ballot(i < n && ne[lo + min(i, n - 1u)].x < s));
+    if (less == 0u) break;
+    const uint32_t at = (less - 1u) * step + 1u;  // entries up to the last one found less are
+    n = min(step - 1u, n - at);
+    lo += at;
+  }
+  return ne[lo].y;
+}
+
+// One wave per volume: its totals and the bases of its numbering.
 __global__ __launch_bounds__(256) void k_batch_counts(BatchCountArgs b) {
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t v = blockIdx.x * (256u / kWave) + wave_id();
   if (v >= b.nvol) return;
   const BatchVol &bv = b.vols[v];
   const uint32_t num_ne = min(b.totals->num_nonempty, b.nsegs);
   const uint2 v0 = b.seg_vq[bv.seg_off], v1 = b.seg_vq[bv.seg_off + bv.nsegs];
+  uint32_t active = 0u;
+  if (bv.counts && bv.nsegs)
+    active = actives_before_wave(b.ne, num_ne, bv.seg_off + bv.nsegs) - actives_before_wave(b.ne, num_ne, bv.seg_off);
+  if (lane_id() != 0u) return;
   b.base[v] = v0;
   if (bv.counts) {
-    bv.counts[0] = bv.nsegs ? actives_before(b.ne, num_ne, bv.seg_off + bv.nsegs) - actives_before(b.ne, num_ne, bv.seg_off)
-                            : 0u;
+    bv.counts[0] = active;
     bv.counts[1] = v1.x - v0.x;
     bv.counts[2] = v1.y - v0.y;
     bv.counts[3] = b.batch_counts[3];
