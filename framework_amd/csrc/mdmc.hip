@@ -221,8 +221,8 @@ int plan_tiling(const uint32_t dims[3], Plan *p, const int *opt) {
   p->tail = pt_tail(p->X, p->XT, p->cap);
   if (p->tail != kPtTailTiny && (rows != pt_rows(W / 4) || p->ptKP != pt_planes(W / 4))) p->tail = kPtTailFull;
   const uint32_t xt_full = p->tail == kPtTailFull ? p->XT : p->XT - 1u;
-  p->tall = pt_tall_when(p->tail, rows, p->ptKP, p->XT, (uint64_t)p->XT * nrb * p->NKBp) != kTallNever;
-  const uint32_t kp_tail = p->tall ? pt_tall(p->tail, rows, p->ptKP) : p->ptKP;
+  p->tall = pt_tall_when(p->tail, W / 4, rows, p->ptKP, p->XT, (uint64_t)p->XT * nrb * p->NKBp) != kTallNever;
+  const uint32_t kp_tail = p->tall ? pt_tall(p->tail, W / 4, rows, p->ptKP) : p->ptKP;
   p->NKBt = (p->cz + kp_tail - 1) / kp_tail;
   // the scan by whole planes, if a workgroup holds one (a plane's segments and
   // the sums are 32-bit counts well within range)
@@ -794,7 +794,8 @@ int fill_batch_table(mdmc_ctx *ctx, int slot, const mdmc_volume *vols, uint32_t 
     const uint32_t XT = empty ? 1 : (cx + cap - 1) / cap;
     const uint32_t NRB = empty ? 0 : (cy + kBatchRows - 1) / kBatchRows;
     const uint32_t tail = empty ? kPtTailFull : pt_tail(X, XT, cap);
-    const uint32_t tall = pt_tall_when(tail, kBatchRows, KP, XT, tiles), kp = tall == kTallAll ? pt_tall(tail, kBatchRows, KP) : KP;
+    const uint32_t tall = pt_tall_when(tail, W4, kBatchRows, KP, XT, tiles);
+    const uint32_t kp = tall == kTallAll ? pt_tall(tail, W4, kBatchRows, KP) : KP;
     const uint32_t NKP = empty ? 0 : (cz + kp - 1) / kp;
     const uint64_t nsegs = (uint64_t)XT * cy * cz;
     b.c.g = FieldDesc{mv.field, X, Y, Z, cx, cy, cz, mv.iso};

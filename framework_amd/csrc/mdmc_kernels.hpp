@@ -451,10 +451,11 @@ __host__ __device__ constexpr uint32_t pt_tail(uint32_t X, uint32_t XT, uint32_t
 // less, but its loads, barriers and list rounds follow each other just as
 // slowly, and it keeps its place on the CU for half as long (256 volumes of 32
 // to 256 points a side: classify 701 us, with tall tiles 584).
-__host__ __device__ constexpr uint32_t pt_tall(uint32_t tail, uint32_t R, uint32_t KP) {
-  const bool narrow = tail == kPtTail16 || tail == kPtTail32 || tail == kPtTail64;
-  const uint32_t most = tail == kPtTail64 ? 4u : 8u;
-  return narrow && R == 7u && most >= KP ? most / KP * KP : KP;
+__host__ __device__ constexpr uint32_t pt_tall(uint32_t tail, uint32_t W4, uint32_t R, uint32_t KP) {
+  if (R != 7u || (tail != kPtTail16 && tail != kPtTail32 && tail != kPtTail64)) return KP;
+  // (tail: its lanes, and LDS words, per row and plane; a full tile has 64 W4)
+  const uint32_t words = KP * W4 * 64u / tail, most = words < 8u ? words : 8u;
+  return most >= KP ? most / KP * KP : KP;
 }
 // Narrow tiles are tall where rows have full x-tiles as well (in a batch, whose
 // tiles are in memory order, every pt_tall / KP-th plane block's narrow tile
@@ -463,8 +464,9 @@ __host__ __device__ constexpr uint32_t pt_tall(uint32_t tail, uint32_t R, uint32
 // 128 points, 4,000 tiles: 31.0 us tall or not).
 constexpr uint32_t kTallNever = 0u, kTallSome = 1u, kTallAll = 2u;
 constexpr uint64_t kTallTiles = 8192;  // of KP planes
-__host__ __device__ constexpr uint32_t pt_tall_when(uint32_t tail, uint32_t R, uint32_t KP, uint64_t XT, uint64_t tiles) {
-  return pt_tall(tail, R, KP) == KP ? kTallNever : XT > 1u ? kTallSome : tiles >= kTallTiles ? kTallAll : kTallNever;
+__host__ __device__ constexpr uint32_t pt_tall_when(uint32_t tail, uint32_t W4, uint32_t R, uint32_t KP, uint64_t XT,
+                                                    uint64_t tiles) {
+  return pt_tall(tail, W4, R, KP) == KP ? kTallNever : XT > 1u ? kTallSome : tiles >= kTallTiles ? kTallAll : kTallNever;
 }
 
 template <int W4, int R, int KP>
@@ -937,9 +939,9 @@ struct PtNarrow {
 };
 
 // One plane tile with the parts TAIL names (pt_tail).
-template <uint32_t TAIL, uint32_t CAP, int R, int KP>
+template <uint32_t TAIL, uint32_t CAP, int R, int KP, uint32_t WORDS>
 __device__ __forceinline__ void classify_pt_parts(const ClassifyArgs &a, uint32_t xt, uint32_t k, uint32_t j0,
-                                                  uint32_t *s_w, PtShared &sh, uint32_t tab_entry, bool store_tab) {
+                                                  uint32_t (&s_w)[WORDS], PtShared &sh, uint32_t tab_entry, bool store_tab) {
   static_assert(KP * R <= (int)kPtRowsMax, "row counts are staged in kPtRowsMax LDS entries");
   constexpr bool TINY = TAIL == kPtTailTiny;
   constexpr int C = TAIL == kPtTailFull ? (int)(CAP / 256u) : TINY ? 0 : (int)(TAIL >> 8);
@@ -947,6 +949,7 @@ __device__ __forceinline__ void classify_pt_parts(const ClassifyArgs &a, uint32_
   constexpr bool TWO = C != 0 && LW != 0;
   using W = PtWide<C ? C : 1, R, KP>;
   using N = PtNarrow<LW ? LW : 16, R, KP, TINY>;
+  static_assert((C != 0 ? KP * W::kPlaneWords : 0u) + (LW != 0 ? KP * N::kPlaneWords : 0u) <= WORDS, "the parts' LDS words");
   const bool tile_ok = (k < a.g.cz) && (j0 < a.g.cy);  // padding tiles do nothing
   const uint32_t x0 = xt * CAP;
   uint32_t *const s_n = s_w + (C ? KP * W::kPlaneWords : 0u);  // the narrow part's words
@@ -987,7 +990,7 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
     zero_scan_state(a, threadIdx.x, kPtThreads);
     if (a.counts_out != nullptr && threadIdx.x < 4) a.counts_out[threadIdx.x] = 0u;
   }
-  constexpr uint32_t KPT = pt_tall(TAIL, R, KP);
+  constexpr uint32_t KPT = pt_tall(TAIL, W4, R, KP);
   constexpr uint32_t CAP = 256u * W4;
   if (TAIL != kPtTailFull && blockIdx.x >= pa.tail_block) {
     const PtTile t = pt_tile_of(blockIdx.x - pa.tail_block, 1u, pa.NRB, pa.NKBT, pa.B);
@@ -1138,16 +1141,16 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 =
     const uint32_t kb = u / nrb, k = kb * KP, j0 = (u - kb * nrb) * R;
     const uint32_t tail = xt + 1u == a.XT ? bv->tail : kPtTailFull, tall = tail == kPtTailFull ? kTallNever : bv->tall;
     constexpr uint32_t CAP = 256u * W4;
-    const uint32_t kpt = pt_tall(tail, R, KP);
+    const uint32_t kpt = pt_tall(tail, W4, R, KP);
     if (tall == kTallSome && kb % (kpt / KP) != 0u) continue;  // (uniform) another's planes
     __syncthreads();  // the previous tile's LDS words are no longer read
     const uint32_t kt = tall == kTallSome ? k : kb * kpt;
     if (W4 <= 2 && tail == kPtTail16 && tall != kTallNever)
-      classify_pt_parts<kPtTail16, CAP, R, (int)pt_tall(kPtTail16, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
+      classify_pt_parts<kPtTail16, CAP, R, (int)pt_tall(kPtTail16, W4, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
     else if (W4 <= 2 && tail == kPtTail32 && tall != kTallNever)
-      classify_pt_parts<kPtTail32, CAP, R, (int)pt_tall(kPtTail32, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
+      classify_pt_parts<kPtTail32, CAP, R, (int)pt_tall(kPtTail32, W4, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
     else if (W4 == 2 && tail == kPtTail64 && tall != kTallNever)
-      classify_pt_parts<kPtTail64, CAP, R, (int)pt_tall(kPtTail64, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
+      classify_pt_parts<kPtTail64, CAP, R, (int)pt_tall(kPtTail64, W4, R, KP)>(a, xt, kt, j0, s_w, sh, 0u, false);
     else if (W4 <= 2 && tail == kPtTail16)
       classify_pt_parts<kPtTail16, CAP, R, KP>(a, xt, k, j0, s_w, sh, 0u, false);
     else if (W4 <= 2 && tail == kPtTail32)

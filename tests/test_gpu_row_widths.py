@@ -84,10 +84,13 @@ def test_narrow_rows_many_tiles(fa_mod, shape):
     ctx.close()
 
 
-def test_batch_of_narrow_rows_many_tiles(fa_mod):
+@pytest.mark.parametrize("planes", [0, 2, 1, 4])
+def test_batch_of_narrow_rows_many_tiles(fa_mod, planes):
+    """Tall narrow tiles for every number of planes a full tile can have."""
     import torch
 
     ctx = fa_mod.Context()
+    ctx.set_option(fa_mod.mdmc.OPT_BATCH_PLANES, planes)
     host = [_tall_field(*s) for s in ((60, 330, 365), (100, 331, 363), (300, 40, 39), (257, 9, 6), (3, 50, 40))]
     for f, (v, q, c) in zip(host, ctx.batch_extract([torch.from_numpy(f).cuda() for f in host], [0.1] * len(host))):
         assert_same_mesh(v.cpu().numpy(), q.cpu().numpy(), oracle.run(f, 0.1))
