@@ -1094,9 +1094,13 @@ __device__ __forceinline__ uint32_t volume_of(const uint32_t *off, uint32_t nvol
 
 // Classify over the flattened tiles of all volumes (tiles of a volume in
 // memory order): with a grid of at least the tile count a workgroup per tile,
-// with a smaller grid each workgroup walks several (persistent).
+// with a smaller grid each workgroup walks several (persistent).  6 waves per
+// SIMD at 256-cell x-tiles and 5 at 512: every kind of tile is in this kernel,
+// and at 8 and 6 waves it spilled 14 vector registers (256 volumes of 32 to 256
+// points: 582 us at 8 waves, 567 at 7, 512 at 6, 530 at 5; 24 volumes of 300 to
+// 511 points a row: 252 us at 6, 203 at 5, 219 at 4).
 template <int W4, int R, int KP>
-__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 == 1 ? 8 : (W4 == 2 ? 6 : 4), W4 == 1 ? 8 : (W4 == 2 ? 6 : 4)))) void k_classify_batch(BatchArgs b) {
+__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 == 1 ? 6 : (W4 == 2 ? 5 : 4), W4 == 1 ? 6 : (W4 == 2 ? 5 : 4)))) void k_classify_batch(BatchArgs b) {
   __shared__ uint32_t s_w[PtShape<W4, R, KP>::kLdsWords];
   __shared__ PtShared sh;
   sh.tab[threadIdx.x] = pt_table_entry();
