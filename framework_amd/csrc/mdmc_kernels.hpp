@@ -1013,33 +1013,6 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(W4 >
 constexpr uint32_t kMaxBatch = 1024;  // volumes per batch call
 constexpr uint32_t kPublishHead = 16;  // words before the counts of k_publish
 
-// Exact division of 32-bit numbers by a divisor known on the host: a multiply
-// and two shifts (round-up multiplier 2^32 (2^l - d) / d + 1, l = ceil(log2 d);
-// Granlund and Montgomery, "Division by invariant integers using
-// multiplication").
-struct FastDiv {
-  uint32_t mul, sh1, sh2;
-};
-__host__ inline FastDiv fast_div(uint32_t d) {
-  uint32_t l = 0;
-  while (l < 32u && (1ull << l) < d) ++l;
-  return FastDiv{(uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1u), l < 1u ? l : 1u, l > 1u ? l - 1u : 0u};
-}
-__device__ __forceinline__ uint32_t div_by(uint32_t n, FastDiv d) {
-  const uint32_t t = __umulhi(d.mul, n);
-  return (t + ((n - t) >> d.sh1)) >> d.sh2;
-}
-
-// Segments from a wave's first one on whose records, group maps and field rows
-// lie within 2 GB of that segment's (32-bit lane offsets from its bases): a
-// record is 4 bytes, and a segment lies at most 2 * (distance / XT + 1) point
-// rows further on.
-__host__ inline uint32_t emit_span(uint32_t X, uint32_t XT, uint32_t cap) {
-  const uint64_t rec = (1ull << 31) / (4ull * cap) - 1u, rows = (1ull << 31) / (4ull * X);
-  const uint64_t fld = rows > 6u ? (uint64_t)XT * ((rows - 4u) / 2u) : 0u;
-  return (uint32_t)(rec < fld ? rec : fld);
-}
-
 // Per-volume part of the emit arguments.
 struct EmitVol {
   FieldDesc g;

@@ -1,5 +1,5 @@
-// Workgroup -> tile map of the plane-tile classify (k_classify_pt), and the
-// chunk tickets of the persistent emit (k_emit).
+// Workgroup -> tile map of the plane-tile classify (k_classify_pt), the chunk
+// tickets of the persistent emit (k_emit), and the emit's address arithmetic.
 //
 // Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
 // b % 8).  A column is one x-tile of one row block; columns form groups of B.
@@ -78,6 +78,33 @@ MDMC_HD inline EmitTickets emit_tickets(uint32_t n, uint32_t x, uint32_t G, uint
 }
 // first chunk of ticket t
 MDMC_HD inline uint64_t emit_ticket_chunk(const EmitTickets &e, uint64_t t, uint32_t W) { return e.lo + t * W; }
+
+// Exact division of 32-bit numbers by a divisor known on the host: a multiply
+// and two shifts (round-up multiplier 2^32 (2^l - d) / d + 1, l = ceil(log2 d);
+// Granlund and Montgomery, "Division by invariant integers using
+// multiplication").
+struct FastDiv {
+  uint32_t mul, sh1, sh2;
+};
+inline FastDiv fast_div(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32u && (1ull << l) < d) ++l;
+  return FastDiv{(uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1u), l < 1u ? l : 1u, l > 1u ? l - 1u : 0u};
+}
+MDMC_HD inline uint32_t div_by(uint32_t n, FastDiv d) {
+  const uint32_t t = (uint32_t)(((uint64_t)d.mul * n) >> 32);
+  return (t + ((n - t) >> d.sh1)) >> d.sh2;
+}
+
+// Segments from a wave's first one on whose records, group maps and field rows
+// lie within 2 GB of that segment's (32-bit lane offsets from its bases): a
+// record is 4 bytes, and a segment lies at most 2 * (distance / XT + 1) point
+// rows further on.
+inline uint32_t emit_span(uint32_t X, uint32_t XT, uint32_t cap) {
+  const uint64_t rec = (1ull << 31) / (4ull * cap) - 1u, rows = (1ull << 31) / (4ull * X);
+  const uint64_t fld = rows > 6u ? (uint64_t)XT * ((rows - 4u) / 2u) : 0u;
+  return (uint32_t)(rec < fld ? rec : fld);
+}
 
 }  // namespace mdmc
 
