@@ -357,6 +357,9 @@ int capture_guard(mdmc_ctx *ctx, hipStream_t st) {
   if (ctx->capturing_now) {
     if (ctx->captured && ctx->capture_id != id)
       return fail(MDMC_ERR_INVALID, "context already belongs to another captured graph (use one context per graph)");
+    // a replay finds the coordinate tables as the last replay left them, so
+    // only what the capture itself fills counts as filled
+    if (!ctx->captured) ctx->coords_valid = false;
     ctx->captured = true;
     ctx->capture_id = id;
     return MDMC_OK;
@@ -568,6 +571,19 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
 }
 
 
+// Fills the coordinate tables for a box, unless they hold it: the count or an
+// earlier emit filled them, in the same capture if this call is captured.
+void fill_coords(mdmc_ctx *ctx, const Plan &p, const float mn[3], const float mx[3], hipStream_t st) {
+  if (ctx->coords_valid && std::memcmp(ctx->coords_box, mn, 3 * sizeof(float)) == 0 &&
+      std::memcmp(ctx->coords_box + 3, mx, 3 * sizeof(float)) == 0)
+    return;
+  hipLaunchKernelGGL(k_coords, dim3((uint32_t)std::min<uint64_t>((p.ncoord + 255) / 256, 1024)), dim3(256), 0, st,
+                     coord_args(p, ctx->s, mn, mx));
+  std::memmove(ctx->coords_box, mn, 3 * sizeof(float));
+  std::memmove(ctx->coords_box + 3, mx, 3 * sizeof(float));
+  ctx->coords_valid = true;
+}
+
 int launch_emit(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
                 const float mn[3], const float mx[3], float *d_vertices, uint64_t vcap,
                 int32_t *d_quads, uint64_t qcap, mdmc_counts *d_counts, hipStream_t st) {
@@ -575,10 +591,6 @@ int launch_emit(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   const Scratch &s = ctx->s;
   EmitArgs ea{};
   ea.v.g = FieldDesc{d_field, p.X, p.Y, p.Z, p.cx, p.cy, p.cz, iso};
-  const CoordArgs co = coord_args(p, s, mn, mx);
-  // the count already filled the tables for this box
-  const bool have_coords = ctx->coords_valid && std::memcmp(ctx->coords_box, mn, 3 * sizeof(float)) == 0 &&
-                           std::memcmp(ctx->coords_box + 3, mx, 3 * sizeof(float)) == 0;
   ea.v.xt_c = s.coords;
   ea.v.yt_c = s.coords + p.X;
   ea.v.zt_c = s.coords + p.X + p.Y;
@@ -604,15 +616,7 @@ int launch_emit(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   ea.v.status = reinterpret_cast<uint32_t *>(d_counts) + 3;
   {
     ProfScope ps(ctx, 2, st);
-    if (!have_coords) {
-      hipLaunchKernelGGL(k_coords, dim3((uint32_t)std::min<uint64_t>((p.ncoord + 255) / 256, 1024)), dim3(256), 0,
-                         st, co);
-      // the tables now hold this box: a later emit of the same count with
-      // another box must rewrite them, one with this box may reuse them
-      std::memcpy(ctx->coords_box, mn, 3 * sizeof(float));
-      std::memcpy(ctx->coords_box + 3, mx, 3 * sizeof(float));
-      ctx->coords_valid = true;
-    }
+    fill_coords(ctx, p, mn, mx, st);
     ea.emit_ctr = s.ticket;
     // the count zeroed the ticket counters; an emit after another (or one
     // being captured, whose replays may follow one) zeroes them first
@@ -641,6 +645,7 @@ int launch_smooth(mdmc_ctx *ctx, float *d_vertices, uint64_t vcap, int32_t *d_qu
   const int bpc = ctx->opt[MDMC_OPT_EMIT_BLOCKS_PER_CU] > 0 ? ctx->opt[MDMC_OPT_EMIT_BLOCKS_PER_CU] : kEmitBlocksPerCu;
   const uint32_t blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, (uint64_t)ctx->num_cus * bpc));
   ProfScope ps(ctx, 3, st);
+  fill_coords(ctx, ctx->plan, ctx->coords_box, ctx->coords_box + 3, st);  // (the last emit's box)
   for (uint32_t it = 0; it < num_smooth; ++it) {
     hipLaunchKernelGGL(k_smooth, dim3(blocks), dim3(kEmitThreads), 0, st, ea);
     hipLaunchKernelGGL(k_reaverage, dim3(blocks), dim3(kEmitThreads), 0, st, ea);
