@@ -37,6 +37,7 @@
 #include <stdint.h>
 
 #include "mdmc_tilemap.h"
+#include "mdmc_wave.h"
 
 #pragma clang fp contract(off)
 
@@ -90,6 +91,15 @@ __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 __device__ __forceinline__ uint32_t wave_id() {
   return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
 }
+
+// The wave passes this point together, with its LDS accesses before it done
+// before those after it, for all lanes (mdmc_wave.h).
+struct WaveOrder {
+  __device__ __forceinline__ void operator()() const {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+  }
+};
 
 // Workgroups are dispatched round-robin over the 8 XCDs (block b -> XCD b%8).
 // Remap so that each XCD works on a contiguous range of tiles: neighbouring
@@ -632,7 +642,7 @@ struct PtList {
     const FieldDesc &g = a.g;
     const uint32_t lane = lane_id();
     const bool valid = lane < n;
-    const uint32_t e = valid ? list[(done + lane) & (kPtListLen - 1u)] : 0u;
+    const uint32_t e = ring_take<kPtListLen>(list, done, lane, n, WaveOrder());  // (and sh.row, sh.cnt behind it)
     const uint32_t m = e >> 10, xl = e & 0x3FFu;
     const uint2 row = sh.row[m];
     const uint2 bef = before(m);
@@ -1806,19 +1816,23 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
     const uint32_t n = cnt & 0xFFu;
     const float dn = (float)n;
     const Float3 r{n ? s_acc[0] / dn : qnan, n ? s_acc[T] / dn : qnan, n ? s_acc[2 * T] / dn : qnan};
-    if (vfit) {
+    auto put = [&]() {
+      if (!vfit) return;
       Float3 *st = reinterpret_cast<Float3 *>(s_wave + 3u * dv);
       *st++ = r;
       if (b6) *st++ = Float3{ex[0], ey[0], ez[0]};
       if (b9) *st++ = Float3{ex[1], ey[1], ez[1]};
       if (b10) *st = Float3{ex[2], ey[2], ez[2]};
-    }
-    const uint64_t fits = __ballot(vfit);
-    const uint32_t total = fits ? (uint32_t)__builtin_amdgcn_readlane((int)(dv + nv), 63 - __builtin_clzll(fits)) : 0u;
-    const uint32_t words = 3u * total, tail = words & ~3u;
-    for (uint32_t i = 4u * idx; i < tail; i += 4u * nlanes)
-      __builtin_nontemporal_store(*reinterpret_cast<const Int4 *>(s_wave + i), at_off<Int4Row>(out, i * 4u));
-    for (uint32_t i = tail + idx; i < words; i += nlanes) __builtin_nontemporal_store(s_wave[i], at_off<float>(out, i * 4u));
+    };
+    auto copy = [&]() {
+      const uint64_t fits = __ballot(vfit);
+      const uint32_t total = fits ? (uint32_t)__builtin_amdgcn_readlane((int)(dv + nv), 63 - __builtin_clzll(fits)) : 0u;
+      const uint32_t words = 3u * total, tail = words & ~3u;
+      for (uint32_t i = 4u * idx; i < tail; i += 4u * nlanes)
+        __builtin_nontemporal_store(*reinterpret_cast<const Int4 *>(s_wave + i), at_off<Int4Row>(out, i * 4u));
+      for (uint32_t i = tail + idx; i < words; i += nlanes) __builtin_nontemporal_store(s_wave[i], at_off<float>(out, i * 4u));
+    };
+    wave_exchange(put, copy, WaveOrder());
   } else if (vfit) {
     uint32_t o = dv * 12u;
 #pragma unroll
@@ -1917,26 +1931,31 @@ __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base
   const bool qfit = (uint64_t)qb0 + dq + nq <= vq_.qcap && dq + nq <= kEmitStage / 4u;
   Int4 *st = reinterpret_cast<Int4 *>(s_wave) + (qfit ? dq : 0u);
   const int32_t self = (int32_t)(vb0 + (dvq & 0xFFFFu) + vq_.vshift);
-  if (e6) {
-    const int32_t m0 = self + (int32_t)(((uint32_t)labels >> 24) & 0xFu);
-    const int32_t m1 = vtx(c0, vq0, 7, ok0), m2 = vtx(c3, vq3, 4, ok3), m3 = vtx(c13.x, vq1, 5, ok1);
-    if (qfit) *st++ = v[2] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
-  }
-  if (e9) {
-    const int32_t m0 = self + (int32_t)((lab_hi >> 4) & 0xFu);
-    const int32_t m1 = vtx(c24.x, vq2, 1, ok2), m2 = vtx(c4, vq4, 3, ok4), m3 = vtx(c0, vq0, 11, ok0);
-    if (qfit) *st++ = v[5] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
-  }
-  if (e10) {
-    const int32_t m0 = self + (int32_t)((lab_hi >> 8) & 0xFu);
-    const int32_t m1 = vtx(c13.x, vq1, 8, ok1), m2 = vtx(c5, vq5, 0, ok5), m3 = vtx(c24.x, vq2, 2, ok2);
-    if (qfit) *st++ = v[7] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
-  }
-  const uint64_t fits = __ballot(qfit);
-  const uint32_t total = fits ? (uint32_t)__builtin_amdgcn_readlane((int)(dq + nq), 63 - __builtin_clzll(fits)) : 0u;
-  int32_t *const qout = vq_.quads + 4ull * qb0;
-  for (uint32_t i = idx; i < total; i += nlanes)
-    __builtin_nontemporal_store(reinterpret_cast<const Int4 *>(s_wave)[i], at_off<Int4>(qout, i * 16u));
+  auto put = [&]() {
+    if (e6) {
+      const int32_t m0 = self + (int32_t)(((uint32_t)labels >> 24) & 0xFu);
+      const int32_t m1 = vtx(c0, vq0, 7, ok0), m2 = vtx(c3, vq3, 4, ok3), m3 = vtx(c13.x, vq1, 5, ok1);
+      if (qfit) *st++ = v[2] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
+    }
+    if (e9) {
+      const int32_t m0 = self + (int32_t)((lab_hi >> 4) & 0xFu);
+      const int32_t m1 = vtx(c24.x, vq2, 1, ok2), m2 = vtx(c4, vq4, 3, ok4), m3 = vtx(c0, vq0, 11, ok0);
+      if (qfit) *st++ = v[5] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
+    }
+    if (e10) {
+      const int32_t m0 = self + (int32_t)((lab_hi >> 8) & 0xFu);
+      const int32_t m1 = vtx(c13.x, vq1, 8, ok1), m2 = vtx(c5, vq5, 0, ok5), m3 = vtx(c24.x, vq2, 2, ok2);
+      if (qfit) *st++ = v[7] <= vq_.g.iso ? Int4{m0, m1, m2, m3} : Int4{m0, m3, m2, m1};
+    }
+  };
+  auto copy = [&]() {
+    const uint64_t fits = __ballot(qfit);
+    const uint32_t total = fits ? (uint32_t)__builtin_amdgcn_readlane((int)(dq + nq), 63 - __builtin_clzll(fits)) : 0u;
+    int32_t *const qout = vq_.quads + 4ull * qb0;
+    for (uint32_t i = idx; i < total; i += nlanes)
+      __builtin_nontemporal_store(reinterpret_cast<const Int4 *>(s_wave)[i], at_off<Int4>(qout, i * 16u));
+  };
+  wave_exchange(put, copy, WaveOrder());
   if (!qfit && nq) atomicOr(vq_.status, kStatusQuadOverflow);
   if (!ok) atomicOr(vq_.status, kStatusLookup);
 }
