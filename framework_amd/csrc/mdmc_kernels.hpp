@@ -1397,15 +1397,12 @@ struct PlaneScanArgs {
   uint32_t planes;      // cell planes per workgroup
 };
 
-// A thread's kScanIpt segment totals from `base`, zeros from `end` on (the
-// totals array is padded to whole tiles).
-__device__ __forceinline__ void scan_load(const uint2 *seg_counts, uint32_t first, uint32_t base, uint32_t end,
-                                          uint2 (&c)[kScanIpt]) {
+// A thread's kScanIpt segment totals from `base`, zeros from `end` on.
+__device__ __forceinline__ void scan_load(const uint2 *seg_counts, uint32_t base, uint32_t end, uint2 (&c)[kScanIpt]) {
   typedef uint32_t Word4 __attribute__((ext_vector_type(4), aligned(8)));
-  const Word4 *src = reinterpret_cast<const Word4 *>(seg_counts + (base < end ? base : first));
 #pragma unroll
   for (int i = 0; i < kScanIpt / 2; ++i) {
-    const Word4 w = src[i];
+    const Word4 w = *reinterpret_cast<const Word4 *>(seg_counts + scan_pair(base, i, end));
     c[2 * i] = base + 2 * i < end ? make_uint2(w.x, w.y) : make_uint2(0u, 0u);
     c[2 * i + 1] = base + 2 * i + 1 < end ? make_uint2(w.z, w.w) : make_uint2(0u, 0u);
   }
@@ -1508,7 +1505,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
   const uint32_t first = blockIdx.x * p.planes * p.plane_segs;
   const uint32_t end = min(first + p.planes * p.plane_segs, a.nsegs);
   uint2 c[kScanIpt];
-  scan_load(a.seg_counts, first, first + tid * kScanIpt, end, c);
+  scan_load(a.seg_counts, first + tid * kScanIpt, end, c);
   // sums of everything before the workgroup's planes
   const uint32_t nbefore = blockIdx.x * p.planes * p.plane_parts;
   uint4 bef = make_uint4(0, 0, 0, 0);
@@ -1545,7 +1542,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_sums(ScanArgs a, uint4 *s
   __shared__ uint4 s_wave[kScanThreads / kWave];
   const uint32_t first = blockIdx.x * kScanTile, end = min(first + kScanTile, a.nsegs);
   uint2 c[kScanIpt];
-  scan_load(a.seg_counts, first, first + threadIdx.x * kScanIpt, end, c);
+  scan_load(a.seg_counts, first + threadIdx.x * kScanIpt, end, c);
   const uint4 inc = scan_incl(scan_sum(c));
   if (lane_id() == kWave - 1) s_wave[wave_id()] = inc;
   __syncthreads();
@@ -1562,7 +1559,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_sums(ScanArgs a, uint4 *s
 __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(ScanArgs a, const uint4 *sums) {
   const uint32_t first = blockIdx.x * kScanTile, end = min(first + kScanTile, a.nsegs);
   uint2 c[kScanIpt];
-  scan_load(a.seg_counts, first, first + threadIdx.x * kScanIpt, end, c);
+  scan_load(a.seg_counts, first + threadIdx.x * kScanIpt, end, c);
   uint4 bef = make_uint4(0, 0, 0, 0);
 #pragma unroll 4
   for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) {

@@ -1,5 +1,6 @@
 // Workgroup -> tile map of the plane-tile classify (k_classify_pt), the chunk
-// tickets of the persistent emit (k_emit), and the emit's address arithmetic.
+// tickets of the persistent emit (k_emit), the scan's reads, and the emit's
+// address arithmetic.
 //
 // Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
 // b % 8).  A column is one x-tile of one row block; columns form groups of B.
@@ -78,6 +79,16 @@ MDMC_HD inline EmitTickets emit_tickets(uint32_t n, uint32_t x, uint32_t G, uint
 }
 // first chunk of ticket t
 MDMC_HD inline uint64_t emit_ticket_chunk(const EmitTickets &e, uint64_t t, uint32_t W) { return e.lo + t * W; }
+
+// A scan thread's pairs of segment totals: it reads entries scan_pair(base, i,
+// end) and the one after, where its segments base + 2 i and the next are below
+// end, the end of its workgroup's segments.  Past that it reads the last one
+// and `end` itself, the next workgroup's first or a padding entry: there is at
+// least one, and behind the padding lies what other workgroups write.
+MDMC_HD inline uint32_t scan_pair(uint32_t base, uint32_t i, uint32_t end) {
+  const uint32_t at = base + 2u * i;
+  return at < end ? at : end - 1u;
+}
 
 // Exact division of 32-bit numbers by a divisor known on the host: a multiply
 // and two shifts (round-up multiplier 2^32 (2^l - d) / d + 1, l = ceil(log2 d);
