@@ -224,11 +224,10 @@ int plan_tiling(const uint32_t dims[3], Plan *p, const int *opt) {
   p->tall = pt_tall_when(p->tail, W / 4, rows, p->ptKP, p->XT, (uint64_t)p->XT * nrb * p->NKBp) != kTallNever;
   const uint32_t kp_tail = p->tall ? pt_tall(p->tail, W / 4, rows, p->ptKP) : p->ptKP;
   p->NKBt = (p->cz + kp_tail - 1) / kp_tail;
-  // the scan by whole planes, if a workgroup holds one (a plane's segments and
-  // the sums are 32-bit counts well within range)
-  const uint64_t plane_segs = (uint64_t)p->XT * p->cy, parts = (uint64_t)p->XT * nrb * p->cz;
-  p->scan_planes = !p->zmarch && plane_segs <= kPlaneScanSegs && parts <= kPlaneScanParts
-                       ? (uint32_t)(kPlaneScanSegs / plane_segs) : 0u;
+  // (the z-marching classify leaves no sums per plane)
+  const uint64_t plane_segs = p->zmarch ? 0u : (uint64_t)p->XT * p->cy;
+  p->scan_planes = scan_form(p->nsegs, plane_segs, (uint64_t)p->XT * nrb) == ScanForm::planes
+                       ? (uint32_t)(kScanTileSegs / plane_segs) : 0u;
   // 8 XCDs, each at most ceil(NKB * groups / 8) group tiles of `band` columns
   auto blocks = [&](uint64_t cols, uint64_t nkb) {
     const uint64_t ng = (cols + p->band - 1) / p->band;
@@ -478,11 +477,11 @@ uint32_t emit_blocks(const mdmc_ctx *ctx, uint64_t max_chunks) {
 // The scan over segment totals that no whole-plane sums cover.  The sums of the
 // scan tiles lie where the look-back keeps its state (32 bytes a tile).
 static void launch_scan(const ScanArgs &sa, hipStream_t st) {
-  const uint32_t tiles = (sa.nsegs + kScanTile - 1u) / kScanTile;
-  if (tiles < kTileScanMin || tiles > kTileScanMax) {
+  if (scan_form(sa.nsegs, 0, 0) != ScanForm::tiles) {
     hipLaunchKernelGGL(k_scan, dim3(sa.ntiles), dim3(kScanThreads), 0, st, sa);
     return;
   }
+  const uint32_t tiles = (sa.nsegs + kScanTile - 1u) / kScanTile;
   uint4 *const sums = reinterpret_cast<uint4 *>(sa.state);
   hipLaunchKernelGGL(k_scan_sums, dim3(tiles), dim3(kScanThreads), 0, st, sa, sums);
   hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(kScanThreads), 0, st, sa, static_cast<const uint4 *>(sums));

@@ -1194,6 +1194,7 @@ __global__ __launch_bounds__(256) void k_coords(CoordArgs c) {
 constexpr int kScanThreads = 256;
 constexpr int kScanIpt = 8;  // segments per thread (16: 1 us slower per 512^3 extraction)
 constexpr int kScanTile = kScanThreads * kScanIpt;
+static_assert((uint32_t)kScanTile == kScanTileSegs, "scan_form's tiles");
 constexpr uint32_t kSpinLimit = 1u << 24;
 
 struct ScanArgs {
@@ -1378,7 +1379,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(ScanArgs a) {
 }
 
 // The scan of a small or medium single volume, without look-back: a workgroup
-// takes whole cell planes of at most kPlaneScanSegs segments and finds what
+// takes whole cell planes of at most a scan tile's segments and finds what
 // precedes them by summing the sums the classify left per plane, row block and
 // x-tile (1/7 of the totals, contiguous in scan order), so that no workgroup
 // waits for another: a look-back's hops between the XCDs' caches cost more
@@ -1386,8 +1387,6 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(ScanArgs a) {
 // 10.2 -> 7.4, 256^3 9.9 -> 9.1, 384^3 12.0 -> 10.5.  The reading grows with
 // the square of the sums: at 512^3 (37,000 sums) it costs what the look-back
 // does, so kPlaneScanParts ends there.
-constexpr uint32_t kPlaneScanSegs = kScanTile;
-constexpr uint32_t kPlaneScanParts = 1u << 15;
 
 struct PlaneScanArgs {
   ScanArgs s;           // (state and ticket unused)
@@ -1536,8 +1535,6 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
 // gyroid (1024) 62.8 -> 44.9, 256 volumes of 32 to 256 points (1,460) 66.7 ->
 // 40.2; with 24 volumes of 32 to 128 points (57 tiles) the look-back is ahead,
 // 9.9 to 11.3.  The reading grows with the square of the tiles.
-constexpr uint32_t kTileScanMin = 96, kTileScanMax = 4096;
-
 __global__ __launch_bounds__(kScanThreads) void k_scan_sums(ScanArgs a, uint4 *sums) {
   __shared__ uint4 s_wave[kScanThreads / kWave];
   const uint32_t first = blockIdx.x * kScanTile, end = min(first + kScanTile, a.nsegs);

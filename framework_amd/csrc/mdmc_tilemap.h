@@ -1,5 +1,5 @@
 // Workgroup -> tile map of the plane-tile classify (k_classify_pt), the chunk
-// tickets of the persistent emit (k_emit), the scan's reads, and the emit's
+// tickets of the persistent emit (k_emit), the scan's forms and reads, and the emit's
 // address arithmetic.
 //
 // Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
@@ -79,6 +79,21 @@ MDMC_HD inline EmitTickets emit_tickets(uint32_t n, uint32_t x, uint32_t G, uint
 }
 // first chunk of ticket t
 MDMC_HD inline uint64_t emit_ticket_chunk(const EmitTickets &e, uint64_t t, uint32_t W) { return e.lo + t * W; }
+
+// Which scan serves a call of nsegs segments (the kernels' comments have the
+// measurements behind the lines): whole cell planes of plane_segs segments and
+// plane_parts sums, where a workgroup holds a plane and all sums are few
+// (plane_segs = 0: no planes, as in a batch); sums per scan tile; look-back.
+enum class ScanForm { lookback, planes, tiles };
+constexpr uint32_t kScanTileSegs = 2048;
+constexpr uint32_t kPlaneScanParts = 1u << 15;
+constexpr uint32_t kTileScanMin = 96, kTileScanMax = 4096;
+inline ScanForm scan_form(uint64_t nsegs, uint64_t plane_segs, uint64_t plane_parts) {
+  if (plane_segs != 0 && plane_segs <= kScanTileSegs && plane_parts * (nsegs / plane_segs) <= kPlaneScanParts)
+    return ScanForm::planes;
+  const uint64_t tiles = (nsegs + kScanTileSegs - 1u) / kScanTileSegs;
+  return tiles >= kTileScanMin && tiles <= kTileScanMax ? ScanForm::tiles : ScanForm::lookback;
+}
 
 // A scan thread's pairs of segment totals: it reads entries scan_pair(base, i,
 // end) and the one after, where its segments base + 2 i and the next are below
