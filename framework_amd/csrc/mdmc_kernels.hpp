@@ -380,8 +380,8 @@ __global__ __launch_bounds__(64) void k_classify(ClassifyArgs a) {
   }
 }
 
-// Plane-tile classify: the main kernel for rows that are a multiple of 4
-// points.  A 256-thread workgroup owns one tile = R cell rows x one x-tile
+// Plane-tile classify: the main kernel, for rows of any length.  A 256-thread
+// workgroup owns one tile = R cell rows x one x-tile
 // (256*W4 cells) x KP cell planes.  Workgroups are dispatched round-robin over
 // the 8 XCDs (block b runs on XCD b % 8), each with its own L2.  A column is
 // one x-tile of one row block; columns form groups of B (the band option).
@@ -470,8 +470,11 @@ __host__ __device__ constexpr uint32_t pt_tall(uint32_t tail, uint32_t W4, uint3
 // Narrow tiles are tall where rows have full x-tiles as well (in a batch, whose
 // tiles are in memory order, every pt_tall / KP-th plane block's narrow tile
 // works and the others leave: kTallSome), and where a row is one narrow tile
-// if enough tiles remain to fill the chip twice (kTallAll; 24 volumes of 32 to
-// 128 points, 4,000 tiles: 31.0 us tall or not).
+// if enough tiles remain to fill the chip twice (kTallAll).  Where the line lies
+// matters little: rows of 64 points, classify with and without tall tiles, 16.3
+// and 17.3 us at 5,300 tiles, 20.7 and 21.6 at 8,400, 30.2 and 37.8 at 18,500;
+// rows of 128 points 27.5 and 27.0 at 7,000, 30.5 and 29.2 at 8,400, 51.3 and
+// 53.8 at 18,500; 24 volumes of 32 to 128 points (4,000) 31.0 both.
 constexpr uint32_t kTallNever = 0u, kTallSome = 1u, kTallAll = 2u;
 constexpr uint64_t kTallTiles = 8192;  // of KP planes
 __host__ __device__ constexpr uint32_t pt_tall_when(uint32_t tail, uint32_t W4, uint32_t R, uint32_t KP, uint64_t XT,
@@ -1182,8 +1185,8 @@ __global__ __launch_bounds__(256) void k_coords(CoordArgs c) {
 }
 
 // ---------------------------------------------------------------------------
-// Decoupled look-back scan over segment totals.  A tile is 4096 segments, 16
-// per thread read as eight 16-byte loads (the totals array is padded to a
+// Decoupled look-back scan over segment totals.  A tile is 2048 segments, 8
+// per thread read as four 16-byte loads (the totals array is padded to a
 // whole number of tiles with zeros).  Four channels are scanned: active
 // cells, vertices, quads and non-empty segments.  Outputs: the first vertex
 // and quad of every segment; the list of non-empty segments with the index
@@ -1534,7 +1537,11 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_planes(PlaneScanArgs p) {
 // 512^3 (128 tiles) 13.3 -> 11.6 us, 603x487x399 (190) 13.3 -> 12.0, 1024^3
 // gyroid (1024) 62.8 -> 44.9, 256 volumes of 32 to 256 points (1,460) 66.7 ->
 // 40.2; with 24 volumes of 32 to 128 points (57 tiles) the look-back is ahead,
-// 9.9 to 11.3.  The reading grows with the square of the tiles.
+// 9.9 to 11.3.  The reading grows with the square of the tiles and the
+// look-back with their number; rows of 64 points, both launches against the
+// look-back: 15.6 and 26 us at 512 tiles, 37 and 66 at 2,048, 69 and 108 at
+// 4,092, 130 and 189 at 8,188.  So the two are still ahead where kTileScanMax
+// ends; volumes of that many cell rows need 17 GB of scratch.
 __global__ __launch_bounds__(kScanThreads) void k_scan_sums(ScanArgs a, uint4 *sums) {
   __shared__ uint4 s_wave[kScanThreads / kWave];
   const uint32_t first = blockIdx.x * kScanTile, end = min(first + kScanTile, a.nsegs);
@@ -1660,7 +1667,7 @@ typedef int Int4Row __attribute__((ext_vector_type(4), aligned(4)));
 // vol.span], so everything a lane addresses is a uniform base, taken for s0,
 // plus a 32-bit lane offset.  base: the volume's first vertex and quad.  (64-bit address arithmetic per lane and load, and
 // the division of a segment number into tile, row and plane on every lane,
-// were a quarter of the kernel's issue slots.)  s_lab: kEmitLab entries.
+// were a quarter of the kernel's issue slots.)  s_lab: 512 entries (emit_label).
 __device__ __forceinline__ void emit_cells(EmitArgsK pa, EmitVolK pv, uint2 base, uint32_t s0, uint32_t s,
                                            uint32_t rank, const uint64_t *s_lab, float *s_wave) {
   const EmitArgs &a = fresh(pa);
