@@ -2118,12 +2118,13 @@ __global__ void k_zero_tickets(uint32_t *t) { zero_tickets(t, threadIdx.x); }
 // edge points only), so neither reads what it writes.
 //
 // Each pass rewrites every other vertex of the mesh, so it moves all of its
-// lines twice: on 3.4 M cells (256x240x272 gyroid) k_smooth has 240 MB to move
-// (52 us at a large copy's rate) and takes 84 us with its vector units 90%
-// busy (92 us with two differences, products and a root per corner instead of
-// per edge and integer divisions for the position); k_reaverage has 200 MB
-// (43 us) and takes 68 us, bound by its chain of lookups (83 us with a gather
-// for each of the 12 edges, a third of the address units' work for nothing).
+// lines twice: on 3.4 M cells (256x240x272 gyroid) k_smooth moves 244 MB (52 us
+// at a large copy's rate) and takes 84 us with VALU issue on at most 84% of its
+// cycles (92 us with two differences, products and a root per corner instead of
+// per edge and integer divisions for the position); k_reaverage moves 186 MB
+// (40 us) and takes 68 us, a chain of lookups with VALU issue on at most 85%
+// (83 us with a gather for each of the 12 edges, a third of the address units'
+// work for nothing).
 //
 // The split of a convex ring is at the corner of the largest angle, taken as
 // the smallest cosine (a.b) / (sqrt(a.a) sqrt(b.b)) with IEEE sqrt and
