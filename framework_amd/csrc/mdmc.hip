@@ -474,21 +474,26 @@ uint32_t emit_blocks(const mdmc_ctx *ctx, uint64_t max_chunks) {
   return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(8, (b + 7) / 8 * 8), 0x7FFFFFF8ull);
 }
 
-// The scan over segment totals that no whole-plane sums cover.  The sums of the
-// scan tiles lie where the look-back keeps its state (32 bytes a tile).
+// Workgroups of the scan over segment totals that no whole-plane sums cover.
+static uint32_t scan_blocks(uint32_t nsegs, uint32_t ntiles) {
+  return scan_form(nsegs, 0, 0) == ScanForm::tiles ? (nsegs + kScanTile - 1u) / kScanTile : ntiles;
+}
+
+// That scan.  The sums of the scan tiles lie where the look-back keeps its state
+// (32 bytes a tile).
 static void launch_scan(const ScanArgs &sa, hipStream_t st) {
+  const uint32_t tiles = scan_blocks(sa.nsegs, sa.ntiles);
   if (scan_form(sa.nsegs, 0, 0) != ScanForm::tiles) {
-    hipLaunchKernelGGL(k_scan, dim3(sa.ntiles), dim3(kScanThreads), 0, st, sa);
+    hipLaunchKernelGGL(k_scan, dim3(tiles), dim3(kScanThreads), 0, st, sa);
     return;
   }
-  const uint32_t tiles = (sa.nsegs + kScanTile - 1u) / kScanTile;
   uint4 *const sums = reinterpret_cast<uint4 *>(sa.state);
   hipLaunchKernelGGL(k_scan_sums, dim3(tiles), dim3(kScanThreads), 0, st, sa, sums);
   hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(kScanThreads), 0, st, sa, static_cast<const uint4 *>(sums));
 }
 
 // box (optional): xyz_min, xyz_max; with it the scan also fills the
-// coordinate tables the emit reads.
+// coordinate tables the emit reads, unless the rows are very long.
 int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
                  mdmc_counts *d_counts, hipStream_t st, const float *box_min = nullptr,
                  const float *box_max = nullptr) {
@@ -549,7 +554,8 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
   sa.ticket = s.ticket;
   sa.totals = s.totals;
   sa.counts_out = reinterpret_cast<uint32_t *>(d_counts);
-  if (box_min && box_max) {
+  const uint32_t blocks = p.scan_planes ? (p.cz + p.scan_planes - 1) / p.scan_planes : scan_blocks(sa.nsegs, sa.ntiles);
+  if (box_min && box_max && scan_fills_coords(p.ncoord, (uint64_t)blocks * kScanThreads)) {
     sa.co = coord_args(p, s, box_min, box_max);
     sa.fill_coords = 1;
     std::memcpy(ctx->coords_box, box_min, 3 * sizeof(float));
@@ -560,7 +566,7 @@ int launch_count(mdmc_ctx *ctx, const Plan &p, const float *d_field, float iso,
     ProfScope ps(ctx, 1, st);
     if (p.scan_planes) {
       const PlaneScanArgs pa{sa, s.part, p.XT * p.cy, p.XT * p.NRBp, p.scan_planes};
-      hipLaunchKernelGGL(k_scan_planes, dim3((p.cz + p.scan_planes - 1) / p.scan_planes), dim3(kScanThreads), 0, st, pa);
+      hipLaunchKernelGGL(k_scan_planes, dim3(blocks), dim3(kScanThreads), 0, st, pa);
     } else {
       launch_scan(sa, st);
     }

@@ -95,6 +95,14 @@ inline ScanForm scan_form(uint64_t nsegs, uint64_t plane_segs, uint64_t plane_pa
   return tiles >= kTileScanMin && tiles <= kTileScanMax ? ScanForm::tiles : ScanForm::lookback;
 }
 
+// Whether the scan's workgroups fill the coordinate tables on the side: not
+// where the rows are so long that its threads get more than 64 of the ncoord
+// entries each.  A launch of its own costs an extraction 3 to 4 us, 64 entries
+// about as much (20,000 x 9 x 9 points, 39 a thread: 14 us, with the launch
+// 17; 100,000 x 5 x 5, 195 a thread: 25 and 17; 1,000,000 x 2 x 2,
+// 3,906 a thread: 322 and 17).
+inline bool scan_fills_coords(uint64_t ncoord, uint64_t scan_threads) { return ncoord <= 64u * scan_threads; }
+
 // A scan thread's pairs of segment totals: it reads entries scan_pair(base, i,
 // end) and the one after, where its segments base + 2 i and the next are below
 // end, the end of its workgroup's segments.  Past that it reads the last one
