@@ -1333,9 +1333,12 @@ int mdmc_counts_read(mdmc_ctx *ctx, const mdmc_counts *d_counts, uint32_t n, mdm
   if (n == 0 || n > kMaxBatch) return fail(MDMC_ERR_INVALID, "1..1024 counts can be read");
   static_assert(sizeof(mdmc_counts) == 4 * sizeof(uint32_t), "counts are four words");
   const hipStream_t st = static_cast<hipStream_t>(stream);
+  // (before the guard, which would give the context to the capture)
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cs));
+  if (cs != hipStreamCaptureStatusNone) return fail(MDMC_ERR_INVALID, "counts cannot be read under stream capture");
   const int grc = capture_guard(ctx, st);
   if (grc != MDMC_OK) return grc;
-  if (ctx->capturing_now) return fail(MDMC_ERR_INVALID, "counts cannot be read under stream capture");
   if (!ctx->pub) {
     void *p = nullptr;
     if (hipHostMalloc(&p, (kPublishHead + 4u * kMaxBatch) * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) {

@@ -53,3 +53,23 @@ def test_work_that_outlasts_the_watch(env):
         assert time.perf_counter() - t > 2e-3  # the stream's own wait was taken
         assert (c == rep + 1).all()
     ctx.close()
+
+
+def test_a_refused_read_leaves_the_context_free(env):
+    """Refused under capture, it does not give the context to the graph."""
+    torch, fa = env
+    ctx = fa.Context()
+    field = torch.rand(9, 8, 7, device="cuda")
+    before = ctx.extract(field, 0.5)
+    d = torch.zeros(4, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        d.fill_(1)
+        with pytest.raises(fa.MDMCError, match="capture"):
+            ctx._wait_counts(d, 1, None)
+    after = ctx.extract(field, 0.5)
+    assert torch.equal(before[1], after[1]) and before[2] == after[2]
+    g.replay()
+    assert (ctx._wait_counts(d, 1, None) == 1).all()
+    ctx.close()
