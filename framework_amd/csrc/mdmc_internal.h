@@ -24,7 +24,7 @@ struct Plan {
   uint32_t tail;             // parts of the last x-tile (pt_tail); if narrow: its plane blocks,
   uint32_t NKBt, tall;       // and whether they are tall
   uint64_t pt_blocks, tail_block;  // plane-tile grid, first block of the narrow x-tiles
-  uint32_t scan_planes;      // cell planes per workgroup of the plane scan (0: look-back scan)
+  uint32_t scan_planes;      // cell planes per workgroup of the plane scan (0: another form, scan_form)
 };
 
 struct Scratch {
