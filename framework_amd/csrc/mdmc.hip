@@ -402,6 +402,16 @@ ScratchLayout scratch_layout(const Plan &p) {
   return L;
 }
 
+// Gives up the context's scratch and with it what counts and emits left there:
+// an emit, a batch emit or a smoothing pass now needs a new count.
+hipError_t drop_scratch(mdmc_ctx *ctx) {
+  const hipError_t e = ctx->scratch && !ctx->scratch_external ? hipFree(ctx->scratch) : hipSuccess;
+  ctx->scratch = nullptr;
+  ctx->scratch_bytes = 0;
+  ctx->counted = ctx->batch_counted = ctx->emitted = ctx->coords_valid = false;
+  return e;
+}
+
 int ensure_scratch(mdmc_ctx *ctx, const Plan &p) {
   Scratch s{};
   const ScratchLayout lay = scratch_layout(p);
@@ -415,12 +425,7 @@ int ensure_scratch(mdmc_ctx *ctx, const Plan &p) {
   if (regrow && ctx->capturing_now)
     return fail(MDMC_ERR_INVALID, "scratch must be sized by a call on this context before stream capture");
   if (regrow) {
-    if (ctx->scratch) {
-      hipError_t e = hipFree(ctx->scratch);
-      (void)e;
-      ctx->scratch = nullptr;
-      ctx->scratch_bytes = 0;
-    }
+    if (drop_scratch(ctx) != hipSuccess) (void)hipGetLastError();
     // headroom for slightly larger grids, unless the context keeps to a budget
     const size_t want = ctx->exact_scratch ? off : off + off / 8;
     if (hipMalloc(&ctx->scratch, want) != hipSuccess) {
@@ -1469,12 +1474,14 @@ int mdmc_batch_scratch_bytes(const mdmc_volume *vols, uint32_t n, uint64_t *byte
 int mdmc_ctx_set_scratch(mdmc_ctx *ctx, void *d_scratch, uint64_t bytes) {
   if (!ctx) return fail(MDMC_ERR_INVALID, "null ctx");
   if (ctx->captured) return fail(MDMC_ERR_INVALID, "context belongs to a captured graph whose nodes use its scratch");
-  if (ctx->scratch && !ctx->scratch_external) HIP_TRY(hipFree(ctx->scratch));
+  // (smoothing may still read memory that the caller gave)
+  const bool emitted = ctx->emitted && ctx->scratch_external, coords = ctx->coords_valid && ctx->scratch_external;
+  HIP_TRY(drop_scratch(ctx));
   ctx->scratch = d_scratch;
   ctx->scratch_bytes = d_scratch ? bytes : 0;
   ctx->scratch_external = d_scratch != nullptr;
-  ctx->counted = false;
-  ctx->batch_counted = false;
+  ctx->emitted = emitted;
+  ctx->coords_valid = coords;
   return MDMC_OK;
 }
 
@@ -1760,11 +1767,7 @@ int mdmc_run_out_of_core(const float *field, const uint32_t dims[3], const float
     rc = plan_tiling(sd, &pmax, ctx->opt);
     if (rc != MDMC_OK) return rc;
     const size_t want = scratch_layout(pmax).total;
-    if (ctx->scratch && ctx->scratch_bytes != want) {
-      (void)hipFree(ctx->scratch);
-      ctx->scratch = nullptr;
-      ctx->scratch_bytes = 0;
-    }
+    if (ctx->scratch && ctx->scratch_bytes != want) (void)drop_scratch(ctx);
     rc = ensure_scratch(ctx, pmax);
     if (rc != MDMC_OK) return rc;
   }
