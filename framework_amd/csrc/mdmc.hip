@@ -1299,6 +1299,7 @@ static int count_impl(mdmc_ctx *ctx, const float *d_field, const uint32_t dims[3
   if (!p.empty && !d_field) return fail(MDMC_ERR_INVALID, "null field");
   rc = ensure_scratch(ctx, p);
   if (rc != MDMC_OK) return rc;
+  ctx->batch_counted = false;  // the scratch now holds this volume
   rc = launch_count(ctx, p, d_field, iso, d_counts, static_cast<hipStream_t>(stream), box_min, box_max);
   if (rc != MDMC_OK) return rc;
   ctx->plan = p;

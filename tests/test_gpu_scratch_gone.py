@@ -55,3 +55,23 @@ def test_scratch_that_cannot_grow(env):
                                     ctx._stream(None))
     assert rc == -3  # no memory, before anything is launched
     _usable_again(fa, ctx, f, field, v, q)
+
+
+def test_a_single_count_ends_a_batch(env):
+    """Between a batch's count and its emit a count of one volume takes the
+    scratch over: the batch's emit is refused."""
+    torch, fa, ctx, f, field, v, q = env
+    fields, isos = [field, field[:5].contiguous()], [0.1, 0.2]
+    refs = [oracle.run(f, 0.1), oracle.run(f[:5], 0.2)]
+    counts = ctx.batch_counts_tensor(2)
+    outs = [(torch.empty((len(r["vertices"]), 3), device="cuda"),
+             torch.empty((len(r["quads"]), 4), dtype=torch.int32, device="cuda")) for r in refs]
+    ctx.batch_count(fields, isos, counts)
+    ctx.count(field, 0.1)
+    with pytest.raises(fa.MDMCError, match="without a matching batch count"):
+        ctx.batch_emit(fields, isos, outs, counts)
+    ctx.batch_count(fields, isos, counts)
+    ctx.batch_emit(fields, isos, outs, counts)
+    torch.cuda.synchronize()
+    for (a, b), r in zip(outs, refs):
+        assert_same_mesh(a.cpu().numpy(), b.cpu().numpy(), r)
